@@ -32,34 +32,13 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemmArgs<T> g)
         tri_decode(blockIdx.x, hi, lo);
         if (g.tri == SYM_LOWER) { tm = hi; tn = lo; } else { tm = lo; tn = hi; }
     }
-    if (tm < g.full_m && tn < g.full_n) return;  // interior tile: fast kernel's
     gemm_tile<T, BM, BN, BK>(g, tm, tn, As, Bs);
 }
 
-// A rectangular grid with both full and ragged tiles in one launch: full
-// tiles take the fast tile routine (patterns PA / PB), ragged ones its
-// guarded variant.  One launch instead of a fast grid followed by an edge
-// grid, whose few tiles would otherwise make a round of their own.
-template <typename T, int BM, int PA, int PB>
-__global__ __launch_bounds__(256, 2) void gemm_mixed_kernel(GemmArgs<T> g)
-{
-    constexpr int PAD = 128 / (int)sizeof(T);
-    __shared__ __attribute__((aligned(16))) T As[2][16][BM + PAD];
-    __shared__ __attribute__((aligned(16))) T Bs[2][16][BM + PAD];
-    const int tm = blockIdx.x % g.tiles_m, tn = blockIdx.x / g.tiles_m;
-    if (tm < g.full_m && tn < g.full_n)
-        gemm_fast_tile<T, BM, BM, 16, PA, PB, SYM_NONE>(g, tm, tn, As, Bs);
-    else
-        gemm_fast_tile<T, BM, BM, 16, PA, PB, SYM_NONE, true>(g, tm, tn, As, Bs);
-}
-
-// Fast kernel: the grid holds only tiles that are full in M and N, both
-// operands are 16-B aligned with leading dimensions a multiple of the vector
-// width, and their access patterns are compile-time constants (PA / PB).
-// That leaves no per-element selects in the main loop and frees enough
-// registers for two workgroups per CU, so one workgroup's global loads and
-// barrier overlap the other's MFMAs.  Only a partial last k-tile takes the
-// guarded element loads.
+// Fast kernel: every tile of a product with m >= BM and n >= BN, access
+// patterns compile-time constants (PA / PB), operands of any alignment
+// (gemm_fast_tile).  Registers for two workgroups per CU, so one workgroup's
+// barrier and epilogue overlap the other's MFMAs.
 template <typename T, int BM, int BN, int BK, int PA, int PB, int TRI>
 __global__ __launch_bounds__(256, 2) void gemm_fast_kernel(GemmArgs<T> g)
 {
@@ -104,14 +83,15 @@ __global__ __launch_bounds__(256, 2) void gemm_fast_sub_kernel(GemmArgs<T> g, in
     tn = 2 * tn + (q >> 1);
     if (TRI == SYM_LOWER && tn > tm) return;
     if (TRI == SYM_UPPER && tm > tn) return;
+    if (tm * 64 >= g.m || tn * 64 >= g.n) return;  // past a ragged edge
     gemm_fast_tile<T, 64, 64, 16, PA, PB, TRI>(g, tm, tn, As, Bs);
 }
 
 // Split-K for problems with too few tiles to fill the chip and a long k:
 // block b is BM x BM tile b % tiles over k chunk b / tiles (kchunk deep, a
-// multiple of 16), written unscaled to P[chunk] (m x n, leading dimension
-// m); splitk_fold_kernel then forms alpha * (sum of chunks in chunk order) +
-// beta * C.  The decomposition depends only on the shape, so the bits
+// multiple of 16; the last one what is left), written unscaled to P[chunk] (m x
+// n, leading dimension m); splitk_fold_kernel then forms alpha * (sum of chunks
+// in chunk order) + beta * C.  The decomposition depends only on the shape, so the bits
 // repeat from call to call.
 template <typename T, int BM, int PA, int PB>
 __global__ __launch_bounds__(256, 2) void gemm_fast_splitk_kernel(GemmArgs<T> g, int kchunk, T *P)
@@ -124,9 +104,9 @@ __global__ __launch_bounds__(256, 2) void gemm_fast_splitk_kernel(GemmArgs<T> g,
     const long koff = (long)kc * kchunk;
     GemmArgs<T> h = g;
     // element (o, k) of an operand is p[o + k*ld] (outer) or p[k + o*ld]
-    h.a.p += pat_base(PA) == PAT_OUTER ? koff * g.a.ld : koff;
-    h.b.p += pat_base(PB) == PAT_OUTER ? koff * g.b.ld : koff;
-    h.k = kchunk;
+    h.a.p += PA == PAT_OUTER ? koff * g.a.ld : koff;
+    h.b.p += PB == PAT_OUTER ? koff * g.b.ld : koff;
+    h.k = min(kchunk, g.k - (int)koff);
     h.alpha = T(1);
     h.beta = T(0);
     h.C = P + (long)kc * g.m * g.n;
@@ -197,13 +177,7 @@ void launch_fast(hipStream_t s, const GemmArgs<T> &g, unsigned blocks)
     hipLaunchKernelGGL((gemm_fast_kernel<T, BM, BM, 16, PA_, PB_, TRI_>), dim3(blocks),         \
                        dim3(256), 0, s, g)
     const int pa = g.a.form, pb = g.b.form;
-    const bool ua = !(g.a.vec_ok && g.b.vec_ok);  // element loads (rectangular grids only)
-    if (g.tri == SYM_NONE && ua) {
-        if (pa == PAT_OUTER && pb == PAT_KCONT) GB_FAST(PAT_OUTER_U, PAT_KCONT_U, SYM_NONE);
-        else if (pa == PAT_OUTER) GB_FAST(PAT_OUTER_U, PAT_OUTER_U, SYM_NONE);
-        else if (pb == PAT_KCONT) GB_FAST(PAT_KCONT_U, PAT_KCONT_U, SYM_NONE);
-        else GB_FAST(PAT_KCONT_U, PAT_OUTER_U, SYM_NONE);
-    } else if (g.tri == SYM_NONE) {
+    if (g.tri == SYM_NONE) {
         if (pa == PAT_OUTER && pb == PAT_KCONT) GB_FAST(PAT_OUTER, PAT_KCONT, SYM_NONE);      // NN
         else if (pa == PAT_OUTER) GB_FAST(PAT_OUTER, PAT_OUTER, SYM_NONE);                    // NT
         else if (pb == PAT_KCONT) GB_FAST(PAT_KCONT, PAT_KCONT, SYM_NONE);                    // TN
@@ -225,13 +199,7 @@ void launch_fast_sub(hipStream_t s, const GemmArgs<T> &g, int base, unsigned blo
     hipLaunchKernelGGL((gemm_fast_sub_kernel<T, PA_, PB_, TRI_>), dim3(blocks), dim3(256), 0, s, \
                        g, base)
     const int pa = g.a.form, pb = g.b.form;
-    const bool ua = !(g.a.vec_ok && g.b.vec_ok);
-    if (g.tri == SYM_NONE && ua) {
-        if (pa == PAT_OUTER && pb == PAT_KCONT) GB_SUB(PAT_OUTER_U, PAT_KCONT_U, SYM_NONE);
-        else if (pa == PAT_OUTER) GB_SUB(PAT_OUTER_U, PAT_OUTER_U, SYM_NONE);
-        else if (pb == PAT_KCONT) GB_SUB(PAT_KCONT_U, PAT_KCONT_U, SYM_NONE);
-        else GB_SUB(PAT_KCONT_U, PAT_OUTER_U, SYM_NONE);
-    } else if (g.tri == SYM_NONE) {
+    if (g.tri == SYM_NONE) {
         if (pa == PAT_OUTER && pb == PAT_KCONT) GB_SUB(PAT_OUTER, PAT_KCONT, SYM_NONE);
         else if (pa == PAT_OUTER) GB_SUB(PAT_OUTER, PAT_OUTER, SYM_NONE);
         else if (pb == PAT_KCONT) GB_SUB(PAT_KCONT, PAT_KCONT, SYM_NONE);
@@ -262,43 +230,34 @@ long fast_slots()
     return slots;
 }
 
-// Split-K launch of a rectangular product whose BM x BM tiles are all full
-// and number at most half the workgroup slots; k is cut into as many chunks
-// as fill the slots (at most 8, each at least 256 deep, k divisible).
-// Returns -1 when the shape does not qualify, so the caller takes the
-// ordinary grid.
+// Split-K launch of a rectangular product whose BM x BM tiles number at most
+// half the workgroup slots; k is cut into as many chunks as fill the slots (at
+// most 8, each at least 256 deep, a multiple of 16).  Returns -1 when the shape
+// does not qualify, so the caller takes the ordinary grid.
 template <typename T, int BM>
 int launch_splitk(hipStream_t s, const GemmArgs<T> &g, int m, int n, int k)
 {
-    const long tiles = (long)(m / BM) * (n / BM), slots = fast_slots();
-    if (m % BM || n % BM || tiles == 0 || 2 * tiles > slots) return -1;
-    int ks = (int)std::min<long>(slots / tiles, 8);
-    while (ks > 1 && (k % (16 * ks) || k / ks < 256)) --ks;
+    const long tiles = (long)ceil_div(m, BM) * ceil_div(n, BM), slots = fast_slots();
+    if (2 * tiles > slots) return -1;
+    const int want = (int)std::min<long>(std::min<long>(slots / tiles, 8), k / 256);
+    if (want < 2) return -1;
+    const int kchunk = ceil_div(ceil_div(k, want), 16) * 16, ks = ceil_div(k, kchunk);
     if (ks < 2) return -1;
     T *P = (T *)gpublas_dev_alloc((size_t)ks * m * n * sizeof(T));
     if (!P) return -1;
     GemmArgs<T> f = g;
-    f.tiles_m = m / BM;
-    f.tiles_n = n / BM;
-    f.full_m = f.full_n = 0;
+    f.tiles_m = ceil_div(m, BM);
+    f.tiles_n = ceil_div(n, BM);
     const unsigned blocks = (unsigned)(tiles * ks);
 #define GB_SK(PA_, PB_)                                                                          \
     hipLaunchKernelGGL((gemm_fast_splitk_kernel<T, BM, PA_, PB_>), dim3(blocks), dim3(256), 0, s, \
-                       f, k / ks, P)
+                       f, kchunk, P)
     const int pa = g.a.form, pb = g.b.form;
-    const bool ua = !(g.a.vec_ok && g.b.vec_ok);
     PROF_BEGIN(s, sizeof(T) == 8 ? "dgemm_splitk" : "sgemm_splitk");
-    if (ua) {
-        if (pa == PAT_OUTER && pb == PAT_KCONT) GB_SK(PAT_OUTER_U, PAT_KCONT_U);
-        else if (pa == PAT_OUTER) GB_SK(PAT_OUTER_U, PAT_OUTER_U);
-        else if (pb == PAT_KCONT) GB_SK(PAT_KCONT_U, PAT_KCONT_U);
-        else GB_SK(PAT_KCONT_U, PAT_OUTER_U);
-    } else {
-        if (pa == PAT_OUTER && pb == PAT_KCONT) GB_SK(PAT_OUTER, PAT_KCONT);
-        else if (pa == PAT_OUTER) GB_SK(PAT_OUTER, PAT_OUTER);
-        else if (pb == PAT_KCONT) GB_SK(PAT_KCONT, PAT_KCONT);
-        else GB_SK(PAT_KCONT, PAT_OUTER);
-    }
+    if (pa == PAT_OUTER && pb == PAT_KCONT) GB_SK(PAT_OUTER, PAT_KCONT);
+    else if (pa == PAT_OUTER) GB_SK(PAT_OUTER, PAT_OUTER);
+    else if (pb == PAT_KCONT) GB_SK(PAT_KCONT, PAT_KCONT);
+    else GB_SK(PAT_KCONT, PAT_OUTER);
 #undef GB_SK
     const long mn = (long)m * n;
     const unsigned fb = (unsigned)std::min<long>((mn + 255) / 256, 4096);
@@ -310,11 +269,9 @@ int launch_splitk(hipStream_t s, const GemmArgs<T> &g, int m, int n, int k)
 }
 
 // Core launcher: C = alpha*op(A)*op(B) + beta*C on an (optionally
-// triangular) tile grid.  k > 0, alpha != 0 assumed.  Tiles that are full in
-// M and N go to the fast kernel (vector loads when both operands are
-// aligned, element loads otherwise; a triangular grid needs aligned
-// operands); the generic kernel takes the ragged edge (and everything, for
-// symmetric operands).
+// triangular) tile grid.  k > 0, alpha != 0 assumed.  Products at least a tile
+// wide in both dimensions go to the fast kernel; the generic kernel takes the
+// narrow ones, symmetric operands and leading dimensions past FAST_LD_MAX.
 template <typename T>
 int launch_gemm(hipStream_t s, int m, int n, int k, T alpha, const Operand<T> &a,
                 const Operand<T> &b, T beta, T *C, long ldc, int tri)
@@ -328,75 +285,38 @@ int launch_gemm(hipStream_t s, int m, int n, int k, T alpha, const Operand<T> &a
     // Tile choice: 128x128 when that alone gives at least one tile per CU,
     // else 64x64 so that mid-size problems still fill the 256 CUs.
     const long t128 = (long)ceil_div(m, 128) * ceil_div(n, 128);
-    const bool big = t128 >= 256;
+    const bool big = t128 >= 256 && m >= 128 && n >= 128;
     const int bm = big ? 128 : 64;
-    // full tiles take the fast kernels: with vector loads when both operands
-    // are aligned, else (rectangular grids) with element loads
-    const bool fast_ok = a.sym == SYM_NONE && b.sym == SYM_NONE &&
-                         ((a.vec_ok && b.vec_ok) || tri == SYM_NONE);
-    if (fast_ok && !big && tri == SYM_NONE) {
+    const bool fast = a.sym == SYM_NONE && b.sym == SYM_NONE && m >= bm && n >= bm &&
+                      a.ld <= FAST_LD_MAX && b.ld <= FAST_LD_MAX;
+    if (fast && !big && tri == SYM_NONE) {
         // few 64 x 64 tiles, long k: split k to fill the workgroup slots
         // (measured: 1024^3 32.8 -> 35.1 TFLOP/s, 512 x 512 x 4096 -> 37.4;
         // splitting 128 x 128 tiles instead lost to the larger fold)
         const int err = launch_splitk<T, 64>(s, g, m, n, k);
         if (err >= 0) return err;
     }
-    const int full_m = fast_ok ? m / bm : 0, full_n = fast_ok ? n / bm : 0;
-    const long fast_blocks = tri ? (long)full_m * (full_m + 1) / 2 : (long)full_m * full_n;
-    if (tri == SYM_NONE && fast_blocks > 0 && (m % bm || n % bm)) {
-        g.tiles_m = ceil_div(m, bm);
-        g.tiles_n = ceil_div(n, bm);
-        g.full_m = full_m;
-        g.full_n = full_n;
-        const unsigned blocks = (unsigned)((long)g.tiles_m * g.tiles_n);
-        const bool ua = !(a.vec_ok && b.vec_ok);
-#define GB_MIX(BM_, PA_, PB_)                                                                            hipLaunchKernelGGL((gemm_mixed_kernel<T, BM_, PA_, PB_>), dim3(blocks), dim3(256), 0, s, g)
-#define GB_MIX4(BM_, O, K)                                                                               if (a.form == PAT_OUTER && b.form == PAT_KCONT) GB_MIX(BM_, O, K);                               else if (a.form == PAT_OUTER) GB_MIX(BM_, O, O);                                                 else if (b.form == PAT_KCONT) GB_MIX(BM_, K, K);                                                 else GB_MIX(BM_, K, O)
-        PROF_BEGIN(s, kname<T>(big, 1));
-        if (big) {
-            if (ua) { GB_MIX4(128, PAT_OUTER_U, PAT_KCONT_U); }
-            else { GB_MIX4(128, PAT_OUTER, PAT_KCONT); }
-        } else {
-            if (ua) { GB_MIX4(64, PAT_OUTER_U, PAT_KCONT_U); }
-            else { GB_MIX4(64, PAT_OUTER, PAT_KCONT); }
-        }
-        PROF_END(s);
-#undef GB_MIX4
-#undef GB_MIX
-        return (int)hipGetLastError();
-    }
-    if (fast_blocks > 0) {
-        GemmArgs<T> f = g;
-        f.tiles_m = full_m;
-        f.tiles_n = full_n;
-        f.full_m = f.full_n = 0;
-        // A last round of 128 x 128 tiles that would leave most of the chip
-        // idle runs as 64 x 64 quarters instead (a quarter of the time).
-        const long slots = fast_slots(), tail = fast_blocks % slots;
-        const long main_blocks =
-            (big && fast_blocks > slots && 2 * tail < slots) ? fast_blocks - tail : fast_blocks;
-        PROF_BEGIN(s, kname<T>(big, 1));
-        if (big) launch_fast<T, 128>(s, f, (unsigned)main_blocks);
-        else launch_fast<T, 64>(s, f, (unsigned)fast_blocks);
-        if (main_blocks < fast_blocks)
-            launch_fast_sub<T>(s, f, (int)main_blocks, (unsigned)(4 * (fast_blocks - main_blocks)));
-        PROF_END(s);
-    }
     g.tiles_m = ceil_div(m, bm);
     g.tiles_n = ceil_div(n, bm);
-    g.full_m = full_m;
-    g.full_n = full_n;
     const long blocks = tri ? (long)g.tiles_m * (g.tiles_m + 1) / 2 : (long)g.tiles_m * g.tiles_n;
-    if (blocks > fast_blocks) {
-        PROF_BEGIN(s, kname<T>(big, 0));
-        if (big)
-            hipLaunchKernelGGL((gemm_mfma_kernel<T, 128, 128, 16>), dim3((unsigned)blocks),
-                               dim3(256), 0, s, g);
-        else
-            hipLaunchKernelGGL((gemm_mfma_kernel<T, 64, 64, 16>), dim3((unsigned)blocks),
-                               dim3(256), 0, s, g);
-        PROF_END(s);
+    PROF_BEGIN(s, kname<T>(big, fast));
+    if (fast) {
+        // A last round of 128 x 128 tiles that would leave most of the chip
+        // idle runs as 64 x 64 quarters instead (a quarter of the time).
+        const long slots = fast_slots(), tail = blocks % slots;
+        const long main_blocks = (big && blocks > slots && 2 * tail < slots) ? blocks - tail : blocks;
+        if (big) launch_fast<T, 128>(s, g, (unsigned)main_blocks);
+        else launch_fast<T, 64>(s, g, (unsigned)blocks);
+        if (main_blocks < blocks)
+            launch_fast_sub<T>(s, g, (int)main_blocks, (unsigned)(4 * (blocks - main_blocks)));
+    } else if (big) {
+        hipLaunchKernelGGL((gemm_mfma_kernel<T, 128, 128, 16>), dim3((unsigned)blocks), dim3(256), 0,
+                           s, g);
+    } else {
+        hipLaunchKernelGGL((gemm_mfma_kernel<T, 64, 64, 16>), dim3((unsigned)blocks), dim3(256), 0, s,
+                           g);
     }
+    PROF_END(s);
     return (int)hipGetLastError();
 }
 
@@ -481,13 +401,14 @@ __global__ __launch_bounds__(256) void symmetrize_kernel(int n, const T *__restr
     }
 }
 
-// C = alpha*op(A)*op(B) where one factor is a full-tile triangle: tile
+// C = alpha*op(A)*op(B) where one factor is a triangle: tile
 // (tm, tn) runs only over the k range where that factor is nonzero (the
 // other products are exact zeros), so a triangular multiply costs half a
 // GEMM.  KR: 1 k < (tm+1)*BM, 2 k >= tm*BM (left factor lower / upper),
 // 3 k >= tn*BM, 4 k < (tn+1)*BM (right factor lower / upper).  Operand
 // pointers are shifted to the range start as in the split-K kernel; tiles
-// are dispatched longest range first.
+// are dispatched longest range first.  (A ragged last tile is moved back, but
+// stores only its own rows and columns, for which the range is right.)
 template <typename T, int BM, int PA, int PB, int KR>
 __global__ __launch_bounds__(256, 2) void gemm_fast_krange_kernel(GemmArgs<T> g)
 {
@@ -601,16 +522,15 @@ template <typename T, int BM>
 int launch_krange(hipStream_t s, int m, int n, int k, T alpha, const Operand<T> &a,
                   const Operand<T> &b, T *C, long ldc, int kr)
 {
-    if (m % BM || n % BM || !a.vec_ok || !b.vec_ok) return -1;
+    if (m < BM || n < BM || a.ld > FAST_LD_MAX || b.ld > FAST_LD_MAX) return -1;
     GemmArgs<T> g;
     g.m = m; g.n = n; g.k = k;
     g.alpha = alpha; g.beta = T(0);
     g.a = a; g.b = b;
     g.C = C; g.ldc = ldc;
     g.tri = SYM_NONE;
-    g.tiles_m = m / BM;
-    g.tiles_n = n / BM;
-    g.full_m = g.full_n = 0;
+    g.tiles_m = ceil_div(m, BM);
+    g.tiles_n = ceil_div(n, BM);
     const unsigned blocks = (unsigned)(g.tiles_m * g.tiles_n);
 #define GB_KR(PA_, PB_)                                                                          \
     do {                                                                                         \
@@ -690,8 +610,9 @@ int trmm_entry(void *stream, char side, char uplo, char transa, char diag, int m
                                   : make_op<T>(Tm, ldt, n, tn ? PAT_KCONT : PAT_OUTER, SYM_NONE);
         const int k = left ? m : n;
         const int kr = left ? (oplower ? 1 : 2) : (oplower ? 3 : 4);
-        const long t128 = (long)(m / 128) * (n / 128);
-        err = t128 >= 256 ? launch_krange<T, 128>(s, m, n, k, alpha, a, b, W, ldw, kr)
+        const long t128 = (long)ceil_div(m, 128) * ceil_div(n, 128);
+        err = t128 >= 256 && m >= 128 && n >= 128
+                          ? launch_krange<T, 128>(s, m, n, k, alpha, a, b, W, ldw, kr)
                           : launch_krange<T, 64>(s, m, n, k, alpha, a, b, W, ldw, kr);
         if (err < 0) err = launch_gemm<T>(s, m, n, k, alpha, a, b, T(0), W, ldw, SYM_NONE);
     }

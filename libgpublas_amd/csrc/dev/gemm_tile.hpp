@@ -23,13 +23,6 @@
 namespace {
 
 enum { PAT_OUTER = 0, PAT_KCONT = 1, PAT_ELEM = 2 };
-// Template-only patterns of the fast tile: full tiles of an operand that is
-// not 16-B aligned (or whose leading dimension is odd), read in the OUTER /
-// KCONT layout with one element per load and no bounds checks.  Same values
-// in the same LDS places as the aligned patterns, hence the same bits.
-enum { PAT_OUTER_U = 3, PAT_KCONT_U = 4 };
-__host__ __device__ constexpr int pat_base(int p) { return p >= PAT_OUTER_U ? p - PAT_OUTER_U : p; }
-__host__ __device__ constexpr bool pat_unaligned(int p) { return p >= PAT_OUTER_U; }
 enum { SYM_NONE = 0, SYM_LOWER = 1, SYM_UPPER = 2 };
 
 // One operand of the product as the loader sees it: element (o, k) of the
@@ -58,7 +51,6 @@ struct GemmArgs {
     long ldc;
     int tiles_m, tiles_n;
     int tri;  // 0 rectangular grid, SYM_LOWER / SYM_UPPER: triangular tile grid + mask
-    int full_m, full_n;  // generic kernel: tiles below both counts were done by the fast kernel
 };
 
 __device__ __forceinline__ bool stored(int sym, long r, long c)
@@ -140,34 +132,57 @@ struct TileLoader {
         }
     }
 
-    // Fast path: full tile, pattern fixed at compile time; a vector load per
-    // VEC elements when the operand is aligned (UA false), one load per
-    // element otherwise.
-    template <int PAT, bool UA = false>
-    __device__ __forceinline__ static void load_pat(const Operand<T> &op, int o0, int k0,
+    // Fast path: the R rows of the tile all exist, pattern fixed at compile
+    // time.  `base` is the tile's first element (uniform over the workgroup),
+    // so a load is one 32-bit lane offset (voff) on a scalar address that the
+    // scalar unit advances; per-lane 64-bit addresses for the 2 * NV loads of
+    // a k-tile cost the registers that the fragment double buffer needs.
+    // Operands may have any alignment: 16-byte loads that are only
+    // element-aligned are legal in global memory.
+    typedef T VecU __attribute__((ext_vector_type(VEC), aligned(sizeof(T))));
+    static constexpr int OUTER_K = 256 * VEC / R;   // k rows one pass covers (PAT_OUTER)
+    static constexpr int KCONT_O = 256 * VEC / BK;  // operand rows one pass covers (PAT_KCONT)
+
+    template <int PAT> __device__ __forceinline__ static unsigned voff(long ld)
+    {
+        const unsigned t = threadIdx.x, l = (unsigned)ld;
+        return (PAT == PAT_OUTER ? (t % (R / VEC)) * VEC + (t / (R / VEC)) * l
+                                 : (t % (BK / VEC)) * VEC + (t / (BK / VEC)) * l) *
+               (unsigned)sizeof(T);
+    }
+    template <int PAT>
+    __device__ __forceinline__ static void load_pat(const T *base, long ld, unsigned vo,
                                                     Vec (&st)[NV])
+    {
+        const long step = (PAT == PAT_OUTER ? OUTER_K : KCONT_O) * ld;
+#pragma unroll
+        for (int r = 0; r < NV; ++r)
+            st[r] = *(const VecU *)((const char *)(base + r * step) + (size_t)vo);
+    }
+    // The last k-tile when only krem < BK of its k rows exist: rows past them
+    // read as zero (their addresses stay on the last row that exists).
+    template <int PAT>
+    __device__ __forceinline__ static void load_ktail(const T *base, long ld, int krem,
+                                                      Vec (&st)[NV])
     {
         const int t = threadIdx.x;
 #pragma unroll
         for (int r = 0; r < NV; ++r) {
-            const int v = t + r * 256;
             if (PAT == PAT_OUTER) {
-                const int o = (v % (R / VEC)) * VEC, kk = v / (R / VEC);
-                const T *src = op.p + (long)(o0 + o) + (long)(k0 + kk) * op.ld;
-                if (UA) {
+                const int o = (t % (R / VEC)) * VEC, kk = t / (R / VEC) + r * OUTER_K;
+                const unsigned off = (unsigned)min(kk, krem - 1) * (unsigned)ld + (unsigned)o;
+                const Vec x = *(const VecU *)((const char *)base + (size_t)(off * (unsigned)sizeof(T)));
 #pragma unroll
-                    for (int e = 0; e < VEC; ++e) st[r][e] = src[e];
-                } else {
-                    st[r] = *(const Vec *)src;
-                }
+                for (int e = 0; e < VEC; ++e) st[r][e] = kk < krem ? x[e] : T(0);
             } else {
-                const int kk = (v % (BK / VEC)) * VEC, o = v / (BK / VEC);
-                const T *src = op.p + (long)(k0 + kk) + (long)(o0 + o) * op.ld;
-                if (UA) {
+                const int kk = (t % (BK / VEC)) * VEC, o = t / (BK / VEC);
+                const T *row = base + r * (KCONT_O * ld);
 #pragma unroll
-                    for (int e = 0; e < VEC; ++e) st[r][e] = src[e];
-                } else {
-                    st[r] = *(const Vec *)src;
+                for (int e = 0; e < VEC; ++e) {
+                    const unsigned off =
+                        (unsigned)o * (unsigned)ld + (unsigned)min(kk + e, krem - 1);
+                    const T x = *(const T *)((const char *)row + (size_t)(off * (unsigned)sizeof(T)));
+                    st[r][e] = kk + e < krem ? x : T(0);
                 }
             }
         }
@@ -366,118 +381,260 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs<T> &g, int tm, int tn,
     }
 }
 
-// Full C tile (tm, tn) of g with access patterns PA / PB fixed at compile
-// time: no per-element selects or bounds checks in the main loop (only a
-// partial last k-tile takes guarded element loads).  PAT_OUTER / PAT_KCONT:
-// both operands 16-B aligned with leading dimensions a multiple of the
-// vector width (vector loads); PAT_OUTER_U / PAT_KCONT_U: any alignment (one
-// load per element).  Same k order and epilogue as gemm_tile, hence the same
-// bits.
-// EDGE: a ragged tile (rows past m or columns past n, any k): every load
-// guarded (load_guard) and the epilogue bounded; elements past an operand's
-// end read as zero, as in gemm_tile, so the bits are still the same.
-template <typename T, int BM, int BN, int BK, int PA_, int PB_, int TRI, bool EDGE = false>
+// Fragments of one k step of 4 from a staged k-tile, and the products of one
+// step: lane l of a wave holds row l%16 (of each 16-row block) at k = kk + l/16.
+template <typename T, int BM, int BN, int BK>
+struct TileMath {
+    static constexpr int PAD = 128 / (int)sizeof(T);
+    static constexpr int WM = BM / 2, WN = BN / 2, FM = WM / 16, FN = WN / 16;
+    typedef typename Mfma<T>::Acc Acc;
+
+    __device__ __forceinline__ static void fetch(const T (*A)[BM + PAD], const T (*B)[BN + PAD],
+                                                 int kk, T (&fa)[FM], T (&fb)[FN])
+    {
+        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+        const int wm = wave & 1, wn = wave >> 1, kr = kk + (lane >> 4);
+        // (c0 + l) ^ swz = (c0 ^ shi) + (l ^ slo) for c0 a multiple of 16 and
+        // l < 16: the high part of the swizzle depends on kk alone (a
+        // constant of the unrolled loop), so the fragment offsets stay
+        // immediate; the low part is one lane-dependent term per step
+        const int shi = lds_swz<T>(kk) & ~15;
+        const int lo = (lane & 15) ^ (lds_swz<T>(kr) & 15);
+#pragma unroll
+        for (int i = 0; i < FM; ++i) fa[i] = A[kr][((wm * WM + i * 16) ^ shi) + lo];
+#pragma unroll
+        for (int j = 0; j < FN; ++j) fb[j] = B[kr][((wn * WN + j * 16) ^ shi) + lo];
+    }
+    __device__ __forceinline__ static void multiply(const T (&fa)[FM], const T (&fb)[FN],
+                                                    Acc (&acc)[FM][FN])
+    {
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) acc[i][j] = Mfma<T>::mma(fb[j], fa[i], acc[i][j]);
+    }
+    // Accumulator (i, j) element r of this lane is C[row][col] with row = m0 +
+    // wm*WM + i*16 + lane%16, col = n0 + wn*WN + j*16 + drow(lane, r); written
+    // where row >= rlo, col >= clo, inside g and inside the triangle.  The 16
+    // columns of a row block are read together before any of them is written
+    // (one memory round trip per row block where beta is not 0); elements that
+    // are not written read the tile's first one instead, so no load is skipped
+    // by a branch.
+    template <int TRI, bool BOUND>
+    __device__ __forceinline__ static void finish(const GemmArgs<T> &g, int m0, int n0, int rlo,
+                                                  int clo, const Acc (&acc)[FM][FN])
+    {
+        const bool inner = !BOUND && m0 == rlo && n0 == clo &&
+                           (TRI == SYM_NONE || (TRI == SYM_LOWER ? m0 >= n0 + BN : n0 >= m0 + BM));
+        if (inner) finish_part<TRI, BOUND, true>(g, m0, n0, rlo, clo, acc);
+        else finish_part<TRI, BOUND, false>(g, m0, n0, rlo, clo, acc);
+    }
+    template <int TRI, bool BOUND, bool INNER>
+    __device__ __forceinline__ static void finish_part(const GemmArgs<T> &g, int m0, int n0, int rlo,
+                                                       int clo, const Acc (&acc)[FM][FN])
+    {
+        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+        const int gi0 = m0 + (wave & 1) * WM + (lane & 15);
+        const int gj0 = n0 + (wave >> 1) * WN + Mfma<T>::drow(lane, 0);
+        constexpr int DR = sizeof(T) == 8 ? 4 : 1;  // columns from element r to r + 1
+        const T alpha = g.alpha, beta = g.beta;
+        T *const c0 = g.C + gi0 + (long)gj0 * g.ldc;
+        const T *const any = g.C + rlo + (long)clo * g.ldc;
+#pragma unroll
+        for (int i = 0; i < FM; ++i) {
+            const int gi = gi0 + i * 16;
+            auto in = [&](int j, int r) {
+                const int gj = gj0 + j * 16 + r * DR;
+                return INNER || (gi >= rlo && gj >= clo && (!BOUND || (gi < g.m && gj < g.n)) &&
+                                 (TRI == SYM_NONE || (TRI == SYM_LOWER ? gi >= gj : gi <= gj)));
+            };
+            T v[FN][4];
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) v[j][r] = alpha * acc[i][j][r];
+            if (beta != T(0)) {
+                T old[FN][4];
+#pragma unroll
+                for (int j = 0; j < FN; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        old[j][r] = *(in(j, r) ? c0 + i * 16 + (long)(j * 16 + r * DR) * g.ldc : any);
+#pragma unroll
+                for (int j = 0; j < FN; ++j)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) v[j][r] += beta * old[j][r];
+            }
+#pragma unroll
+            for (int j = 0; j < FN; ++j)
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (in(j, r)) c0[i * 16 + (long)(j * 16 + r * DR) * g.ldc] = v[j][r];
+        }
+    }
+};
+
+// Leading dimensions that the fast tile's 32-bit lane offsets reach (a pass
+// of one operand covers at most 64 rows of its leading dimension).
+constexpr long FAST_LD_MAX = 1l << 23;
+
+// C tile (tm, tn) of g with access patterns PA / PB fixed at compile time, for
+// m >= BM and n >= BN.  The last tile of a ragged dimension is moved back to
+// end at the matrix's edge: it recomputes a few rows (columns) of its
+// neighbour and does not store them, so every load is a full, unguarded
+// vector load of any alignment.  Same k order and epilogue as gemm_tile, hence
+// the same bits.
+//
+// Pipeline (bound: the matrix cores; LDS and memory have to stay out of their
+// way): k-tile t+2 travels from memory to registers while t is multiplied,
+// t+1 is stored to the other LDS buffer during the first k step of t, and the
+// fragments of a k step are read during the step before it -- across the one
+// barrier of a k-tile too, which therefore sits in front of a step's products
+// and not in front of its reads.  The barrier waits for LDS traffic alone.
+// Measured against reads in front of each step and guarded edge tiles: FP64
+// 8192^3 NT 65.3 -> 68.0 TFLOP/s, FP32 4096^3 NN 121 -> 130, FP64 2047 x 1531 x
+// 1789 TN on odd leading dimensions 44.4 -> 58.7, 100^3 13.5 -> 8.4 us.  (More
+// than 256 registers a lane make the compiler move the accumulators to and
+// from the accumulation registers in every k-tile: 48 TFLOP/s.)
+template <typename T, int BM, int BN, int BK, int PA, int PB, int TRI>
 __device__ __forceinline__ void gemm_fast_tile(const GemmArgs<T> &g, int tm, int tn,
                                                T (*As)[BK][BM + 128 / sizeof(T)],
                                                T (*Bs)[BK][BN + 128 / sizeof(T)])
 {
-    constexpr int PA = pat_base(PA_), PB = pat_base(PB_);
-    constexpr bool UA = pat_unaligned(PA_), UB = pat_unaligned(PB_);
-    constexpr int PAD = 128 / (int)sizeof(T);
-    constexpr int WM = BM / 2, WN = BN / 2, FM = WM / 16, FN = WN / 16;
+    typedef TileMath<T, BM, BN, BK> M;
     typedef TileLoader<T, BM, BK> LA;
     typedef TileLoader<T, BN, BK> LB;
-    typedef typename Mfma<T>::Acc Acc;
+    constexpr int STEPS = BK / 4;
+    static_assert(STEPS % 2 == 0, "the fragment buffers alternate over a k-tile");
 
-    const int m0 = tm * BM, n0 = tn * BN;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int wm = wave & 1, wn = wave >> 1;
-    const int K = g.k;
-    const int ktiles = (K + BK - 1) / BK;
+    const int m0 = min(tm * BM, g.m - BM), n0 = min(tn * BN, g.n - BN);
+    const int K = g.k, kfull = K / BK, ktiles = (K + BK - 1) / BK;
+    const long lda = g.a.ld, ldb = g.b.ld;
+    const T *pa = g.a.p + (PA == PAT_OUTER ? (long)m0 : (long)m0 * lda);
+    const T *pb = g.b.p + (PB == PAT_OUTER ? (long)n0 : (long)n0 * ldb);
+    const long stepa = PA == PAT_OUTER ? BK * lda : BK, stepb = PB == PAT_OUTER ? BK * ldb : BK;
+    const unsigned va = LA::template voff<PA>(lda), vb = LB::template voff<PB>(ldb);
 
-    Acc acc[FM][FN];
+    typename M::Acc acc[M::FM][M::FN];
 #pragma unroll
-    for (int i = 0; i < FM; ++i)
+    for (int i = 0; i < M::FM; ++i)
 #pragma unroll
-        for (int j = 0; j < FN; ++j) acc[i][j] = Acc{};
+        for (int j = 0; j < M::FN; ++j) acc[i][j] = typename M::Acc{};
 
     typename LA::Vec sa[LA::NV];
     typename LB::Vec sb[LB::NV];
-    auto load = [&](int k0) -> bool {
-        if (EDGE) {
-            LA::template load_guard<PA>(g.a, m0, k0, K, sa);
-            LB::template load_guard<PB>(g.b, n0, k0, K, sb);
-            return false;  // laid out as the patterns
-        }
-        if (k0 + BK <= K) {
-            LA::template load_pat<PA, UA>(g.a, m0, k0, sa);
-            LB::template load_pat<PB, UB>(g.b, n0, k0, sb);
-            return false;
-        }
-        LA::load(g.a, m0, k0, K, PAT_ELEM, sa);
-        LB::load(g.b, n0, k0, K, PAT_ELEM, sb);
-        return true;
+    // the next k-tile into registers; pa / pb are uniform and move on
+    auto load_full = [&]() {
+        LA::template load_pat<PA>(pa, lda, va, sa);
+        LB::template load_pat<PB>(pb, ldb, vb, sb);
+        pa += stepa;
+        pb += stepb;
     };
-    auto store = [&](int buf, bool tail) {
-        if (!tail) {
-            LA::template store_pat<PA, BM + PAD>(As[buf], sa);
-            LB::template store_pat<PB, BN + PAD>(Bs[buf], sb);
+    auto load_any = [&](int t) {
+        if (t < kfull) {
+            load_full();
         } else {
-            LA::template store_pat<PAT_OUTER, BM + PAD>(As[buf], sa);
-            LB::template store_pat<PAT_OUTER, BN + PAD>(Bs[buf], sb);
+            LA::template load_ktail<PA>(pa, lda, K - t * BK, sa);
+            LB::template load_ktail<PB>(pb, ldb, K - t * BK, sb);
         }
     };
+    auto store = [&](int buf) {
+        LA::template store_pat<PA, BM + M::PAD>(As[buf], sa);
+        LB::template store_pat<PB, BN + M::PAD>(Bs[buf], sb);
+    };
+    T fa[2][M::FM], fb[2][M::FN];
 
-    store(0, load(0));
+    load_any(0);
+    store(0);
+    if (ktiles > 1) load_any(1);
+    lds_barrier();
+    M::fetch(As[0], Bs[0], 0, fa[0], fb[0]);
+    int kt = 0;
+    for (; kt + 2 < kfull; ++kt) {
+        const int cur = kt & 1;
+#pragma unroll
+        for (int st = 0; st < STEPS; ++st) {
+            if (st + 1 < STEPS) {
+                M::fetch(As[cur], Bs[cur], (st + 1) * 4, fa[(st + 1) & 1], fb[(st + 1) & 1]);
+            } else {
+                lds_barrier();
+                M::fetch(As[cur ^ 1], Bs[cur ^ 1], 0, fa[0], fb[0]);
+            }
+            if (st == 0) {
+                store(cur ^ 1);
+                load_full();
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            M::multiply(fa[st & 1], fb[st & 1], acc);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    for (; kt < ktiles; ++kt) {  // the last two k-tiles: nothing or the ragged one to load
+        const int cur = kt & 1;
+#pragma unroll
+        for (int st = 0; st < STEPS; ++st) {
+            if (st + 1 < STEPS) {
+                M::fetch(As[cur], Bs[cur], (st + 1) * 4, fa[(st + 1) & 1], fb[(st + 1) & 1]);
+            } else {
+                lds_barrier();
+                M::fetch(As[cur ^ 1], Bs[cur ^ 1], 0, fa[0], fb[0]);
+            }
+            if (st == 0 && kt + 1 < ktiles) {
+                store(cur ^ 1);
+                if (kt + 2 < ktiles) load_any(kt + 2);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            M::multiply(fa[st & 1], fb[st & 1], acc);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    M::template finish<TRI, false>(g, m0, n0, tm * BM, tn * BN, acc);
+}
+
+// The same tile where a dimension of C is smaller than the tile: every load
+// guarded (load_guard) and the epilogue bounded; elements past an operand's
+// end read as zero, as in gemm_tile, so the bits are still the same.
+template <typename T, int BM, int BN, int BK, int PA, int PB>
+__device__ __forceinline__ void gemm_edge_tile(const GemmArgs<T> &g, int tm, int tn,
+                                               T (*As)[BK][BM + 128 / sizeof(T)],
+                                               T (*Bs)[BK][BN + 128 / sizeof(T)])
+{
+    typedef TileMath<T, BM, BN, BK> M;
+    typedef TileLoader<T, BM, BK> LA;
+    typedef TileLoader<T, BN, BK> LB;
+    const int m0 = tm * BM, n0 = tn * BN, K = g.k, ktiles = (K + BK - 1) / BK;
+    typename M::Acc acc[M::FM][M::FN];
+#pragma unroll
+    for (int i = 0; i < M::FM; ++i)
+#pragma unroll
+        for (int j = 0; j < M::FN; ++j) acc[i][j] = typename M::Acc{};
+    typename LA::Vec sa[LA::NV];
+    typename LB::Vec sb[LB::NV];
+    auto load = [&](int k0) {
+        LA::template load_guard<PA>(g.a, m0, k0, K, sa);
+        LB::template load_guard<PB>(g.b, n0, k0, K, sb);
+    };
+    auto store = [&](int buf) {
+        LA::template store_pat<PA, BM + M::PAD>(As[buf], sa);
+        LB::template store_pat<PB, BN + M::PAD>(Bs[buf], sb);
+    };
+    load(0);
+    store(0);
     __syncthreads();
     for (int kt = 0; kt < ktiles; ++kt) {
         const int cur = kt & 1;
         const bool more = kt + 1 < ktiles;
-        bool tail = false;
-        if (more) tail = load((kt + 1) * BK);
+        if (more) load((kt + 1) * BK);
 #pragma unroll
         for (int kk = 0; kk < BK; kk += 4) {
-            T fa[FM], fb[FN];
-            const int kr = kk + (lane >> 4);
-            // (c0 + l) ^ swz = (c0 ^ shi) + (l ^ slo) for c0 a multiple of 16 and
-            // l < 16: the high part of the swizzle depends on kk alone (a
-            // constant of the unrolled loop), so the fragment offsets stay
-            // immediate; the low part is one lane-dependent term per step
-            const int shi = lds_swz<T>(kk) & ~15;
-            const int lo = (lane & 15) ^ (lds_swz<T>(kr) & 15);
-#pragma unroll
-            for (int i = 0; i < FM; ++i)
-                fa[i] = As[cur][kr][((wm * WM + i * 16) ^ shi) + lo];
-#pragma unroll
-            for (int j = 0; j < FN; ++j)
-                fb[j] = Bs[cur][kr][((wn * WN + j * 16) ^ shi) + lo];
-#pragma unroll
-            for (int i = 0; i < FM; ++i)
-#pragma unroll
-                for (int j = 0; j < FN; ++j) acc[i][j] = Mfma<T>::mma(fb[j], fa[i], acc[i][j]);
+            T fa[M::FM], fb[M::FN];
+            M::fetch(As[cur], Bs[cur], kk, fa, fb);
+            M::multiply(fa, fb, acc);
         }
-        if (more) store(cur ^ 1, tail);
+        if (more) store(cur ^ 1);
         __syncthreads();
     }
-
-    const T alpha = g.alpha, beta = g.beta;
-#pragma unroll
-    for (int i = 0; i < FM; ++i) {
-        const long gi = m0 + wm * WM + i * 16 + (lane & 15);
-#pragma unroll
-        for (int j = 0; j < FN; ++j) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const long gj = n0 + wn * WN + j * 16 + Mfma<T>::drow(lane, r);
-                if (EDGE && (gi >= g.m || gj >= g.n)) continue;
-                if (TRI == SYM_LOWER && gi < gj) continue;
-                if (TRI == SYM_UPPER && gi > gj) continue;
-                T *c = g.C + gi + gj * g.ldc;
-                const T v = alpha * acc[i][j][r];
-                *c = beta == T(0) ? v : v + beta * *c;
-            }
-        }
-    }
+    M::template finish<SYM_NONE, true>(g, m0, n0, m0, n0, acc);
 }
 
 inline bool is_n(char c) { return c == 'N' || c == 'n'; }

@@ -50,20 +50,18 @@ enum { TY_D = 0, TY_S = 1 };
 // (<= 4 KB) kernel argument
 constexpr int kCapGemm = 22, kCapGemv = 32, kCapTrsm = 48;
 
-// One GEMM of a group.  Its tiles split into interior tiles (g.full_m x
-// g.full_n, only when both operands allow the vector loads), run by the
-// fast kernel with the trans pattern `pat`, and edge tiles (the rest), run
-// by the generic kernel.  A product with few tiles and a long k is also
-// split along k into `ksplit` chunks of `kchunk` (a multiple of 16): chunk
-// s computes its tiles into part + s*m*n (alpha 1, beta 0) and the fold
-// kernel sums the chunks in order and applies alpha / beta.  The split
-// depends only on (m, n, k).
+// One GEMM of a group: all its tiles run on the fast tile with the trans
+// pattern `pat` where it is at least a tile wide in both dimensions, else all on
+// the guarded edge tile.  A product with few tiles and a long k is also split
+// along k into `ksplit` chunks of `kchunk` (a multiple of 16): chunk s computes
+// its tiles into part + s*m*n (alpha 1, beta 0) and the fold kernel sums the
+// chunks in order and applies alpha / beta.  The split depends only on (m, n, k).
 template <typename T>
 struct GGemm {
     GemmArgs<T> g;
     T *part;
     int fast_begin, edge_begin, fold_begin;
-    int pat;  // 0 NN, 1 NT, 2 TN, 3 TT; + 4: an operand not aligned (element loads)
+    int pat;  // 0 NN, 1 NT, 2 TN, 3 TT
     int ksplit, kchunk;
 };
 
@@ -151,63 +149,35 @@ __device__ __forceinline__ GemmArgs<T> chunk_args(const GGemm<T> &e, int s)
     return g;
 }
 
-// Full tile t of the group (numbered over its problems' fast tiles).
-template <typename T, int BM>
-__device__ __forceinline__ void fast_group_tile(const GemmGroup<T> &G, int np, int t,
-                                                T (*As)[16][BM + 128 / sizeof(T)],
-                                                T (*Bs)[16][BM + 128 / sizeof(T)])
+// Tile t of the group's fast problems (EDGE = false: at least a tile wide in
+// both dimensions) or of its narrow ones, numbered over the problems of that
+// class, chunks of a split problem one after the other.
+template <typename T, int BM, bool EDGE>
+__device__ __forceinline__ void group_tile(const GemmGroup<T> &G, int np, int t,
+                                           T (*As)[16][BM + 128 / sizeof(T)],
+                                           T (*Bs)[16][BM + 128 / sizeof(T)])
 {
-    const int p = find_unit(&G.p[0].fast_begin, sizeof(GGemm<T>), np, t);
-    const int per = G.p[p].g.full_m * G.p[p].g.full_n;
-    const int tl0 = t - G.p[p].fast_begin, tl = tl0 % per;
-    const GemmArgs<T> g = chunk_args(G.p[p], tl0 / per);
-    const int tm = tl % g.full_m, tn = tl / g.full_m;
+    const int p = find_unit(EDGE ? &G.p[0].edge_begin : &G.p[0].fast_begin, sizeof(GGemm<T>), np, t);
+    const int per = G.p[p].g.tiles_m * G.p[p].g.tiles_n;
+    const int t0 = t - (EDGE ? G.p[p].edge_begin : G.p[p].fast_begin), tl = t0 % per;
+    const GemmArgs<T> g = chunk_args(G.p[p], t0 / per);
+    const int tm = tl % g.tiles_m, tn = tl / g.tiles_m;
+#define GB_TILE(PA_, PB_)                                                                        \
+    do {                                                                                         \
+        if constexpr (EDGE) gemm_edge_tile<T, BM, BM, 16, PA_, PB_>(g, tm, tn, As, Bs);          \
+        else gemm_fast_tile<T, BM, BM, 16, PA_, PB_, SYM_NONE>(g, tm, tn, As, Bs);               \
+    } while (0)
     switch (G.p[p].pat) {
-    case 0: gemm_fast_tile<T, BM, BM, 16, PAT_OUTER, PAT_KCONT, SYM_NONE>(g, tm, tn, As, Bs); break;
-    case 1: gemm_fast_tile<T, BM, BM, 16, PAT_OUTER, PAT_OUTER, SYM_NONE>(g, tm, tn, As, Bs); break;
-    case 2: gemm_fast_tile<T, BM, BM, 16, PAT_KCONT, PAT_KCONT, SYM_NONE>(g, tm, tn, As, Bs); break;
-    case 3: gemm_fast_tile<T, BM, BM, 16, PAT_KCONT, PAT_OUTER, SYM_NONE>(g, tm, tn, As, Bs); break;
-    // operands not both aligned: element loads
-    case 4: gemm_fast_tile<T, BM, BM, 16, PAT_OUTER_U, PAT_KCONT_U, SYM_NONE>(g, tm, tn, As, Bs); break;
-    case 5: gemm_fast_tile<T, BM, BM, 16, PAT_OUTER_U, PAT_OUTER_U, SYM_NONE>(g, tm, tn, As, Bs); break;
-    case 6: gemm_fast_tile<T, BM, BM, 16, PAT_KCONT_U, PAT_KCONT_U, SYM_NONE>(g, tm, tn, As, Bs); break;
-    default: gemm_fast_tile<T, BM, BM, 16, PAT_KCONT_U, PAT_OUTER_U, SYM_NONE>(g, tm, tn, As, Bs); break;
+    case 0: GB_TILE(PAT_OUTER, PAT_KCONT); break;
+    case 1: GB_TILE(PAT_OUTER, PAT_OUTER); break;
+    case 2: GB_TILE(PAT_KCONT, PAT_KCONT); break;
+    default: GB_TILE(PAT_KCONT, PAT_OUTER); break;
     }
+#undef GB_TILE
 }
 
-// Ragged tile t of the group (numbered over its problems' edge tiles; a
-// problem's are the column strip past the full columns, all rows, followed
-// by the row strip past the full rows), on the guarded fast tile with the
-// problem's access patterns (element loads; same bits as the generic tile).
-template <typename T, int BM>
-__device__ __forceinline__ void edge_group_tile(const GemmGroup<T> &G, int np, int t,
-                                                T (*As)[16][BM + 128 / sizeof(T)],
-                                                T (*Bs)[16][BM + 128 / sizeof(T)])
-{
-    const int p = find_unit(&G.p[0].edge_begin, sizeof(GGemm<T>), np, t);
-    const int per = G.p[p].g.tiles_m * G.p[p].g.tiles_n - G.p[p].g.full_m * G.p[p].g.full_n;
-    const int e0 = t - G.p[p].edge_begin, e = e0 % per;
-    const GemmArgs<T> g = chunk_args(G.p[p], e0 / per);
-    const int strip = g.tiles_m * (g.tiles_n - g.full_n);
-    int tm, tn;
-    if (e < strip) {
-        tm = e % g.tiles_m;
-        tn = g.full_n + e / g.tiles_m;
-    } else {
-        const int e2 = e - strip, rows = g.tiles_m - g.full_m;
-        tm = g.full_m + e2 % rows;
-        tn = e2 / rows;
-    }
-    switch (G.p[p].pat & 3) {
-    case 0: gemm_fast_tile<T, BM, BM, 16, PAT_OUTER, PAT_KCONT, SYM_NONE, true>(g, tm, tn, As, Bs); break;
-    case 1: gemm_fast_tile<T, BM, BM, 16, PAT_OUTER, PAT_OUTER, SYM_NONE, true>(g, tm, tn, As, Bs); break;
-    case 2: gemm_fast_tile<T, BM, BM, 16, PAT_KCONT, PAT_KCONT, SYM_NONE, true>(g, tm, tn, As, Bs); break;
-    default: gemm_fast_tile<T, BM, BM, 16, PAT_KCONT, PAT_OUTER, SYM_NONE, true>(g, tm, tn, As, Bs); break;
-    }
-}
-
-// Every tile of the group, full ones first, in one grid: the ragged tiles
-// of a batch do not make a round of their own after the full ones.
+// Every tile of the group, the fast problems' first, in one grid: the narrow
+// problems of a batch do not make a round of their own after them.
 template <typename T, int BM>
 __device__ __forceinline__ void gemm_group_body(const GemmGroup<T> &G)
 {
@@ -218,9 +188,9 @@ __device__ __forceinline__ void gemm_group_body(const GemmGroup<T> &G)
     const int nf = BM == 32 ? 0 : G.fast_tiles, total = nf + G.edge_tiles;
     for (int t = blockIdx.x; t < total; t += gridDim.x) {
         if (t < nf) {
-            if constexpr (BM != 32) fast_group_tile<T, BM>(G, np, t, As, Bs);
+            if constexpr (BM != 32) group_tile<T, BM, false>(G, np, t, As, Bs);
         } else {
-            edge_group_tile<T, BM>(G, np, t - nf, As, Bs);
+            group_tile<T, BM, true>(G, np, t - nf, As, Bs);
         }
     }
 }
@@ -701,15 +671,10 @@ int add_gemm(gpublas_batch *b, char ta, char tb, int m, int n, int k, T alpha, c
     g.tiles_m = ceil_div(m, bm);
     g.tiles_n = ceil_div(n, bm);
     g.tri = SYM_NONE;
-    // interior tiles take the fast tile: vector loads when both operands
-    // allow them, element loads otherwise (the 32-wide shape has no fast
-    // variant)
-    const bool fast = cfg != CFG_32;
-    g.full_m = fast ? m / bm : 0;
-    g.full_n = fast ? n / bm : 0;
-    if (g.full_m == 0 || g.full_n == 0) g.full_m = g.full_n = 0;
-    e.pat = (g.a.form == PAT_OUTER ? 0 : 2) + (g.b.form == PAT_KCONT ? 0 : 1) +
-            (g.a.vec_ok && g.b.vec_ok ? 0 : 4);
+    // a problem at least a tile wide in both dimensions takes the fast tile
+    // (the 32-wide shape has no fast variant)
+    const bool fast = cfg != CFG_32 && m >= bm && n >= bm && lda <= FAST_LD_MAX && ldb <= FAST_LD_MAX;
+    e.pat = (g.a.form == PAT_OUTER ? 0 : 2) + (g.b.form == PAT_KCONT ? 0 : 1);
     // split along k when the tiles alone cannot spread over the CUs: about
     // 256 units, chunks of at least 256, partials of at most 16 MiB.  Counted
     // in 64 x 64 tiles whatever the tile shape, so every shape splits alike
@@ -735,8 +700,7 @@ int add_gemm(gpublas_batch *b, char ta, char tb, int m, int n, int k, T alpha, c
     }
     e.fast_begin = G.fast_tiles;
     e.edge_begin = G.edge_tiles;
-    G.fast_tiles += g.full_m * g.full_n * e.ksplit;
-    G.edge_tiles += (g.tiles_m * g.tiles_n - g.full_m * g.full_n) * e.ksplit;
+    (fast ? G.fast_tiles : G.edge_tiles) += g.tiles_m * g.tiles_n * e.ksplit;
     G.np++;
     return 0;
 }
