@@ -27,14 +27,13 @@
 //  * group_gemv_part_kernel / group_gemv_fold_kernel: y = alpha*op(A)*x +
 //    beta*y as column-block (N) or row-chunk (T) partial sums followed by a
 //    fixed-order fold; the split depends only on (m, n);
-//  * group_trsm_kernel: left-side triangular solves (m <= 1024), one
-//    workgroup per 16-column panel of B held in LDS, right-looking over
-//    16-row blocks (in-register substitution of the diagonal block, MFMA
-//    updates of the blocks below);
+//  * group_trsm_arg / _tab: left-side triangular solves (m <= 1024), one
+//    workgroup per 16-column panel of B (trsm_panel.hpp).
 // Roofline: GEMM tiles are MFMA-bound (2mnk flop), GEMV is HBM-bound
 // (8(mn + m + n) bytes), TRSM panels are bound by their sequential
 // substitution chain for small n.
 #include "gemm_tile.hpp"
+#include "trsm_panel.hpp"
 #include "gpublas_dev.h"
 
 #include <mutex>
@@ -411,144 +410,90 @@ __global__ __launch_bounds__(256) void group_gemv_fold_arg(const GemvGroup G) { 
 __global__ __launch_bounds__(256) void group_gemv_fold_tab(const GemvGroup *G) { gemv_fold_body(*G); }
 
 // ---- grouped TRSM (left side) ----------------------------------------------
-// One 1024-thread workgroup solves op(A) X = alpha B for a 16-column panel
-// of B with the panel resident in LDS (m <= 1024), right-looking over
-// 16-row blocks: the owner wave of block I substitutes X_I in registers
-// from the diagonal block, then every wave subtracts op(A)[J, I] X_I from
-// the blocks J it owns (J = wave + 16 s) with one MFMA chain per block.
-// The op(A) column blocks of the next step are loaded into registers while
-// the current step runs.  Subtractions reach each row of B in increasing
-// (forward) or decreasing (backward) block order, as in the netlib loop.
+// One workgroup per 16-column panel of B (trsm_panel.hpp).  Orders past 512
+// take two panels: the first 512 rows are solved, their X (still in LDS) is
+// applied to the rest, and the rest is solved.  Measured at orders 64..512 with
+// 256 right-hand sides each (4 problems): 113 -> 38 us against the 1024-thread
+// kernel that substituted 16 rows at a time between two barriers.
 constexpr int TR_MAXM = 1024;
-constexpr int TR_WAVES = 16;
+constexpr int TR_PART = 512;
 
-__device__ __forceinline__ double opa(const GTrsm &d, int i, int k)
+union TrsmLds {
+    PanelLds<2> two;
+    PanelLds<4> four;
+};
+
+__device__ __forceinline__ void trsm_part(const PanelArgs &p, int trans, TrsmLds &s)
 {
-    if (i >= d.m || k >= d.m) return 0.0;
-    return d.trans ? d.A[k + (long)i * d.lda] : d.A[i + (long)k * d.lda];
+    if (p.order <= 256) {
+        if (trans) trsm_panel<double, 2, true>(p, s.two);
+        else trsm_panel<double, 2, false>(p, s.two);
+    } else {
+        if (trans) trsm_panel<double, 4, true>(p, s.four);
+        else trsm_panel<double, 4, false>(p, s.four);
+    }
+    __syncthreads();  // the panel's LDS is free again, its rows are in memory
 }
 
-// op(A)[J rows, I cols] for the blocks J = wave + 16 s this wave will touch
-// at step I (J >= I forward, J <= I backward), in MFMA A-operand layout:
-// buf[s][u] = op(A)(16 J + l%16, 16 I + 4 u + l/16).
-__device__ __forceinline__ void trsm_load_col(const GTrsm &d, int I, int nb, int wave, int q0,
-                                              int cl, double (&buf)[4][4])
+// Rows [512, m) of the panel: alpha B - op(T)[rows, 0..511] X, X in s.X.
+__device__ __forceinline__ void trsm_rest(const PanelArgs &p, int m, const PanelLds<4> &s)
 {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int q0 = lane >> 4, cl = lane & 15;
+    const double *A = (const double *)p.A;
+    double *B = (double *)p.B;
+    for (int r0 = TR_PART + 16 * wave; r0 < m; r0 += 16 * TP_WAVES) {
+        const double *a = A + min(r0 + cl, m - 1) * p.si + q0 * p.sk;
+        double b[4];
+        v4d acc = {0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-        const int J = wave + TR_WAVES * s;
-        const bool need = J < nb && (d.fwd ? J >= I : J <= I);
+        for (int u = 0; u < 4; ++u) {
+            const int r = r0 + q0 + 4 * u;
+            b[u] = r < m && cl < p.cols ? p.alpha * B[r * p.ss + cl * p.rs] : 0.0;
+        }
+        for (int k = 0; k < TR_PART; k += 32) {
+            double f[8];
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
-            buf[s][u] = need ? opa(d, 16 * J + cl, 16 * I + 4 * u + q0) : 0.0;
+            for (int u = 0; u < 8; ++u) f[u] = a[(long)(k + 4 * u) * p.sk];
+#pragma unroll
+            for (int u = 0; u < 8; ++u)
+                acc = __builtin_amdgcn_mfma_f64_16x16x4f64(f[u], s.X[k + 4 * u + q0][cl], acc, 0, 0, 0);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int r = r0 + q0 + 4 * u;
+            if (r < m && cl < p.cols) B[r * p.ss + cl * p.rs] = b[u] - acc[u];
+        }
     }
+    __syncthreads();
 }
 
 __device__ __forceinline__ void trsm_group_body(const TrsmGroup &G)
 {
-    __shared__ double Bs[TR_MAXM][17];
-    __shared__ double Ds[16][17];
+    __shared__ TrsmLds s;
     const int np = min(G.np, kCapTrsm);
     const int total = G.units;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int q0 = lane >> 4, cl = lane & 15;
     for (int u = blockIdx.x; u < total; u += gridDim.x) {
-        const int p = find_unit(&G.p[0].unit_begin, sizeof(GTrsm), np, u);
-        const GTrsm d = G.p[p];
+        const int i = find_unit(&G.p[0].unit_begin, sizeof(GTrsm), np, u);
+        const GTrsm d = G.p[i];
         const int c0 = (u - d.unit_begin) * 16;
-        const int nb = (d.m + 15) / 16;
-        const int rows = nb * 16;
-        // alpha * B panel into LDS, zero past m and past n
-        for (int idx = threadIdx.x; idx < rows * 16; idx += 1024) {
-            const int r = idx % rows, c = idx / rows;
-            double v = 0.0;
-            if (r < d.m && c0 + c < d.n) v = d.alpha * d.B[r + (long)(c0 + c) * d.ldb];
-            Bs[r][c] = v;
-        }
-        double cur[4][4], nxt[4][4];
-        trsm_load_col(d, d.fwd ? 0 : nb - 1, nb, wave, q0, cl, cur);
-        __syncthreads();
-        for (int st = 0; st < nb; ++st) {
-            const int I = d.fwd ? st : nb - 1 - st;
-            const int I0 = 16 * I;
-            if (st + 1 < nb) trsm_load_col(d, d.fwd ? I + 1 : I - 1, nb, wave, q0, cl, nxt);
-            if (wave == (I & (TR_WAVES - 1))) {
-                // diagonal block (identity past m; unit diagonal if asked)
-#pragma unroll
-                for (int s = 0; s < 4; ++s) {
-                    if (s != I / TR_WAVES) continue;
-#pragma unroll
-                    for (int v = 0; v < 4; ++v) {
-                        const int k = 4 * v + q0;
-                        double a = cur[s][v];
-                        if (k == cl && (d.unit || I0 + cl >= d.m)) a = 1.0;
-                        Ds[cl][k] = a;
-                    }
-                }
-                double t[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) t[e] = Bs[I0 + q0 + 4 * e][cl];
-                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                __builtin_amdgcn_wave_barrier();
-                if (d.fwd) {
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const int q = r & 3, e = r >> 2;
-                        const double v = t[e] / Ds[r][r];
-                        const double xr = __shfl(v, cl + 16 * q);
-                        if (q0 == q) t[e] = xr;
-#pragma unroll
-                        for (int e2 = 0; e2 < 4; ++e2)
-                            if (q0 + 4 * e2 > r) t[e2] = fma(-Ds[q0 + 4 * e2][r], xr, t[e2]);
-                    }
-                } else {
-#pragma unroll
-                    for (int r = 15; r >= 0; --r) {
-                        const int q = r & 3, e = r >> 2;
-                        const double v = t[e] / Ds[r][r];
-                        const double xr = __shfl(v, cl + 16 * q);
-                        if (q0 == q) t[e] = xr;
-#pragma unroll
-                        for (int e2 = 0; e2 < 4; ++e2)
-                            if (q0 + 4 * e2 < r) t[e2] = fma(-Ds[q0 + 4 * e2][r], xr, t[e2]);
-                    }
-                }
-                const bool cok = c0 + cl < d.n;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const int row = I0 + q0 + 4 * e;
-                    Bs[row][cl] = t[e];
-                    if (cok && row < d.m) d.B[row + (long)(c0 + cl) * d.ldb] = t[e];
-                }
+        PanelArgs p = panel_args<double>(d.A, d.lda, !d.trans, d.fwd, d.unit, d.B + (long)c0 * d.ldb, 1,
+                                         d.ldb, d.m, min(16, d.n - c0), d.alpha);
+        for (int left = d.m; left > 0; left -= TR_PART) {
+            if (left < d.m) {  // past the first part
+                trsm_rest(p, d.m, s.four);
+                p.A = (const double *)p.A + TR_PART * (p.si + p.sk);
+                p.B = (double *)p.B + TR_PART * p.ss;
+                p.alpha = 1.0;
             }
-            __syncthreads();
-            // B_J -= op(A)[J, I] X_I for this wave's remaining blocks
-#pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                const int J = wave + TR_WAVES * s;
-                if (J >= nb || (d.fwd ? J <= I : J >= I)) continue;
-                const int J0 = 16 * J;
-                v4d acc;
-#pragma unroll
-                for (int r = 0; r < 4; ++r) acc[r] = Bs[J0 + q0 + 4 * r][cl];
-#pragma unroll
-                for (int v = 0; v < 4; ++v)
-                    acc = __builtin_amdgcn_mfma_f64_16x16x4f64(-cur[s][v], Bs[I0 + 4 * v + q0][cl],
-                                                              acc, 0, 0, 0);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) Bs[J0 + q0 + 4 * r][cl] = acc[r];
-            }
-            __syncthreads();
-#pragma unroll
-            for (int s = 0; s < 4; ++s)
-#pragma unroll
-                for (int v = 0; v < 4; ++v) cur[s][v] = nxt[s][v];
+            p.order = min(left, TR_PART);
+            trsm_part(p, d.trans, s);
         }
     }
 }
 
-__global__ __launch_bounds__(1024) void group_trsm_arg(const TrsmGroup G) { trsm_group_body(G); }
-__global__ __launch_bounds__(1024) void group_trsm_tab(const TrsmGroup *G) { trsm_group_body(*G); }
+__global__ __launch_bounds__(TP_THREADS) void group_trsm_arg(const TrsmGroup G) { trsm_group_body(G); }
+__global__ __launch_bounds__(TP_THREADS) void group_trsm_tab(const TrsmGroup *G) { trsm_group_body(*G); }
 
 // ---- tile-shape table (autotuned) ------------------------------------------
 // Bucket = (round(log2 sqrt(m n)), round(log2 k)), each clamped to 5..11.
@@ -603,7 +548,7 @@ int cfg_bm(int cfg) { return cfg == CFG_32 ? 32 : cfg == CFG_64 ? 64 : 128; }
 // grid of each persistent kernel: enough workgroups to fill 256 CUs at the
 // kernel's occupancy (double / single), capped by the work when eager
 constexpr int kGridGemm[2][kCfgs] = {{1024, 512, 512}, {1024, 512, 512}};  // 2 per CU from 64
-constexpr int kGridGemv = 1024, kGridFold = 512, kGridTrsm = 256;  // TRSM: 1024-thread groups
+constexpr int kGridGemv = 1024, kGridFold = 512, kGridTrsm = 256;  // TRSM: one per CU (LDS)
 constexpr size_t kWsDoubles = (size_t)8 << 20;  // 64 MiB of GEMV partial sums
 
 }  // namespace
@@ -795,7 +740,7 @@ void enqueue(gpublas_batch *b, unsigned mask, bool capture)
                 if (gf) hipLaunchKernelGGL(group_gemv_fold_arg, dim3(gf), dim3(256), 0, s0, t->gv);
             } else {
                 const int g = t->tr.units < kGridTrsm ? t->tr.units : kGridTrsm;
-                hipLaunchKernelGGL(group_trsm_arg, dim3(g), dim3(1024), 0, s0, t->tr);
+                hipLaunchKernelGGL(group_trsm_arg, dim3(g), dim3(TP_THREADS), 0, s0, t->tr);
             }
             (void)hipEventRecord(b->ev_kind[k], s0);
         }
@@ -819,7 +764,7 @@ void enqueue(gpublas_batch *b, unsigned mask, bool capture)
         hipLaunchKernelGGL(group_gemv_fold_tab, dim3(kGridFold), dim3(256), 0, sv, &b->d_tab->gv);
     }
     if (mask & 128u)
-        hipLaunchKernelGGL(group_trsm_tab, dim3(kGridTrsm), dim3(1024), 0, st, &b->d_tab->tr);
+        hipLaunchKernelGGL(group_trsm_tab, dim3(kGridTrsm), dim3(TP_THREADS), 0, st, &b->d_tab->tr);
     (void)hipEventRecord(b->ev_join[0], sg);
     (void)hipEventRecord(b->ev_join[1], sv);
     (void)hipEventRecord(b->ev_join[2], st);

@@ -1,0 +1,347 @@
+// trsm_panel.hpp -- triangular solve of one panel of 16 right-hand sides on
+// the FP64 matrix cores, shared by the per-call solves (trsm.hip) and the
+// grouped ones of the serving loop (group.hip).
+//
+// One 512-thread workgroup solves op(T) X = alpha B for an order of at most
+// 128 * SB, in blocks of 16 rows.  The four lower / upper, plain / transposed
+// forms are one: the rows are numbered in the order in which they are solved,
+// and op(T)(i, k) = A[i * si + k * sk], B(i, c) = B[i * ss + c * rs] with
+// strides of either sign reach them.  FP32 operands are solved in FP64 and
+// rounded once.
+//
+//  * Prologue: the 16 x 16 diagonal blocks are inverted in LDS, four per wave,
+//    one lane per column, while the panel's loads are still in flight.
+//  * Wave w keeps the sums of T[J, I] X_I over the solved blocks I for its blocks
+//    J = w, w + 8, ... in MFMA accumulators.  When X of block st is published,
+//    every wave adds T[J, st] X_st for its later blocks, the owner of block st + 1
+//    that one first: it then forms X = inv(T_JJ) (B_J - sum) (the accumulator
+//    layout is the operand layout) and publishes it.
+//  * No barrier between steps: X_st is followed by a flag word in LDS, and a
+//    wave waits for that word alone, so the chain of solves never waits for
+//    the other blocks' updates.  The next owner reads word and X together (LDS
+//    serves one wave's requests in order, so X is valid if the word was set).
+//    All eight waves are resident and each publishes its blocks in increasing
+//    order from words of lower blocks, so every wait ends.
+//  * op(T) fragments are fetched DIST steps ahead.
+//
+// Bound: per step the chain of 4 + 4 dependent v_mfma_f64_16x16x4 (64 cycles
+// each) and two LDS trips: 0.7 us a block where barriers between the steps and
+// substitution or an LDS wait before each read took 1.0 to 1.4.  Order 256, 4096
+// right-hand sides: 15 us, 4 of them the loads and the inversion.
+// Error of FP64 solves against 80-bit arithmetic, orders 64..2000: 1.0 to 2.7e-16
+// (substitution and recursion with products: 1.9 to 4.8e-16); FP32: 2.5e-8 up to
+// order 512, 1.4e-7 at 2000 (1.4 to 3.2e-7).
+#pragma once
+#include "devcommon.hpp"
+#include <type_traits>
+
+namespace {
+
+constexpr int TP_WAVES = 8, TP_THREADS = 64 * TP_WAVES;
+
+// LDS of one panel of order up to 128 * SB.
+template <int SB>
+struct PanelLds {
+    // the solved rows; four rows are 32 banks apart modulo the 64, so a fragment
+    // read (rows r, r + 4, ...) is free of conflicts
+    double X[128 * SB][20];
+    double L[8 * SB][16][17];  // diagonal blocks, then their inverses
+    double R[8 * SB][16];      // reciprocals of the diagonal
+    int ready[8 * SB];         // X of the block is in place
+    int odd;                   // a result that is not finite
+};
+
+struct PanelArgs {
+    const void *A;    // op(T)(0, 0) in solve order
+    void *B;          // row 0 of the panel's first right-hand side
+    long si, sk;      // op(T)(i, k) = A[i * si + k * sk]
+    long ss, rs;      // B(i, c) = B[i * ss + c * rs]
+    int order, cols;  // cols <= 16 right-hand sides
+    int unit;
+    double alpha;
+};
+
+__device__ __forceinline__ void lds_order()
+{
+    __builtin_amdgcn_s_waitcnt(vm_wait(63) & ~(15 << 8));
+    __atomic_signal_fence(__ATOMIC_SEQ_CST);
+    __builtin_amdgcn_wave_barrier();
+}
+
+// An LDS read that stays in program order with the other ones of its wave
+// (a volatile one would also wait for its result before the next is issued).
+__device__ __forceinline__ double lds_value(const double *p)
+{
+    return __builtin_bit_cast(double, __hip_atomic_load((const unsigned long long *)p, __ATOMIC_RELAXED,
+                                                        __HIP_MEMORY_SCOPE_WORKGROUP));
+}
+
+// The same panel by plain substitution, row by row, from the right-hand sides
+// that are still in memory: for panels whose fast result is not finite.  There
+// a product with an inverse's zeros would carry an infinity or a NaN of one row
+// to the rows above it in the block, which a substitution leaves alone.
+template <typename IO, int SB>
+__device__ __forceinline__ void panel_by_rows(const PanelArgs &p, PanelLds<SB> &s)
+{
+    const IO *A = (const IO *)p.A;
+    const IO *B = (const IO *)p.B;
+    const int c = threadIdx.x & 15, r0 = threadIdx.x >> 4;
+    for (int r = r0; r < p.order; r += TP_THREADS / 16)
+        s.X[r][c] = c < p.cols ? p.alpha * (double)B[r * p.ss + c * p.rs] : 0.0;
+    for (int k = 0; k < p.order; ++k) {
+        __syncthreads();
+        double x = s.X[k][c];
+        if (!p.unit) x /= (double)A[k * (p.si + p.sk)];
+        __syncthreads();  // every reader of row k has it
+        if (r0 == 0) s.X[k][c] = x;
+        for (int r = k + 1 + r0; r < p.order; r += TP_THREADS / 16)
+            s.X[r][c] = fma(-(double)A[r * p.si + k * p.sk], x, s.X[r][c]);
+    }
+    __syncthreads();
+}
+
+// f(0), f(1), ... f(N - 1) with compile-time arguments until one returns false
+template <int S, int N, typename F> __device__ __forceinline__ void panel_steps(F &f)
+{
+    if constexpr (S < N) {
+        if (f(std::integral_constant<int, S>{})) panel_steps<S + 1, N>(f);
+    }
+}
+
+// KC: op(T)(i, k) is contiguous along k (|sk| = 1).
+template <typename IO, int SB, bool KC>
+__device__ __forceinline__ void trsm_panel(const PanelArgs &p, PanelLds<SB> &s)
+{
+    constexpr int NBMAX = 8 * SB;               // blocks
+    constexpr int PER = NBMAX * 256 / TP_THREADS;  // elements per thread: diagonal blocks, panel
+    constexpr int DIST = 2;
+    const IO *__restrict__ A = (const IO *)p.A;
+    IO *B = (IO *)p.B;
+    // (opaque, so that a caller's loop over panels keeps no address of this code
+    // in registers across it: it spilled 240 of them)
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    // (the wave number as a scalar: the branches on it are scalar branches, which
+    // MFMA, blind to the lane mask, needs)
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int q0 = lane >> 4, cl = lane & 15;
+    const int order = p.order, nb = (order + 15) / 16, rows = nb * 16;
+    const bool runs = p.ss == 1 || p.ss == -1;  // a right-hand side is contiguous
+
+    if (tid < NBMAX) s.ready[tid] = 0;
+    if (tid == NBMAX) s.odd = 0;
+    // Diagonal blocks first, the panel after them: loads complete in order, so
+    // the inversion waits for the former alone.
+    IO d[PER], v[PER];
+    auto diag = [&](int e, int &bk, int &i, int &k) {
+        const int idx = tid + TP_THREADS * e;
+        bk = idx >> 8, i = (idx >> 4) & 15, k = idx & 15;
+        const int gi = 16 * bk + i;
+        return bk < nb && gi < order && (p.unit ? k < i : k <= i);
+    };
+#pragma unroll
+    for (int e = 0; e < PER; ++e) {
+        int bk, i, k;
+        const bool in = diag(e, bk, i, k);
+        d[e] = A[in ? (16 * bk + i) * p.si + (16 * bk + k) * p.sk : 0];
+    }
+    auto elem = [&](int e, int &r, int &c) {
+        // contiguous along a right-hand side: 32 of its rows per pass; else 16 of a row
+        r = runs ? (tid & 31) + 32 * e : (tid >> 4) + TP_THREADS / 16 * e;
+        c = runs ? tid >> 5 : tid & 15;
+        return r < rows;
+    };
+#pragma unroll
+    for (int e = 0; e < PER; ++e) {
+        int r, c;
+        const bool in = elem(e, r, c) && r < order && c < p.cols;
+        v[e] = B[in ? r * p.ss + c * p.rs : 0];
+    }
+#pragma unroll
+    for (int e = 0; e < PER; ++e) {
+        int bk, i, k;
+        const bool in = diag(e, bk, i, k);
+        s.L[bk][i][k] = in ? (double)d[e] : i == k ? 1.0 : 0.0;  // identity past the order
+    }
+    lds_barrier();
+    {
+        // column cl of the inverse of block 4 * wave + q0; one division per lane
+        // (16 of them in every lane took 1.5 us)
+        const int bk = 4 * wave + q0;
+        if (bk < nb && bk < NBMAX) {
+            double y[16];
+            s.R[bk][cl] = 1.0 / s.L[bk][cl][cl];
+            lds_order();
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const double rc = s.R[bk][i];
+                double t = i == cl ? 1.0 : 0.0;
+#pragma unroll
+                for (int k = 0; k < i; ++k) t = fma(-s.L[bk][i][k], y[k], t);
+                y[i] = t * rc;
+            }
+            lds_order();  // every lane's reads of the block are done
+#pragma unroll
+            for (int i = 0; i < 16; ++i) s.L[bk][i][cl] = y[i];
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < PER; ++e) {
+        int r, c;
+        if (!elem(e, r, c)) continue;
+        s.X[r][c] = r < order && c < p.cols ? p.alpha * (double)v[e] : 0.0;
+    }
+    // op(T)[J, st] in MFMA A-operand layout for the wave's blocks J = wave + 8 q:
+    // element u of a lane is op(T)(16 J + cl, 16 st + 4 q0 + u) -- the k order
+    // that lets a lane read its four elements as one run where k is contiguous
+    // (KC).  Rows past the order read the last one: they are finite where it is,
+    // and reach nothing but the panel's rows past the order.
+    const IO *row[SB];
+#pragma unroll
+    for (int q = 0; q < SB; ++q)
+        row[q] = A + min(16 * (wave + TP_WAVES * q) + cl, order - 1) * p.si +
+                 (KC && p.sk < 0 ? -(4 * q0 + 3) : 4 * q0 * p.sk);
+    IO ring[DIST + 1][SB][4];
+    auto fetch = [&](int st, IO (&f)[SB][4]) {
+        const long k = 16l * min(st, nb - 2) * p.sk;
+#pragma unroll
+        for (int q = 0; q < SB; ++q)
+            if (TP_WAVES * q + TP_WAVES - 1 > st) {
+                if constexpr (KC) {
+                    typedef IO Run __attribute__((ext_vector_type(4), aligned(sizeof(IO))));
+                    const Run r = *(const Run *)(row[q] + k);
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) f[q][u] = r[u];
+                } else {
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) f[q][u] = row[q][k + u * p.sk];
+                }
+            }
+    };
+    // a run of stride -1 was read from its far end: element u is then k = 3 - u
+    const int flip = KC && p.sk < 0 ? 3 : 0;
+    if (nb > 1)
+#pragma unroll
+        for (int st = 0; st < DIST; ++st) fetch(st, ring[st]);
+    __syncthreads();  // inverses and panel are in LDS
+
+    // sums of op(T)[J, I] X_I, subtracted from B_J at the end: a running
+    // difference would be rounded at B_J's size in every step
+    v4d acc[SB];
+#pragma unroll
+    for (int q = 0; q < SB; ++q) acc[q] = v4d{0.0, 0.0, 0.0, 0.0};
+    double inv[4], rhs[4];  // the inverse and B_J of the wave's next block to solve
+    auto upcoming = [&](int q) {
+        const int J = wave + TP_WAVES * q;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            inv[u] = s.L[J][cl][4 * u + q0];
+            rhs[u] = s.X[16 * J + q0 + 4 * u][cl];
+        }
+    };
+    upcoming(0);
+    bool finite = true;
+    // X_J = inv(T_JJ) B_J, published
+    auto solve = [&](int q) {
+        const int J = wave + TP_WAVES * q;
+        v4d x = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            x = __builtin_amdgcn_mfma_f64_16x16x4f64(inv[u], rhs[u] - acc[q][u], x, 0, 0, 0);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) s.X[16 * J + q0 + 4 * u][cl] = x[u];
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+        if (lane == 0) __hip_atomic_store(&s.ready[J], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+        __atomic_signal_fence(__ATOMIC_SEQ_CST);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) finite = finite && __builtin_isfinite(x[u]);
+        if (q + 1 < SB) upcoming(q + 1);
+    };
+    if (wave == 0) solve(0);
+    const int last = min(nb, NBMAX) - 1;  // the wave's last block is at most this one
+    const int mine = last - ((last - wave) & (TP_WAVES - 1));  // its last block (< 0: none)
+    // one block's sum takes on op(T)[J, st] X_st
+    auto update = [&](int q, const IO (&f)[4], const double (&x)[4]) {
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            acc[q] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)f[u], x[u], acc[q], 0, 0, 0);
+    };
+    // step st, a compile-time constant: the fragment ring and the accumulators
+    // stay in registers.  False once nothing of this wave waits for X_st.
+    auto step = [&](auto stc) {
+        constexpr int st = decltype(stc)::value, W = TP_WAVES;
+        if (st >= mine) return false;
+        if constexpr (st + DIST < NBMAX - 1) fetch(st + DIST, ring[(st + DIST) % (DIST + 1)]);
+        IO(&f)[SB][4] = ring[st % (DIST + 1)];
+        constexpr int qn = (st + 1) / W;  // block st + 1 at its owner
+        double x[4];
+        auto flag = [&] {
+            return __builtin_amdgcn_readfirstlane(
+                __hip_atomic_load(&s.ready[st], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+        };
+        auto read_x = [&] {
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                x[u] = lds_value(&s.X[16 * st + 4 * q0 + (u ^ flip)][cl]);
+        };
+        if (wave == (st + 1) % W) {
+            // ahead of the other wave of this SIMD until X is out: its trailing
+            // updates would take every second slot of the matrix core
+            __builtin_amdgcn_s_setprio(3);
+            int ok;
+            do {
+                ok = __hip_atomic_load(&s.ready[st], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                read_x();
+            } while (!__builtin_amdgcn_readfirstlane(ok));
+            update(qn, f[qn], x);
+            solve(qn);
+            __builtin_amdgcn_s_setprio(0);
+        } else {
+            while (!flag()) __builtin_amdgcn_s_sleep(1);
+            read_x();
+            if (wave + W * qn > st + 1) update(qn, f[qn], x);
+        }
+#pragma unroll
+        for (int q = qn + 1; q < SB; ++q) update(q, f[q], x);
+        return true;
+    };
+    panel_steps<0, NBMAX - 1>(step);
+    if (__any(!finite) && lane == 0) s.odd = 1;
+    __syncthreads();  // all of X, and whether it is finite
+    if (s.odd) panel_by_rows<IO, SB>(p, s);
+#pragma unroll
+    for (int e = 0; e < PER; ++e) {
+        int r, c;
+        if (elem(e, r, c) && r < order && c < p.cols) B[r * p.ss + c * p.rs] = (IO)s.X[r][c];
+    }
+}
+
+// Panel arguments of op(T) X = alpha B: T lower (`lower`) in plain or transposed
+// storage (transN: op(T)(i, k) = A[i + k * lda]), rows of B `ss` apart.
+template <typename IO>
+__device__ __forceinline__ PanelArgs panel_args(const IO *A, long lda, int transN, int lower,
+                                                int unit, IO *B, long ss, long rs, int order,
+                                                int cols, double alpha)
+{
+    PanelArgs p;
+    p.si = transN ? 1 : lda;
+    p.sk = transN ? lda : 1;
+    p.ss = ss;
+    p.rs = rs;
+    p.A = A;
+    p.B = B;
+    if (!lower) {  // upper: solved from the last row up
+        p.A = A + (long)(order - 1) * (1 + lda);
+        p.B = B + (order - 1) * ss;
+        p.si = -p.si;
+        p.sk = -p.sk;
+        p.ss = -ss;
+    }
+    p.order = order;
+    p.cols = cols;
+    p.unit = unit;
+    p.alpha = alpha;
+    return p;
+}
+
+}  // namespace
