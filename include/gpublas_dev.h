@@ -341,7 +341,8 @@ void gpublas_dev_batch_destroy(gpublas_batch *b);
 void gpublas_dev_batch_clear(gpublas_batch *b);
 int gpublas_dev_batch_count(const gpublas_batch *b);
 void *gpublas_dev_batch_stream(gpublas_batch *b);
-/* -1 = tile shape from the tuned table (default); 0/1/2 = 32/64/128 square tiles */
+/* -1 = tile shape from the tuned table (default); 0/1/2 = 32/64/128-row tiles
+ * (square; 128 x 64 in FP64) */
 void gpublas_dev_batch_force_cfg(gpublas_batch *b, int cfg);
 int gpublas_dev_batch_dgemm(gpublas_batch *b, char transa, char transb, int m, int n, int k,
                             double alpha, const double *d_A, int lda, const double *d_B, int ldb,

@@ -35,16 +35,15 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemmArgs<T> g)
     gemm_tile<T, BM, BN, BK>(g, tm, tn, As, Bs);
 }
 
-// Fast kernel: every tile of a product with m >= BM and n >= BN, access
-// patterns compile-time constants (PA / PB), operands of any alignment
-// (gemm_fast_tile).  Registers for two workgroups per CU, so one workgroup's
-// barrier and epilogue overlap the other's MFMAs.
-template <typename T, int BM, int BN, int BK, int PA, int PB, int TRI>
+// Fast kernel: every tile of a product at least a tile wide in both dimensions,
+// access patterns compile-time constants (PA / PB), operands of any alignment
+// (gemm_fast_tile, tile shape S).
+template <typename T, int S, int PA, int PB, int TRI>
 __global__ __launch_bounds__(256, 2) void gemm_fast_kernel(GemmArgs<T> g)
 {
-    constexpr int PAD = 128 / (int)sizeof(T);
-    __shared__ __attribute__((aligned(16))) T As[2][BK][BM + PAD];
-    __shared__ __attribute__((aligned(16))) T Bs[2][BK][BN + PAD];
+    typedef FastShape<T, S> F;
+    __shared__ __attribute__((aligned(16))) T As[2][F::BK][F::LDA];
+    __shared__ __attribute__((aligned(16))) T Bs[2][F::BK][F::LDB];
 
     int tm, tn;
     if (TRI == SYM_NONE) {
@@ -55,50 +54,21 @@ __global__ __launch_bounds__(256, 2) void gemm_fast_kernel(GemmArgs<T> g)
         tri_decode(blockIdx.x, hi, lo);
         if (TRI == SYM_LOWER) { tm = hi; tn = lo; } else { tm = lo; tn = hi; }
     }
-    gemm_fast_tile<T, BM, BN, BK, PA, PB, TRI>(g, tm, tn, As, Bs);
-}
-
-// The last, partly filled round of a 128 x 128 fast grid, run as 64 x 64
-// quarter tiles: block b is quarter b % 4 of big tile base + b / 4 (same
-// decoding as gemm_fast_kernel), so the round is four times shorter.
-// Quarters wholly outside the stored triangle have nothing to do.  Same k
-// order per element as the big tile: the bits do not change.
-template <typename T, int PA, int PB, int TRI>
-__global__ __launch_bounds__(256, 2) void gemm_fast_sub_kernel(GemmArgs<T> g, int base)
-{
-    constexpr int PAD = 128 / (int)sizeof(T);
-    __shared__ __attribute__((aligned(16))) T As[2][16][64 + PAD];
-    __shared__ __attribute__((aligned(16))) T Bs[2][16][64 + PAD];
-    const int big = base + (int)(blockIdx.x >> 2), q = blockIdx.x & 3;
-    int tm, tn;
-    if (TRI == SYM_NONE) {
-        tm = big % g.tiles_m;
-        tn = big / g.tiles_m;
-    } else {
-        int hi, lo;
-        tri_decode(big, hi, lo);
-        if (TRI == SYM_LOWER) { tm = hi; tn = lo; } else { tm = lo; tn = hi; }
-    }
-    tm = 2 * tm + (q & 1);
-    tn = 2 * tn + (q >> 1);
-    if (TRI == SYM_LOWER && tn > tm) return;
-    if (TRI == SYM_UPPER && tm > tn) return;
-    if (tm * 64 >= g.m || tn * 64 >= g.n) return;  // past a ragged edge
-    gemm_fast_tile<T, 64, 64, 16, PA, PB, TRI>(g, tm, tn, As, Bs);
+    gemm_fast_tile<T, F::BM, F::BN, F::BK, F::NST, PA, PB, TRI>(g, tm, tn, As, Bs);
 }
 
 // Split-K for problems with too few tiles to fill the chip and a long k:
-// block b is BM x BM tile b % tiles over k chunk b / tiles (kchunk deep, a
+// block b is 32 x 32 tile b % tiles over k chunk b / tiles (kchunk deep, a
 // multiple of 16; the last one what is left), written unscaled to P[chunk] (m x
 // n, leading dimension m); splitk_fold_kernel then forms alpha * (sum of chunks
-// in chunk order) + beta * C.  The decomposition depends only on the shape, so the bits
-// repeat from call to call.
-template <typename T, int BM, int PA, int PB>
+// in chunk order) + beta * C.  The decomposition depends only on the shape, so
+// the bits repeat from call to call.
+template <typename T, int PA, int PB>
 __global__ __launch_bounds__(256, 2) void gemm_fast_splitk_kernel(GemmArgs<T> g, int kchunk, T *P)
 {
-    constexpr int PAD = 128 / (int)sizeof(T);
-    __shared__ __attribute__((aligned(16))) T As[2][16][BM + PAD];
-    __shared__ __attribute__((aligned(16))) T Bs[2][16][BM + PAD];
+    typedef FastShape<T, 32> F;
+    __shared__ __attribute__((aligned(16))) T As[2][F::BK][F::LDA];
+    __shared__ __attribute__((aligned(16))) T Bs[2][F::BK][F::LDB];
     const int tiles = g.tiles_m * g.tiles_n;
     const int t = (int)(blockIdx.x % (unsigned)tiles), kc = (int)(blockIdx.x / (unsigned)tiles);
     const long koff = (long)kc * kchunk;
@@ -111,7 +81,8 @@ __global__ __launch_bounds__(256, 2) void gemm_fast_splitk_kernel(GemmArgs<T> g,
     h.beta = T(0);
     h.C = P + (long)kc * g.m * g.n;
     h.ldc = g.m;
-    gemm_fast_tile<T, BM, BM, 16, PA, PB, SYM_NONE>(h, t % g.tiles_m, t / g.tiles_m, As, Bs);
+    gemm_fast_tile<T, F::BM, F::BN, F::BK, F::NST, PA, PB, SYM_NONE>(h, t % g.tiles_m, t / g.tiles_m,
+                                                                     As, Bs);
 }
 
 template <typename T>
@@ -158,66 +129,51 @@ int launch_scale(hipStream_t s, int m, int n, T beta, T *C, long ldc, int tri)
     return (int)hipGetLastError();
 }
 
-template <typename T> const char *kname(int big, int fast);
-template <> const char *kname<double>(int big, int fast)
+template <typename T> const char *kname(int shape);
+template <> const char *kname<double>(int shape)
 {
-    if (fast) return big ? "dgemm_fast_128x128" : "dgemm_fast_64x64";
-    return big ? "dgemm_edge_128x128" : "dgemm_edge_64x64";
+    return shape == 128  ? "dgemm_fast_128x64"
+           : shape == 64 ? "dgemm_fast_64x64"
+           : shape == 32 ? "dgemm_fast_32x32"
+                         : "dgemm_edge_64x64";
 }
-template <> const char *kname<float>(int big, int fast)
+template <> const char *kname<float>(int shape)
 {
-    if (fast) return big ? "sgemm_fast_128x128" : "sgemm_fast_64x64";
-    return big ? "sgemm_edge_128x128" : "sgemm_edge_64x64";
+    return shape == 128  ? "sgemm_fast_128x128"
+           : shape == 64 ? "sgemm_fast_64x64"
+           : shape == 32 ? "sgemm_fast_32x32"
+                         : "sgemm_edge_64x64";
 }
 
-template <typename T, int BM>
+template <typename T, int S>
 void launch_fast(hipStream_t s, const GemmArgs<T> &g, unsigned blocks)
 {
 #define GB_FAST(PA_, PB_, TRI_)                                                                  \
-    hipLaunchKernelGGL((gemm_fast_kernel<T, BM, BM, 16, PA_, PB_, TRI_>), dim3(blocks),         \
-                       dim3(256), 0, s, g)
+    hipLaunchKernelGGL((gemm_fast_kernel<T, S, PA_, PB_, TRI_>), dim3(blocks), dim3(256), 0, s, g)
     const int pa = g.a.form, pb = g.b.form;
     if (g.tri == SYM_NONE) {
         if (pa == PAT_OUTER && pb == PAT_KCONT) GB_FAST(PAT_OUTER, PAT_KCONT, SYM_NONE);      // NN
         else if (pa == PAT_OUTER) GB_FAST(PAT_OUTER, PAT_OUTER, SYM_NONE);                    // NT
         else if (pb == PAT_KCONT) GB_FAST(PAT_KCONT, PAT_KCONT, SYM_NONE);                    // TN
         else GB_FAST(PAT_KCONT, PAT_OUTER, SYM_NONE);                                         // TT
-    } else if (g.tri == SYM_LOWER) {
-        if (pa == PAT_OUTER) GB_FAST(PAT_OUTER, PAT_OUTER, SYM_LOWER);  // A*A^T
-        else GB_FAST(PAT_KCONT, PAT_KCONT, SYM_LOWER);                  // A^T*A
-    } else {
-        if (pa == PAT_OUTER) GB_FAST(PAT_OUTER, PAT_OUTER, SYM_UPPER);
-        else GB_FAST(PAT_KCONT, PAT_KCONT, SYM_UPPER);
+        return;
+    }
+    if constexpr (FastShape<T, S>::BM == FastShape<T, S>::BN) {  // triangular grids: square tiles
+        if (g.tri == SYM_LOWER) {
+            if (pa == PAT_OUTER) GB_FAST(PAT_OUTER, PAT_OUTER, SYM_LOWER);  // A*A^T
+            else GB_FAST(PAT_KCONT, PAT_KCONT, SYM_LOWER);                  // A^T*A
+        } else {
+            if (pa == PAT_OUTER) GB_FAST(PAT_OUTER, PAT_OUTER, SYM_UPPER);
+            else GB_FAST(PAT_KCONT, PAT_KCONT, SYM_UPPER);
+        }
     }
 #undef GB_FAST
 }
 
-template <typename T>
-void launch_fast_sub(hipStream_t s, const GemmArgs<T> &g, int base, unsigned blocks)
+// Compute units of the current device.
+long device_cus()
 {
-#define GB_SUB(PA_, PB_, TRI_)                                                                   \
-    hipLaunchKernelGGL((gemm_fast_sub_kernel<T, PA_, PB_, TRI_>), dim3(blocks), dim3(256), 0, s, \
-                       g, base)
-    const int pa = g.a.form, pb = g.b.form;
-    if (g.tri == SYM_NONE) {
-        if (pa == PAT_OUTER && pb == PAT_KCONT) GB_SUB(PAT_OUTER, PAT_KCONT, SYM_NONE);
-        else if (pa == PAT_OUTER) GB_SUB(PAT_OUTER, PAT_OUTER, SYM_NONE);
-        else if (pb == PAT_KCONT) GB_SUB(PAT_KCONT, PAT_KCONT, SYM_NONE);
-        else GB_SUB(PAT_KCONT, PAT_OUTER, SYM_NONE);
-    } else if (g.tri == SYM_LOWER) {
-        if (pa == PAT_OUTER) GB_SUB(PAT_OUTER, PAT_OUTER, SYM_LOWER);
-        else GB_SUB(PAT_KCONT, PAT_KCONT, SYM_LOWER);
-    } else {
-        if (pa == PAT_OUTER) GB_SUB(PAT_OUTER, PAT_OUTER, SYM_UPPER);
-        else GB_SUB(PAT_KCONT, PAT_KCONT, SYM_UPPER);
-    }
-#undef GB_SUB
-}
-
-// Concurrent workgroup slots of the fast kernels: two per CU.
-long fast_slots()
-{
-    static const long slots = [] {
+    static const long n = [] {
         int dev = 0, cus = 0;
         if (hipGetDevice(&dev) != hipSuccess ||
             hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess ||
@@ -225,32 +181,32 @@ long fast_slots()
             (void)hipGetLastError();
             cus = 256;
         }
-        return 2L * cus;
+        return (long)cus;
     }();
-    return slots;
+    return n;
 }
 
-// Split-K launch of a rectangular product whose BM x BM tiles number at most
-// half the workgroup slots; k is cut into as many chunks as fill the slots (at
-// most 8, each at least 256 deep, a multiple of 16).  Returns -1 when the shape
-// does not qualify, so the caller takes the ordinary grid.
-template <typename T, int BM>
+// Split-K launch of a rectangular product whose 32 x 32 tiles leave half of the
+// CUs idle: k is cut into as many chunks as fill them (at most 16, each at least
+// 256 deep, a multiple of 16; the fold costs about 5 us, 256 of k about 3).  More
+// than one workgroup a CU gains too little to pay the fold.  Returns -1 when the
+// shape does not qualify, so the caller takes the ordinary grid.
+template <typename T>
 int launch_splitk(hipStream_t s, const GemmArgs<T> &g, int m, int n, int k)
 {
-    const long tiles = (long)ceil_div(m, BM) * ceil_div(n, BM), slots = fast_slots();
-    if (2 * tiles > slots) return -1;
-    const int want = (int)std::min<long>(std::min<long>(slots / tiles, 8), k / 256);
+    const long tiles = (long)ceil_div(m, 32) * ceil_div(n, 32);
+    const int want = (int)std::min<long>(std::min<long>(device_cus() / tiles, 16), k / 256);
     if (want < 2) return -1;
     const int kchunk = ceil_div(ceil_div(k, want), 16) * 16, ks = ceil_div(k, kchunk);
     if (ks < 2) return -1;
     T *P = (T *)gpublas_dev_alloc((size_t)ks * m * n * sizeof(T));
     if (!P) return -1;
     GemmArgs<T> f = g;
-    f.tiles_m = ceil_div(m, BM);
-    f.tiles_n = ceil_div(n, BM);
+    f.tiles_m = ceil_div(m, 32);
+    f.tiles_n = ceil_div(n, 32);
     const unsigned blocks = (unsigned)(tiles * ks);
 #define GB_SK(PA_, PB_)                                                                          \
-    hipLaunchKernelGGL((gemm_fast_splitk_kernel<T, BM, PA_, PB_>), dim3(blocks), dim3(256), 0, s, \
+    hipLaunchKernelGGL((gemm_fast_splitk_kernel<T, PA_, PB_>), dim3(blocks), dim3(256), 0, s, \
                        f, kchunk, P)
     const int pa = g.a.form, pb = g.b.form;
     PROF_BEGIN(s, sizeof(T) == 8 ? "dgemm_splitk" : "sgemm_splitk");
@@ -268,10 +224,56 @@ int launch_splitk(hipStream_t s, const GemmArgs<T> &g, int m, int n, int k)
     return (int)hipGetLastError();
 }
 
+// Tile shape of a product on the fast kernel, by the time the busiest CU takes:
+// its number of tiles times a tile's area over the rate that the shape reaches
+// with the chip full (TFLOP/s at 4096^3: FP64 57 / 68 / 69.5 for 32 x 32, 64 x 64
+// and 128 x 64; FP32 88 / 130 / 138 for 32 x 32, 64 x 64 and 128 x 128).  A 32 x 32
+// tile is bound by L2: where a column's 32 rows (`skewed`: an operand read along
+// its columns whose leading dimension is no multiple of 128 bytes) lie across one
+// more cache line, it reaches three quarters of that (3001 x 768 x 768 NN FP64: 95
+// us against 77 with 64 x 64, but 73 where the leading dimensions are even).  The
+// large shape also needs several tiles a CU (FP64 eight, FP32 two), below which
+// the 64 x 64 one measured the same.  Both sides, 32 against 64: FP64 512^3 8.2 and
+// 20.8 us, 768^3 24.5 and 30.3, 1024^3 41.2 and 39.2, 1536^2 x 1024 84 and 98, 2047 x
+// 1531 x 1789 209 and 173; FP32 512^3 6.0 and 11.9, 768^3 16.9 and 16.7, 1024^3 28.9
+// and 21.9.  64 against 128: FP64 8192^2 x 2048 4.08 and 3.97 ms, FP32 2900^2 x 1500
+// 229 and 287 us, 4096^3 1007 and 996.  0: narrower than every tile.
+template <typename T>
+int fast_shape(long m, long n, int tri, bool skewed)
+{
+    const bool dp = sizeof(T) == 8;
+    const long cus = device_cus();
+    auto count = [&](long bm, long bn) {
+        const long tm = (m + bm - 1) / bm, tn = (n + bn - 1) / bn;
+        return tri ? tm * (tm + 1) / 2 : tm * tn;
+    };
+    auto cost = [&](long bm, long bn, double rate) {
+        return (double)((count(bm, bn) + cus - 1) / cus * bm * bn) / rate;
+    };
+    const long bn = dp ? 64 : 128;
+    if (m < 32 || n < 32) return 0;
+    int best = 32;
+    double least = cost(32, 32, (dp ? 57 : 88) * (skewed ? 0.75 : 1));
+    if (m >= 64 && n >= 64) {
+        const double c = cost(64, 64, dp ? 68 : 130);
+        if (c <= least) best = 64, least = c;
+    }
+    if (m >= 128 && n >= bn && !(dp && tri) && count(128, bn) >= (dp ? 8 : 2) * cus &&
+        cost(128, bn, dp ? 69.5 : 138) <= least)
+        best = 128;
+    return best;
+}
+
+// An operand read along its columns whose columns start at any byte of a cache line.
+template <typename T> bool skewed(const Operand<T> &o)
+{
+    return o.form == PAT_OUTER && (o.ld * sizeof(T)) % 128 != 0;
+}
+
 // Core launcher: C = alpha*op(A)*op(B) + beta*C on an (optionally
-// triangular) tile grid.  k > 0, alpha != 0 assumed.  Products at least a tile
-// wide in both dimensions go to the fast kernel; the generic kernel takes the
-// narrow ones, symmetric operands and leading dimensions past FAST_LD_MAX.
+// triangular) tile grid.  k > 0, alpha != 0 assumed.  Products at least 32 wide
+// in both dimensions go to the fast kernel; the generic kernel takes the narrow
+// ones, symmetric operands and leading dimensions past FAST_LD_MAX.
 template <typename T>
 int launch_gemm(hipStream_t s, int m, int n, int k, T alpha, const Operand<T> &a,
                 const Operand<T> &b, T beta, T *C, long ldc, int tri)
@@ -282,40 +284,24 @@ int launch_gemm(hipStream_t s, int m, int n, int k, T alpha, const Operand<T> &a
     g.a = a; g.b = b;
     g.C = C; g.ldc = ldc;
     g.tri = tri;
-    // Tile choice: 128x128 when that alone gives at least one tile per CU,
-    // else 64x64 so that mid-size problems still fill the 256 CUs.
-    const long t128 = (long)ceil_div(m, 128) * ceil_div(n, 128);
-    const bool big = t128 >= 256 && m >= 128 && n >= 128;
-    const int bm = big ? 128 : 64;
-    const bool fast = a.sym == SYM_NONE && b.sym == SYM_NONE && m >= bm && n >= bm &&
-                      a.ld <= FAST_LD_MAX && b.ld <= FAST_LD_MAX;
-    if (fast && !big && tri == SYM_NONE) {
-        // few 64 x 64 tiles, long k: split k to fill the workgroup slots
-        // (measured: 1024^3 32.8 -> 35.1 TFLOP/s, 512 x 512 x 4096 -> 37.4;
-        // splitting 128 x 128 tiles instead lost to the larger fold)
-        const int err = launch_splitk<T, 64>(s, g, m, n, k);
+    const bool plain = a.sym == SYM_NONE && b.sym == SYM_NONE && a.ld <= FAST_LD_MAX &&
+                       b.ld <= FAST_LD_MAX;
+    const int shape = plain ? fast_shape<T>(m, n, tri, skewed(a) || skewed(b)) : 0;
+    if (shape && tri == SYM_NONE) {
+        const int err = launch_splitk<T>(s, g, m, n, k);
         if (err >= 0) return err;
     }
+    const int bm = shape ? shape : 64, bn = shape == 128 && sizeof(T) == 8 ? 64 : bm;
     g.tiles_m = ceil_div(m, bm);
-    g.tiles_n = ceil_div(n, bm);
+    g.tiles_n = ceil_div(n, bn);
     const long blocks = tri ? (long)g.tiles_m * (g.tiles_m + 1) / 2 : (long)g.tiles_m * g.tiles_n;
-    PROF_BEGIN(s, kname<T>(big, fast));
-    if (fast) {
-        // A last round of 128 x 128 tiles that would leave most of the chip
-        // idle runs as 64 x 64 quarters instead (a quarter of the time).
-        const long slots = fast_slots(), tail = blocks % slots;
-        const long main_blocks = (big && blocks > slots && 2 * tail < slots) ? blocks - tail : blocks;
-        if (big) launch_fast<T, 128>(s, g, (unsigned)main_blocks);
-        else launch_fast<T, 64>(s, g, (unsigned)blocks);
-        if (main_blocks < blocks)
-            launch_fast_sub<T>(s, g, (int)main_blocks, (unsigned)(4 * (blocks - main_blocks)));
-    } else if (big) {
-        hipLaunchKernelGGL((gemm_mfma_kernel<T, 128, 128, 16>), dim3((unsigned)blocks), dim3(256), 0,
-                           s, g);
-    } else {
+    PROF_BEGIN(s, kname<T>(shape));
+    if (shape == 128) launch_fast<T, 128>(s, g, (unsigned)blocks);
+    else if (shape == 64) launch_fast<T, 64>(s, g, (unsigned)blocks);
+    else if (shape == 32) launch_fast<T, 32>(s, g, (unsigned)blocks);
+    else
         hipLaunchKernelGGL((gemm_mfma_kernel<T, 64, 64, 16>), dim3((unsigned)blocks), dim3(256), 0, s,
                            g);
-    }
     PROF_END(s);
     return (int)hipGetLastError();
 }
@@ -409,12 +395,14 @@ __global__ __launch_bounds__(256) void symmetrize_kernel(int n, const T *__restr
 // pointers are shifted to the range start as in the split-K kernel; tiles
 // are dispatched longest range first.  (A ragged last tile is moved back, but
 // stores only its own rows and columns, for which the range is right.)
-template <typename T, int BM, int PA, int PB, int KR>
+template <typename T, int S, int PA, int PB, int KR>
 __global__ __launch_bounds__(256, 2) void gemm_fast_krange_kernel(GemmArgs<T> g)
 {
-    constexpr int PAD = 128 / (int)sizeof(T);
-    __shared__ __attribute__((aligned(16))) T As[2][16][BM + PAD];
-    __shared__ __attribute__((aligned(16))) T Bs[2][16][BM + PAD];
+    typedef FastShape<T, S> F;
+    constexpr int BM = F::BM;
+    static_assert(BM == F::BN, "square tiles");
+    __shared__ __attribute__((aligned(16))) T As[2][F::BK][F::LDA];
+    __shared__ __attribute__((aligned(16))) T Bs[2][F::BK][F::LDB];
     // longest ranges first, so the last round holds the shortest tiles
     const int b = (int)blockIdx.x;
     int tm, tn;
@@ -436,7 +424,7 @@ __global__ __launch_bounds__(256, 2) void gemm_fast_krange_kernel(GemmArgs<T> g)
     h.a.p += PA == PAT_OUTER ? (long)kb * g.a.ld : kb;
     h.b.p += PB == PAT_OUTER ? (long)kb * g.b.ld : kb;
     h.k = ke - kb;
-    gemm_fast_tile<T, BM, BM, 16, PA, PB, SYM_NONE>(h, tm, tn, As, Bs);
+    gemm_fast_tile<T, BM, BM, F::BK, F::NST, PA, PB, SYM_NONE>(h, tm, tn, As, Bs);
 }
 
 // Full n x n matrix of a triangle of A: the stored triangle copied, zeros
@@ -610,10 +598,12 @@ int trmm_entry(void *stream, char side, char uplo, char transa, char diag, int m
                                   : make_op<T>(Tm, ldt, n, tn ? PAT_KCONT : PAT_OUTER, SYM_NONE);
         const int k = left ? m : n;
         const int kr = left ? (oplower ? 1 : 2) : (oplower ? 3 : 4);
-        const long t128 = (long)ceil_div(m, 128) * ceil_div(n, 128);
-        err = t128 >= 256 && m >= 128 && n >= 128
-                          ? launch_krange<T, 128>(s, m, n, k, alpha, a, b, W, ldw, kr)
-                          : launch_krange<T, 64>(s, m, n, k, alpha, a, b, W, ldw, kr);
+        if constexpr (sizeof(T) == 8)
+            err = launch_krange<T, 64>(s, m, n, k, alpha, a, b, W, ldw, kr);
+        else
+            err = fast_shape<T>(m, n, SYM_NONE, false) == 128
+                      ? launch_krange<T, 128>(s, m, n, k, alpha, a, b, W, ldw, kr)
+                      : launch_krange<T, 64>(s, m, n, k, alpha, a, b, W, ldw, kr);
         if (err < 0) err = launch_gemm<T>(s, m, n, k, alpha, a, b, T(0), W, ldw, SYM_NONE);
     }
     if (!err)

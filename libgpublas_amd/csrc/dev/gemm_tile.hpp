@@ -60,15 +60,16 @@ __device__ __forceinline__ bool stored(int sym, long r, long c)
 
 // Pattern for the tile o in [o0, o0+R), k in [k0, k0+BK).
 // LDS tile layout: element (k, o) of a staged tile lives at column
-// o ^ lds_swz<T>(k).  Rows are BM + 128 bytes apart (0 modulo the 64 banks
+// o ^ lds_swz<T, R>(k).  Rows are BM + 128 bytes apart (0 modulo the 64 banks
 // for every other row), so the transposed stores of a k-contiguous operand
 // would put the 8 (double) or 4 (float) k rows one wave writes for a
 // column on the same banks; the XOR moves each row pair (quad) to its own
 // bank group.  It keeps 16-byte vectors and 32-column blocks intact, so
 // vector stores and the MFMA fragment reads stay conflict-free.
-template <typename T> __device__ __forceinline__ int lds_swz(int k)
+// (R: columns of the tile, within which the XOR has to stay.)
+template <typename T, int R> __device__ __forceinline__ int lds_swz(int k)
 {
-    return sizeof(T) == 8 ? 4 * (k >> 1) : 16 * (k >> 2);
+    return (sizeof(T) == 8 ? 4 * (k >> 1) : 16 * (k >> 2)) & (R - 1);
 }
 
 template <typename T, int R, int BK>
@@ -106,9 +107,7 @@ struct TileLoader {
     static constexpr int VEC = 16 / (int)sizeof(T);
     static constexpr int NV = R * BK / VEC / 256;
     static_assert(NV >= 1, "tile too small for 256 threads");
-    static_assert((R & (R - 1)) == 0 &&
-                      (sizeof(T) == 8 ? 4 * ((BK - 1) >> 1) : 16 * ((BK - 1) >> 2)) < R,
-                  "lds_swz must stay inside the tile rows");
+    static_assert((R & (R - 1)) == 0, "lds_swz must stay inside the tile rows");
     typedef T Vec __attribute__((ext_vector_type(VEC)));
 
     __device__ __forceinline__ static void load(const Operand<T> &op, int o0, int k0, int K,
@@ -224,10 +223,10 @@ struct TileLoader {
             if (PAT == PAT_KCONT) {
                 const int kk = (v % (BK / VEC)) * VEC, o = v / (BK / VEC);
 #pragma unroll
-                for (int e = 0; e < VEC; ++e) s[kk + e][o ^ lds_swz<T>(kk + e)] = st[r][e];
+                for (int e = 0; e < VEC; ++e) s[kk + e][o ^ lds_swz<T, R>(kk + e)] = st[r][e];
             } else {
                 const int o = (v % (R / VEC)) * VEC, kk = v / (R / VEC);
-                *(Vec *)&s[kk][o ^ lds_swz<T>(kk)] = st[r];
+                *(Vec *)&s[kk][o ^ lds_swz<T, R>(kk)] = st[r];
             }
         }
     }
@@ -242,10 +241,10 @@ struct TileLoader {
             if (pat == PAT_KCONT) {
                 const int kk = (v % (BK / VEC)) * VEC, o = v / (BK / VEC);
 #pragma unroll
-                for (int e = 0; e < VEC; ++e) s[kk + e][o ^ lds_swz<T>(kk + e)] = st[r][e];
+                for (int e = 0; e < VEC; ++e) s[kk + e][o ^ lds_swz<T, R>(kk + e)] = st[r][e];
             } else {
                 const int o = (v % (R / VEC)) * VEC, kk = v / (R / VEC);
-                *(Vec *)&s[kk][o ^ lds_swz<T>(kk)] = st[r];
+                *(Vec *)&s[kk][o ^ lds_swz<T, R>(kk)] = st[r];
             }
         }
     }
@@ -337,8 +336,9 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs<T> &g, int tm, int tn,
             // l < 16: the high part of the swizzle depends on kk alone (a
             // constant of the unrolled loop), so the fragment offsets stay
             // immediate; the low part is one lane-dependent term per step
-            const int shi = lds_swz<T>(kk) & ~15;
-            const int lo = (lane & 15) ^ (lds_swz<T>(kr) & 15);
+            static_assert(BM == BN, "one swizzle for both operands");
+            const int shi = lds_swz<T, BM>(kk) & ~15;
+            const int lo = (lane & 15) ^ (lds_swz<T, BM>(kr) & 15);
 #pragma unroll
             for (int i = 0; i < FM; ++i)
                 fa[i] = As[cur][kr][((wm * WM + i * 16) ^ shi) + lo];
@@ -394,16 +394,17 @@ struct TileMath {
     {
         const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
         const int wm = wave & 1, wn = wave >> 1, kr = kk + (lane >> 4);
-        // (c0 + l) ^ swz = (c0 ^ shi) + (l ^ slo) for c0 a multiple of 16 and
+        // (c0 + l) ^ swz = (c0 ^ high) + (l ^ low) for c0 a multiple of 16 and
         // l < 16: the high part of the swizzle depends on kk alone (a
         // constant of the unrolled loop), so the fragment offsets stay
         // immediate; the low part is one lane-dependent term per step
-        const int shi = lds_swz<T>(kk) & ~15;
-        const int lo = (lane & 15) ^ (lds_swz<T>(kr) & 15);
+        const int ha = lds_swz<T, BM>(kk) & ~15, hb = lds_swz<T, BN>(kk) & ~15;
+        const int la = (lane & 15) ^ (lds_swz<T, BM>(kr) & 15);
+        const int lb = (lane & 15) ^ (lds_swz<T, BN>(kr) & 15);
 #pragma unroll
-        for (int i = 0; i < FM; ++i) fa[i] = A[kr][((wm * WM + i * 16) ^ shi) + lo];
+        for (int i = 0; i < FM; ++i) fa[i] = A[kr][((wm * WM + i * 16) ^ ha) + la];
 #pragma unroll
-        for (int j = 0; j < FN; ++j) fb[j] = B[kr][((wn * WN + j * 16) ^ shi) + lo];
+        for (int j = 0; j < FN; ++j) fb[j] = B[kr][((wn * WN + j * 16) ^ hb) + lb];
     }
     __device__ __forceinline__ static void multiply(const T (&fa)[FM], const T (&fb)[FN],
                                                     Acc (&acc)[FM][FN])
@@ -478,6 +479,15 @@ struct TileMath {
 // of one operand covers at most 64 rows of its leading dimension).
 constexpr long FAST_LD_MAX = 1l << 23;
 
+// The fast tile's shapes.  NST: k-tiles of one operand on their way in registers.
+// A 32 x 32 FP32 tile takes 32 of k at a time, one 16-byte load per thread.
+template <typename T, int S> struct FastShape {
+    static constexpr int BM = S, BN = S == 128 && sizeof(T) == 8 ? 64 : S;
+    static constexpr int BK = S == 32 && sizeof(T) == 4 ? 32 : 16;
+    static constexpr int NST = (S == 128 && sizeof(T) == 8) || BK == 32 ? 2 : 4;
+    static constexpr int LDA = BM + 128 / (int)sizeof(T), LDB = BN + 128 / (int)sizeof(T);
+};
+
 // C tile (tm, tn) of g with access patterns PA / PB fixed at compile time, for
 // m >= BM and n >= BN.  The last tile of a ragged dimension is moved back to
 // end at the matrix's edge: it recomputes a few rows (columns) of its
@@ -486,17 +496,19 @@ constexpr long FAST_LD_MAX = 1l << 23;
 // the same bits.
 //
 // Pipeline (bound: the matrix cores; LDS and memory have to stay out of their
-// way): k-tile t+2 travels from memory to registers while t is multiplied,
-// t+1 is stored to the other LDS buffer during the first k step of t, and the
-// fragments of a k step are read during the step before it -- across the one
-// barrier of a k-tile too, which therefore sits in front of a step's products
+// way): k-tiles t+2 ... t+1+NST travel from memory to registers while t is
+// multiplied, t+1 is stored to the other LDS buffer during the first k step of t,
+// and the fragments of a k step are read during the step before it -- across the
+// one barrier of a k-tile too, which therefore sits in front of a step's products
 // and not in front of its reads.  The barrier waits for LDS traffic alone.
-// Measured against reads in front of each step and guarded edge tiles: FP64
-// 8192^3 NT 65.3 -> 68.0 TFLOP/s, FP32 4096^3 NN 121 -> 130, FP64 2047 x 1531 x
-// 1789 TN on odd leading dimensions 44.4 -> 58.7, 100^3 13.5 -> 8.4 us.  (More
-// than 256 registers a lane make the compiler move the accumulators to and
-// from the accumulation registers in every k-tile: 48 TFLOP/s.)
-template <typename T, int BM, int BN, int BK, int PA, int PB, int TRI>
+// Measured, from reads in front of each step and guarded edge tiles over NST = 1 to
+// the NST of FastShape: FP64 8192^3 NT 65.3, 68.0, 69.1 TFLOP/s; 2047 x 1531 x 1789
+// TN on odd leading dimensions 44.4, 58.7, 65.6; FP32 4096^3 NN 121, 130, 137.
+// NST is even: with an odd one the LDS buffer is no constant of the unrolled code
+// (NST 3 was slower than 2).  128 x 128 FP64 tiles have no registers for a second
+// stage; more than 256 registers a lane make the compiler move the accumulators to
+// and from the accumulation registers in every k-tile (48 TFLOP/s).
+template <typename T, int BM, int BN, int BK, int NST, int PA, int PB, int TRI>
 __device__ __forceinline__ void gemm_fast_tile(const GemmArgs<T> &g, int tm, int tn,
                                                T (*As)[BK][BM + 128 / sizeof(T)],
                                                T (*Bs)[BK][BN + 128 / sizeof(T)])
@@ -521,37 +533,39 @@ __device__ __forceinline__ void gemm_fast_tile(const GemmArgs<T> &g, int tm, int
 #pragma unroll
         for (int j = 0; j < M::FN; ++j) acc[i][j] = typename M::Acc{};
 
-    typename LA::Vec sa[LA::NV];
-    typename LB::Vec sb[LB::NV];
-    // the next k-tile into registers; pa / pb are uniform and move on
-    auto load_full = [&]() {
-        LA::template load_pat<PA>(pa, lda, va, sa);
-        LB::template load_pat<PB>(pb, ldb, vb, sb);
+    // k-tile t passes through register stage t % NST; pa / pb are uniform and
+    // move on with the loads
+    typename LA::Vec sa[NST][LA::NV];
+    typename LB::Vec sb[NST][LB::NV];
+    auto load_full = [&](int r) {
+        LA::template load_pat<PA>(pa, lda, va, sa[r]);
+        LB::template load_pat<PB>(pb, ldb, vb, sb[r]);
         pa += stepa;
         pb += stepb;
     };
-    auto load_any = [&](int t) {
+    auto load_any = [&](int t, int r) {
         if (t < kfull) {
-            load_full();
-        } else {
-            LA::template load_ktail<PA>(pa, lda, K - t * BK, sa);
-            LB::template load_ktail<PB>(pb, ldb, K - t * BK, sb);
+            load_full(r);
+        } else if (t < ktiles) {
+            LA::template load_ktail<PA>(pa, lda, K - t * BK, sa[r]);
+            LB::template load_ktail<PB>(pb, ldb, K - t * BK, sb[r]);
         }
     };
-    auto store = [&](int buf) {
-        LA::template store_pat<PA, BM + M::PAD>(As[buf], sa);
-        LB::template store_pat<PB, BN + M::PAD>(Bs[buf], sb);
+    auto store = [&](int buf, int r) {
+        LA::template store_pat<PA, BM + M::PAD>(As[buf], sa[r]);
+        LB::template store_pat<PB, BN + M::PAD>(Bs[buf], sb[r]);
     };
     T fa[2][M::FM], fb[2][M::FN];
 
-    load_any(0);
-    store(0);
-    if (ktiles > 1) load_any(1);
+#pragma unroll
+    for (int t = 0; t < NST; ++t) load_any(t, t);
+    store(0, 0);
+    load_any(NST, 0);
     lds_barrier();
     M::fetch(As[0], Bs[0], 0, fa[0], fb[0]);
+    // k-tile kt out of buffer cur; kt + 1 leaves stage r for the other buffer
     int kt = 0;
-    for (; kt + 2 < kfull; ++kt) {
-        const int cur = kt & 1;
+    auto tile = [&](int cur, int r, bool steady) {
 #pragma unroll
         for (int st = 0; st < STEPS; ++st) {
             if (st + 1 < STEPS) {
@@ -561,32 +575,31 @@ __device__ __forceinline__ void gemm_fast_tile(const GemmArgs<T> &g, int tm, int
                 M::fetch(As[cur ^ 1], Bs[cur ^ 1], 0, fa[0], fb[0]);
             }
             if (st == 0) {
-                store(cur ^ 1);
-                load_full();
+                if (steady) {
+                    store(cur ^ 1, r);
+                    load_full(r);
+                } else if (kt + 1 < ktiles) {
+                    store(cur ^ 1, r);
+                    load_any(kt + 1 + NST, r);
+                }
             }
             __builtin_amdgcn_sched_barrier(0);
             M::multiply(fa[st & 1], fb[st & 1], acc);
             __builtin_amdgcn_sched_barrier(0);
         }
-    }
-    for (; kt < ktiles; ++kt) {  // the last two k-tiles: nothing or the ragged one to load
-        const int cur = kt & 1;
+        ++kt;
+    };
+    // U k-tiles per pass: buffer and stage are constants of the unrolled code
+    constexpr int U = NST < 2 ? 2 : NST;
+    static_assert(U % 2 == 0 && U % NST == 0, "a pass starts at buffer 0 and stage 1");
+    while (kt + U + NST < kfull) {
 #pragma unroll
-        for (int st = 0; st < STEPS; ++st) {
-            if (st + 1 < STEPS) {
-                M::fetch(As[cur], Bs[cur], (st + 1) * 4, fa[(st + 1) & 1], fb[(st + 1) & 1]);
-            } else {
-                lds_barrier();
-                M::fetch(As[cur ^ 1], Bs[cur ^ 1], 0, fa[0], fb[0]);
-            }
-            if (st == 0 && kt + 1 < ktiles) {
-                store(cur ^ 1);
-                if (kt + 2 < ktiles) load_any(kt + 2);
-            }
-            __builtin_amdgcn_sched_barrier(0);
-            M::multiply(fa[st & 1], fb[st & 1], acc);
-            __builtin_amdgcn_sched_barrier(0);
-        }
+        for (int q = 0; q < U; ++q) tile(q & 1, (q + 1) % NST, true);
+    }
+    while (kt < ktiles) {  // what is left: the ragged k-tile or nothing to load
+#pragma unroll
+        for (int q = 0; q < U; ++q)
+            if (kt < ktiles) tile(q & 1, (q + 1) % NST, false);
     }
     M::template finish<TRI, false>(g, m0, n0, tm * BM, tn * BN, acc);
 }

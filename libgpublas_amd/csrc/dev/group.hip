@@ -18,8 +18,8 @@
 //
 // Kernels (all persistent: a fixed grid loops over the batch's work units,
 // so one captured graph serves every batch of the slot):
-//  * group_gemm_arg / _tab<T, BM>: every tile of every GEMM problem that the
-//    tile-shape table assigns to BM x BM, full tiles first, in one grid;
+//  * group_gemm_arg / _tab<T, S>: every tile of every GEMM problem that the
+//    tile-shape table assigns to shape S (FastShape), in one grid;
 //    tile t -> problem by binary search over the prefix sums; the tile
 //    itself is the per-call fast tile routine (gemm_tile.hpp; its guarded
 //    variant for ragged tiles), so a product's bits do not depend on the
@@ -151,11 +151,12 @@ __device__ __forceinline__ GemmArgs<T> chunk_args(const GGemm<T> &e, int s)
 // Tile t of the group's fast problems (EDGE = false: at least a tile wide in
 // both dimensions) or of its narrow ones, numbered over the problems of that
 // class, chunks of a split problem one after the other.
-template <typename T, int BM, bool EDGE>
+template <typename T, int S, bool EDGE>
 __device__ __forceinline__ void group_tile(const GemmGroup<T> &G, int np, int t,
-                                           T (*As)[16][BM + 128 / sizeof(T)],
-                                           T (*Bs)[16][BM + 128 / sizeof(T)])
+                                           T (*As)[FastShape<T, S>::BK][FastShape<T, S>::LDA],
+                                           T (*Bs)[FastShape<T, S>::BK][FastShape<T, S>::LDB])
 {
+    typedef FastShape<T, S> F;
     const int p = find_unit(EDGE ? &G.p[0].edge_begin : &G.p[0].fast_begin, sizeof(GGemm<T>), np, t);
     const int per = G.p[p].g.tiles_m * G.p[p].g.tiles_n;
     const int t0 = t - (EDGE ? G.p[p].edge_begin : G.p[p].fast_begin), tl = t0 % per;
@@ -163,8 +164,10 @@ __device__ __forceinline__ void group_tile(const GemmGroup<T> &G, int np, int t,
     const int tm = tl % g.tiles_m, tn = tl / g.tiles_m;
 #define GB_TILE(PA_, PB_)                                                                        \
     do {                                                                                         \
-        if constexpr (EDGE) gemm_edge_tile<T, BM, BM, 16, PA_, PB_>(g, tm, tn, As, Bs);          \
-        else gemm_fast_tile<T, BM, BM, 16, PA_, PB_, SYM_NONE>(g, tm, tn, As, Bs);               \
+        if constexpr (EDGE)                                                                      \
+            gemm_edge_tile<T, F::BM, F::BN, F::BK, PA_, PB_>(g, tm, tn, As, Bs);                 \
+        else                                                                                     \
+            gemm_fast_tile<T, F::BM, F::BN, F::BK, F::NST, PA_, PB_, SYM_NONE>(g, tm, tn, As, Bs); \
     } while (0)
     switch (G.p[p].pat) {
     case 0: GB_TILE(PAT_OUTER, PAT_KCONT); break;
@@ -177,20 +180,17 @@ __device__ __forceinline__ void group_tile(const GemmGroup<T> &G, int np, int t,
 
 // Every tile of the group, the fast problems' first, in one grid: the narrow
 // problems of a batch do not make a round of their own after them.
-template <typename T, int BM>
+template <typename T, int S>
 __device__ __forceinline__ void gemm_group_body(const GemmGroup<T> &G)
 {
-    constexpr int PAD = 128 / (int)sizeof(T);
-    __shared__ __attribute__((aligned(16))) T As[2][16][BM + PAD];
-    __shared__ __attribute__((aligned(16))) T Bs[2][16][BM + PAD];
+    typedef FastShape<T, S> F;
+    __shared__ __attribute__((aligned(16))) T As[2][F::BK][F::LDA];
+    __shared__ __attribute__((aligned(16))) T Bs[2][F::BK][F::LDB];
     const int np = min(G.np, kCapGemm);
-    const int nf = BM == 32 ? 0 : G.fast_tiles, total = nf + G.edge_tiles;
+    const int nf = G.fast_tiles, total = nf + G.edge_tiles;
     for (int t = blockIdx.x; t < total; t += gridDim.x) {
-        if (t < nf) {
-            if constexpr (BM != 32) group_tile<T, BM, false>(G, np, t, As, Bs);
-        } else {
-            group_tile<T, BM, true>(G, np, t - nf, As, Bs);
-        }
+        if (t < nf) group_tile<T, S, false>(G, np, t, As, Bs);
+        else group_tile<T, S, true>(G, np, t - nf, As, Bs);
     }
 }
 
@@ -519,13 +519,16 @@ int bucket(double v)
     return e - 5;
 }
 
-bool cfg_valid(int ty, int cfg) { return !(ty == TY_S && cfg == CFG_32); }
+// Shapes that a tuned table can name.
+bool cfg_tuned(int ty, int cfg) { return !(ty == TY_S && cfg == CFG_32); }
 
-int heuristic_cfg(int ty, int m, int n)
+// Without a measured table: a small problem's time in a batch is its k chain,
+// which a 32 x 32 tile runs about three times as fast as a 64 x 64 one (0.18
+// against 0.5 us per 16 of k); large ones take the shape with the better rate.
+int heuristic_cfg(int m, int n)
 {
-    if (m >= 384 && n >= 384) return CFG_128;
-    if (ty == TY_D && m <= 48 && n <= 48) return CFG_32;
-    return CFG_64;
+    if (m >= 1024 && n >= 1024) return CFG_128;
+    return (long)ceil_div(m, 64) * ceil_div(n, 64) <= 36 ? CFG_32 : CFG_64;
 }
 
 void tune_init_locked()
@@ -540,14 +543,18 @@ int choose_cfg(int ty, int m, int n, int k)
     std::lock_guard<std::mutex> lk(g_tune_mu);
     tune_init_locked();
     const int c = g_tune[ty][bucket(sqrt((double)m * (double)n))][bucket((double)k)];
-    return c >= 0 && cfg_valid(ty, c) ? c : heuristic_cfg(ty, m, n);
+    const int h = heuristic_cfg(m, n);
+    // FP32 tables name two shapes, as ever: the smaller one covers 32 x 32 too
+    if (ty == TY_S && c == CFG_64 && h == CFG_32) return CFG_32;
+    return c >= 0 ? c : h;
 }
 
 int cfg_bm(int cfg) { return cfg == CFG_32 ? 32 : cfg == CFG_64 ? 64 : 128; }
+int cfg_bn(int ty, int cfg) { return ty == TY_D && cfg == CFG_128 ? 64 : cfg_bm(cfg); }
 
 // grid of each persistent kernel: enough workgroups to fill 256 CUs at the
 // kernel's occupancy (double / single), capped by the work when eager
-constexpr int kGridGemm[2][kCfgs] = {{1024, 512, 512}, {1024, 512, 512}};  // 2 per CU from 64
+constexpr int kGridGemm[2][kCfgs] = {{1024, 512, 512}, {1024, 512, 512}};
 constexpr int kGridGemv = 1024, kGridFold = 512, kGridTrsm = 256;  // TRSM: one per CU (LDS)
 constexpr size_t kWsDoubles = (size_t)8 << 20;  // 64 MiB of GEMV partial sums
 
@@ -596,8 +603,7 @@ int add_gemm(gpublas_batch *b, char ta, char tb, int m, int n, int k, T alpha, c
 {
     constexpr int ty = sizeof(T) == 8 ? TY_D : TY_S;
     if (m <= 0 || n <= 0 || k <= 0 || alpha == T(0)) return -1;
-    const int cfg = b->force_cfg >= 0 && cfg_valid(ty, b->force_cfg) ? b->force_cfg
-                                                                     : choose_cfg(ty, m, n, k);
+    const int cfg = b->force_cfg >= 0 ? b->force_cfg : choose_cfg(ty, m, n, k);
     GemmGroup<T> &G = group_of<T>(b->h_tab, cfg);
     if (G.np >= kCapGemm) return 1;
     GGemm<T> &e = G.p[G.np];
@@ -612,13 +618,12 @@ int add_gemm(gpublas_batch *b, char ta, char tb, int m, int n, int k, T alpha, c
     g.b = make_op<T>(B, ldb, n, is_n(tb) ? PAT_KCONT : PAT_OUTER, SYM_NONE);
     g.C = C;
     g.ldc = ldc;
-    const int bm = cfg_bm(cfg);
+    const int bm = cfg_bm(cfg), bn = cfg_bn(ty, cfg);
     g.tiles_m = ceil_div(m, bm);
-    g.tiles_n = ceil_div(n, bm);
+    g.tiles_n = ceil_div(n, bn);
     g.tri = SYM_NONE;
     // a problem at least a tile wide in both dimensions takes the fast tile
-    // (the 32-wide shape has no fast variant)
-    const bool fast = cfg != CFG_32 && m >= bm && n >= bm && lda <= FAST_LD_MAX && ldb <= FAST_LD_MAX;
+    const bool fast = m >= bm && n >= bn && lda <= FAST_LD_MAX && ldb <= FAST_LD_MAX;
     e.pat = (g.a.form == PAT_OUTER ? 0 : 2) + (g.b.form == PAT_KCONT ? 0 : 1);
     // split along k when the tiles alone cannot spread over the CUs: about
     // 256 units, chunks of at least 256, partials of at most 16 MiB.  Counted
@@ -674,7 +679,7 @@ void launch_gemm_group(gpublas_batch *b, hipStream_t s, int cfg, bool capture)
         hipLaunchKernelGGL((group_gemm_fold_tab<T>), dim3(512), dim3(256), 0, s, dG);
         return;
     }
-    const int tiles = (BM == 32 ? 0 : G.fast_tiles) + G.edge_tiles;
+    const int tiles = G.fast_tiles + G.edge_tiles;
     if (tiles)
         hipLaunchKernelGGL((group_gemm_arg<T, BM>), dim3(tiles < fix ? tiles : fix), dim3(256), 0,
                            s, G);
@@ -714,7 +719,7 @@ void enqueue(gpublas_batch *b, unsigned mask, bool capture)
     if (!capture) {
         double cost[4];
         kind_costs(t, cost);
-        const unsigned kmask[4] = {1u | 2u | 4u, 16u | 32u, 64u, 128u};
+        const unsigned kmask[4] = {1u | 2u | 4u, 8u | 16u | 32u, 64u, 128u};
         int order[4] = {0, 1, 2, 3};
         for (int i = 1; i < 4; ++i)
             for (int j = i; j > 0 && cost[order[j]] < cost[order[j - 1]]; --j) {
@@ -731,6 +736,7 @@ void enqueue(gpublas_batch *b, unsigned mask, bool capture)
                 if (mask & 2u) launch_gemm_group<double, 64>(b, s0, CFG_64, false);
                 if (mask & 4u) launch_gemm_group<double, 128>(b, s0, CFG_128, false);
             } else if (k == 1) {
+                if (mask & 8u) launch_gemm_group<float, 32>(b, s0, CFG_32, false);
                 if (mask & 16u) launch_gemm_group<float, 64>(b, s0, CFG_64, false);
                 if (mask & 32u) launch_gemm_group<float, 128>(b, s0, CFG_128, false);
             } else if (k == 2) {
@@ -757,6 +763,7 @@ void enqueue(gpublas_batch *b, unsigned mask, bool capture)
     if (mask & 1u) launch_gemm_group<double, 32>(b, sg, CFG_32, true);
     if (mask & 2u) launch_gemm_group<double, 64>(b, sg, CFG_64, true);
     if (mask & 4u) launch_gemm_group<double, 128>(b, sg, CFG_128, true);
+    if (mask & 8u) launch_gemm_group<float, 32>(b, sg, CFG_32, true);
     if (mask & 16u) launch_gemm_group<float, 64>(b, sg, CFG_64, true);
     if (mask & 32u) launch_gemm_group<float, 128>(b, sg, CFG_128, true);
     if (mask & 64u) {
@@ -1049,7 +1056,7 @@ int gpublas_dev_tune_gemm(const char *path, int force)
                 float best = 1e30f;
                 int bestc = -1;
                 for (int c = 0; c < kCfgs; ++c) {
-                    if (!cfg_valid(ty, c)) continue;
+                    if (!cfg_tuned(ty, c)) continue;
                     float tot = 0;
                     for (int rep = 0; rep < 4; ++rep) {
                         batch_clear(b);

@@ -44,20 +44,22 @@ def _gemm(gb, single, ta, tb, m, n, k, pad, off, beta):
 @pytest.mark.parametrize("single", [False, True])
 @pytest.mark.parametrize("ta,tb", [("N", "N"), ("N", "T"), ("T", "N"), ("T", "T")])
 @pytest.mark.parametrize("m,n,k", [
+    (32, 32, 1), (33, 47, 16), (40, 34, 33), (31, 64, 40), (45, 70, 1000), (32, 33, 5000),
     (64, 64, 1), (64, 65, 15), (65, 64, 16), (127, 66, 17), (128, 129, 31), (129, 127, 32),
     (191, 193, 33), (64, 200, 47), (63, 65, 48), (200, 63, 49), (65, 66, 1000)])
 def test_gemm_tile_edges(gpu, single, ta, tb, m, n, k):
-    """64 x 64 tiles (and the generic tile below 64), k from one step to a split k."""
+    """32 x 32 and 64 x 64 tiles (the generic tile below 32), k from one step to a split k."""
     _gemm(gpu, single, ta, tb, m, n, k, pad=1, off=1, beta=-1.0)
     _gemm(gpu, single, ta, tb, m, n, k, pad=0, off=0, beta=0.0)
 
 
 @pytest.mark.parametrize("single", [False, True])
 @pytest.mark.parametrize("ta,tb", [("N", "N"), ("N", "T"), ("T", "N"), ("T", "T")])
-@pytest.mark.parametrize("m,n,k", [(2049, 2055, 33), (2944, 2816, 48), (129, 32769, 18)])
+@pytest.mark.parametrize("m,n,k", [(2049, 2055, 33), (2944, 2816, 48), (129, 32769, 18),
+                                   (1030, 1100, 130), (2816, 2910, 161)])
 def test_gemm_large_tile_edges(gpu, single, ta, tb, m, n, k):
-    """128 x 128 tiles, ragged and not, with a last round that runs as quarters
-    (23 x 22 = 506 tiles; 17 x 17; 2 x 257 = 514 = 512 + 2)."""
+    """Products large enough for 64 x 64 tiles at every stage of the k pipeline, and for
+    128 x 64 (FP64) and 128 x 128 (FP32) ones, ragged in both dimensions."""
     _gemm(gpu, single, ta, tb, m, n, k, pad=3, off=1, beta=1.0)
 
 
