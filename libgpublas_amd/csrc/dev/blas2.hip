@@ -28,29 +28,37 @@
 namespace {
 
 typedef double d2 __attribute__((ext_vector_type(2)));
+// Two neighbouring elements at any element address: global memory takes 16-byte
+// accesses that are only 8-byte aligned, so columns of an odd leading dimension
+// stream like aligned ones (5001 x 5001, lda 5003: DGER 228 -> 98 us, DGEMV 'T'
+// 57 -> 42 us, against one or two 8-byte accesses a column in flight).
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
 constexpr int GN_ROWS = 512;  // rows per workgroup panel (256 threads x 2)
 constexpr int GN_U = 8;       // columns in flight per wave
 
 __global__ __launch_bounds__(256) void gemv_n_stream(int m, int n, double alpha, const double *A,
                                                      long lda, const double *x, long incx, long x0,
                                                      double beta, double *y, long incy, long y0,
-                                                     int nrb, int cbw, int direct, int vec,
+                                                     int nrb, int cbw, int direct,
                                                      double *partials)
 {
     const int rb = blockIdx.x % nrb, cb = blockIdx.x / nrb;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const long row = (long)rb * GN_ROWS + wave * 128 + 2 * lane;
+    long row = (long)rb * GN_ROWS + wave * 128 + 2 * lane;
+    if (row >= m) return;
+    const bool odd = row + 1 == m;
+    if (odd) row = m > 1 ? m - 2 : 0;  // the last row of an odd m: the second of a pair
     const int c0 = cb * cbw;
     const int c1 = min(n, c0 + cbw);
     double s0 = 0, s1 = 0;
-    if (vec && row + 1 < m) {
+    if (m > 1) {
         const double *a = A + row;
         int c = c0;
         for (; c + GN_U <= c1; c += GN_U) {
             d2 v[GN_U];
 #pragma unroll
             for (int u = 0; u < GN_U; ++u)
-                v[u] = __builtin_nontemporal_load((const d2 *)(a + (long)(c + u) * lda));
+                v[u] = __builtin_nontemporal_load((const d2u *)(a + (long)(c + u) * lda));
 #pragma unroll
             for (int u = 0; u < GN_U; ++u) {
                 const double xv = x[x0 + (long)(c + u) * incx];
@@ -59,32 +67,27 @@ __global__ __launch_bounds__(256) void gemv_n_stream(int m, int n, double alpha,
             }
         }
         for (; c < c1; ++c) {
-            const d2 v = *(const d2 *)(a + (long)c * lda);
+            const d2 v = *(const d2u *)(a + (long)c * lda);
             const double xv = x[x0 + (long)c * incx];
             s0 = fma(v.x, xv, s0);
             s1 = fma(v.y, xv, s1);
         }
     } else {
-        for (int c = c0; c < c1; ++c) {
-            const double xv = x[x0 + (long)c * incx];
-            if (row < m) s0 = fma(A[row + (long)c * lda], xv, s0);
-            if (row + 1 < m) s1 = fma(A[row + 1 + (long)c * lda], xv, s1);
-        }
+        for (int c = c0; c < c1; ++c) s0 = fma(A[(long)c * lda], x[x0 + (long)c * incx], s0);
     }
+    if (odd && m > 1) ++row, s0 = s1;
     if (direct) {
-        if (row < m) {
-            double *yp = y + y0 + row * incy;
-            *yp = beta == 0.0 ? alpha * s0 : fma(beta, *yp, alpha * s0);
-        }
-        if (row + 1 < m) {
+        double *yp = y + y0 + row * incy;
+        *yp = beta == 0.0 ? alpha * s0 : fma(beta, *yp, alpha * s0);
+        if (!odd) {
             double *yp = y + y0 + (row + 1) * incy;
             *yp = beta == 0.0 ? alpha * s1 : fma(beta, *yp, alpha * s1);
         }
         return;
     }
     double *pp = partials + (long)cb * m;
-    if (row < m) pp[row] = s0;
-    if (row + 1 < m) pp[row + 1] = s1;
+    pp[row] = s0;
+    if (!odd) pp[row + 1] = s1;
 }
 
 __global__ __launch_bounds__(256) void gemv_n_fold(int m, int ncb, const double *partials,
@@ -112,21 +115,20 @@ __global__ __launch_bounds__(256) void gemv_n_fold(int m, int ncb, const double 
 
 __global__ __launch_bounds__(256) void gemv_t_kernel(int m, int n, double alpha, const double *A,
                                                      long lda, const double *x, long incx, long x0,
-                                                     double beta, double *y, long incy, long y0,
-                                                     int vec)
+                                                     double beta, double *y, long incy, long y0)
 {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     for (long j = (long)blockIdx.x * 4 + wave; j < n; j += (long)gridDim.x * 4) {
         const double *a = A + j * lda;
         double s = 0;
-        if (vec && incx == 1 && x0 == 0) {
+        if (incx == 1) {
             int i = 2 * lane;
             for (; i + 128 * 7 + 1 < m; i += 128 * 8) {
                 d2 av[8], xv[8];
 #pragma unroll
                 for (int u = 0; u < 8; ++u) {
-                    av[u] = __builtin_nontemporal_load((const d2 *)(a + i + 128 * u));
-                    xv[u] = *(const d2 *)(x + i + 128 * u);
+                    av[u] = __builtin_nontemporal_load((const d2u *)(a + i + 128 * u));
+                    xv[u] = *(const d2u *)(x + i + 128 * u);
                 }
 #pragma unroll
                 for (int u = 0; u < 8; ++u) {
@@ -135,8 +137,8 @@ __global__ __launch_bounds__(256) void gemv_t_kernel(int m, int n, double alpha,
                 }
             }
             for (; i + 1 < m; i += 128) {
-                const d2 av = *(const d2 *)(a + i);
-                const d2 xv = *(const d2 *)(x + i);
+                const d2 av = *(const d2u *)(a + i);
+                const d2 xv = *(const d2u *)(x + i);
                 s = fma(av.x, xv.x, s);
                 s = fma(av.y, xv.y, s);
             }
@@ -173,55 +175,60 @@ __global__ void scal_vec_kernel(int n, double beta, double *y, long incy, long y
 constexpr int GR_U = 8;
 __global__ __launch_bounds__(256) void ger_stream(int m, int n, double alpha, const double *x,
                                                   long incx, long x0, const double *y, long incy,
-                                                  long y0, double *A, long lda, int nrb, int cbw,
-                                                  int vec)
+                                                  long y0, double *A, long lda, int nrb, int cbw)
 {
     const int rb = blockIdx.x % nrb, cb = blockIdx.x / nrb;
-    const long row = (long)rb * GN_ROWS + 2 * threadIdx.x;
+    long row = (long)rb * GN_ROWS + 2 * threadIdx.x;
     const int c0 = cb * cbw, c1 = min(n, c0 + cbw);
     if (row >= m) return;
-    const double xa = x[x0 + row * incx];
-    const double xb = row + 1 < m ? x[x0 + (row + 1) * incx] : 0.0;
-    if (vec && row + 1 < m) {
-        double *a = A + row;
-        int c = c0;
-        for (; c + GR_U <= c1; c += GR_U) {
-            d2 v[GR_U];
-            double t[GR_U];
-#pragma unroll
-            for (int u = 0; u < GR_U; ++u) {
-                v[u] = __builtin_nontemporal_load((const d2 *)(a + (long)(c + u) * lda));
-                t[u] = y[y0 + (long)(c + u) * incy];
-            }
-#pragma unroll
-            for (int u = 0; u < GR_U; ++u) {
-                if (t[u] == 0.0) continue;
-                const double ay = alpha * t[u];
-                d2 w;
-                w.x = fma(xa, ay, v[u].x);
-                w.y = fma(xb, ay, v[u].y);
-                __builtin_nontemporal_store(w, (d2 *)(a + (long)(c + u) * lda));
-            }
-        }
-        for (; c < c1; ++c) {
+    const bool odd = row + 1 == m;
+    if (m == 1) {
+        for (int c = c0; c < c1; ++c) {
             const double t = y[y0 + (long)c * incy];
-            if (t == 0.0) continue;
-            const double ay = alpha * t;
-            d2 *p = (d2 *)(a + (long)c * lda);
-            d2 w = *p;
-            w.x = fma(xa, ay, w.x);
-            w.y = fma(xb, ay, w.y);
-            *p = w;
+            double *p = A + (long)c * lda;
+            if (t != 0.0) *p = fma(x[x0], alpha * t, *p);
         }
         return;
     }
-    for (int c = c0; c < c1; ++c) {
+    // the last row of an odd m is the second of a pair whose first is another
+    // lane's: loaded, not stored (a lane of single elements with one column in
+    // flight took 160 us of a 5001 x 5001 update while all others took 80)
+    if (odd) row = m - 2;
+    const double xa = x[x0 + row * incx], xb = x[x0 + (row + 1) * incx];
+    double *a = A + row;
+    auto put = [&](d2 w, long c) {
+        double *p = a + c * lda;
+        if (odd) p[1] = w.y;
+        else __builtin_nontemporal_store(w, (d2u *)p);
+    };
+    int c = c0;
+    for (; c + GR_U <= c1; c += GR_U) {
+        d2 v[GR_U];
+        double t[GR_U];
+#pragma unroll
+        for (int u = 0; u < GR_U; ++u) {
+            v[u] = __builtin_nontemporal_load((const d2u *)(a + (long)(c + u) * lda));
+            t[u] = y[y0 + (long)(c + u) * incy];
+        }
+#pragma unroll
+        for (int u = 0; u < GR_U; ++u) {
+            if (t[u] == 0.0) continue;
+            const double ay = alpha * t[u];
+            d2 w;
+            w.x = fma(xa, ay, v[u].x);
+            w.y = fma(xb, ay, v[u].y);
+            put(w, c + u);
+        }
+    }
+    for (; c < c1; ++c) {
         const double t = y[y0 + (long)c * incy];
         if (t == 0.0) continue;
         const double ay = alpha * t;
-        double *p = A + row + (long)c * lda;
-        p[0] = fma(xa, ay, p[0]);
-        if (row + 1 < m) p[1] = fma(xb, ay, p[1]);
+        const d2 v = *(const d2u *)(a + (long)c * lda);
+        d2 w;
+        w.x = fma(xa, ay, v.x);
+        w.y = fma(xb, ay, v.y);
+        put(w, c);
     }
 }
 
@@ -241,8 +248,7 @@ __global__ __launch_bounds__(256) void ger_stream(int m, int n, double alpha, co
 // at 5.5).  Row sums land in rowP[J][i], column sums in colP[I][j] (one writer
 // each); symv_fold adds them per output in a fixed order and applies alpha /
 // beta.  Diagonal tiles count the diagonal once, in the row sum.  Ragged
-// edge tiles and a misaligned A (16-B loads need an even lda) take a
-// per-element tested path.  The same tiles give DTRMV / DTPMV x := op(T) x
+// edge tiles take a per-element tested path.  The same tiles give DTRMV / DTPMV x := op(T) x
 // with only the row sums ('N') or only the column sums ('T'): one read of the
 // triangle, no copy of x (the fold writes x after every tile has read it).
 constexpr int SY_T = 128;  // tile rows and columns
@@ -251,8 +257,8 @@ constexpr int SY_C = 8;    // columns per LDS pass
 // Tile kinds: interior (16-B loads), diagonal inside the matrix (16-B loads
 // of the whole tile, the unreferenced half -- still inside the caller's
 // lda x n array -- replaced by zeros with a select, so garbage there never
-// reaches the arithmetic), and edge (ragged rows or columns, or a misaligned
-// A: every element tested before it is loaded).
+// reaches the arithmetic), and edge (ragged rows or columns: every element
+// tested before it is loaded).
 enum { SY_INTERIOR = 0, SY_DIAG = 1, SY_EDGE = 2 };
 // What a tile contributes: DSYMV / DSPMV both sums (the diagonal in the row
 // sum only); op(T) x for a stored triangle T (DTRMV / DTPMV) the row sums
@@ -285,7 +291,7 @@ __device__ __forceinline__ void symv_load(d2 (&a)[SY_C], const double *A, long l
                 a[u].x = __builtin_nontemporal_load(A + sy_at<true, LOWER>(ra, j, lda, n));
                 a[u].y = __builtin_nontemporal_load(A + sy_at<true, LOWER>(rb, j, lda, n));
             } else {
-                a[u] = __builtin_nontemporal_load((const d2 *)(A + ra + j * lda));
+                a[u] = __builtin_nontemporal_load((const d2u *)(A + ra + j * lda));
             }
         } else if (KIND == SY_DIAG) {
             d2 v;
@@ -293,7 +299,7 @@ __device__ __forceinline__ void symv_load(d2 (&a)[SY_C], const double *A, long l
                 v.x = __builtin_nontemporal_load(A + sy_at<true, LOWER>(ra, j, lda, n));
                 v.y = __builtin_nontemporal_load(A + sy_at<true, LOWER>(rb, j, lda, n));
             } else {
-                v = __builtin_nontemporal_load((const d2 *)(A + ra + j * lda));
+                v = __builtin_nontemporal_load((const d2u *)(A + ra + j * lda));
             }
             a[u].x = (LOWER ? ra >= j : ra <= j) ? (UNIT && ra == j ? 1.0 : v.x) : 0.0;
             a[u].y = (LOWER ? rb >= j : rb <= j) ? (UNIT && rb == j ? 1.0 : v.y) : 0.0;
@@ -377,7 +383,7 @@ __device__ __forceinline__ void symv_tile_body(int n, int I, int J, const double
 
 template <bool LOWER, bool PACKED, int MODE, bool UNIT>  // template parameters: as run-time
                                     // values the triangle tests turn into branches that wait on every load
-__global__ __launch_bounds__(64) void symv_tile(int n, int nb, int vec, const double *A,
+__global__ __launch_bounds__(64) void symv_tile(int n, int nb, const double *A,
                                                 long lda, const double *x, long incx, long x0,
                                                 double *rowP, double *colP)
 {
@@ -411,7 +417,7 @@ __global__ __launch_bounds__(64) void symv_tile(int n, int nb, int vec, const do
     d2 xi;
     xi.x = ra < n ? x[x0 + ra * incx] : 0.0;
     xi.y = rb < n ? x[x0 + rb * incx] : 0.0;
-    const bool edge = !vec || (long)(I + 1) * SY_T > n || (long)(J + 1) * SY_T > n;
+    const bool edge = (long)(I + 1) * SY_T > n || (long)(J + 1) * SY_T > n;
     if (edge)
         symv_tile_body<SY_EDGE, LOWER, PACKED, MODE, UNIT>(n, I, J, A, lda, xi, xs, rowP, colP, pr);
     else if (I == J)
@@ -470,7 +476,7 @@ __global__ __launch_bounds__(256) void symv_fold(int n, int lower, int nb, int m
 // loads) and then updates and stores them.  Blocks wholly inside the stored
 // triangle and the matrix take that path unconditionally (a column with
 // x(j) == 0 keeps its values, as netlib skips it); blocks cut by the diagonal
-// or the matrix edge, or a misaligned A, test every element; blocks wholly
+// or the matrix edge test every element; blocks wholly
 // outside the triangle return at once.
 constexpr int SR_ROWS = 512;  // rows per workgroup (256 threads x 2)
 constexpr int SR_COLS = 16;   // columns per workgroup
@@ -480,13 +486,13 @@ constexpr int SR_COLS = 16;   // columns per workgroup
 template <bool LOWER, bool TWO>
 __global__ __launch_bounds__(256) void syr_kernel(int n, double alpha, const double *x, long incx,
                                                   long x0, const double *y, long incy, long y0,
-                                                  double *A, long lda, int vec)
+                                                  double *A, long lda)
 {
     const long r0 = (long)blockIdx.x * SR_ROWS, c0 = (long)blockIdx.y * SR_COLS;
     const long rl = r0 + SR_ROWS - 1, cl = c0 + SR_COLS - 1;
     if (LOWER ? rl < c0 : r0 > cl) return;  // no stored element in the block
     const long i = r0 + 2 * threadIdx.x;
-    const bool full = vec && rl < n && cl < n && (LOWER ? r0 >= cl : rl <= c0);
+    const bool full = rl < n && cl < n && (LOWER ? r0 >= cl : rl <= c0);
     double xt[SR_COLS], yt[SR_COLS];
 #pragma unroll
     for (int u = 0; u < SR_COLS; ++u) {
@@ -499,7 +505,7 @@ __global__ __launch_bounds__(256) void syr_kernel(int n, double alpha, const dou
         d2 v[SR_COLS];
 #pragma unroll
         for (int u = 0; u < SR_COLS; ++u)
-            v[u] = __builtin_nontemporal_load((const d2 *)(A + i + (c0 + u) * lda));
+            v[u] = __builtin_nontemporal_load((const d2u *)(A + i + (c0 + u) * lda));
 #pragma unroll
         for (int u = 0; u < SR_COLS; ++u) {
             d2 w;
@@ -513,7 +519,7 @@ __global__ __launch_bounds__(256) void syr_kernel(int n, double alpha, const dou
                 w.x = xt[u] != 0.0 ? fma(xi0, t, v[u].x) : v[u].x;
                 w.y = xt[u] != 0.0 ? fma(xi1, t, v[u].y) : v[u].y;
             }
-            __builtin_nontemporal_store(w, (d2 *)(A + i + (c0 + u) * lda));
+            __builtin_nontemporal_store(w, (d2u *)(A + i + (c0 + u) * lda));
         }
         return;
     }
@@ -630,11 +636,10 @@ int gemv_run(hipStream_t s, char trans, int m, int n, double alpha, const double
                 if (!partials) return (int)hipErrorOutOfMemory;
             }
         }
-        const int vec = (((uintptr_t)d_A & 15) == 0) && (lda % 2 == 0);
         if (prof) prof_begin(s, "dgemv_n");
         hipLaunchKernelGGL(gemv_n_stream, dim3((unsigned)pl.nrb * pl.ncb), dim3(256), 0, s, m, n,
                            alpha, d_A, (long)lda, d_x, (long)incx, x0, beta, d_y, (long)incy, y0,
-                           pl.nrb, pl.cbw, pl.ncb == 1, vec, partials);
+                           pl.nrb, pl.cbw, pl.ncb == 1, partials);
         if (prof) prof_end(s);
         if (pl.ncb > 1) {
             if (prof) prof_begin(s, "dgemv_n_fold");
@@ -644,12 +649,11 @@ int gemv_run(hipStream_t s, char trans, int m, int n, double alpha, const double
         }
         return (int)hipGetLastError();
     }
-    const int vec = (((uintptr_t)d_A & 15) == 0) && (lda % 2 == 0) && (((uintptr_t)d_x & 15) == 0);
     int blocks = ceil_div(n, 4);
     if (blocks > 2048) blocks = 2048;
     if (prof) prof_begin(s, "dgemv_t");
     hipLaunchKernelGGL(gemv_t_kernel, dim3((unsigned)blocks), dim3(256), 0, s, m, n, alpha, d_A,
-                       (long)lda, d_x, (long)incx, x0, beta, d_y, (long)incy, y0, vec);
+                       (long)lda, d_x, (long)incx, x0, beta, d_y, (long)incy, y0);
     if (prof) prof_end(s);
     return (int)hipGetLastError();
 }
@@ -706,11 +710,10 @@ int gpublas_dev_dger(void *stream, int m, int n, double alpha, const double *d_x
     hipStream_t s = pick_stream(stream);
     if (m <= 0 || n <= 0 || alpha == 0.0) return 0;
     const GemvNPlan pl = gemv_n_plan(m, n, 256);
-    const int vec = (((uintptr_t)d_A & 15) == 0) && (lda % 2 == 0);
     PROF_BEGIN(s, "dger");
     hipLaunchKernelGGL(ger_stream, dim3((unsigned)pl.nrb * pl.ncb), dim3(256), 0, s, m, n, alpha,
                        d_x, (long)incx, start_of(m, incx), d_y, (long)incy, start_of(n, incy), d_A,
-                       (long)lda, pl.nrb, pl.cbw, vec);
+                       (long)lda, pl.nrb, pl.cbw);
     PROF_END(s);
     return (int)hipGetLastError();
 }
@@ -721,7 +724,7 @@ namespace {
 // tiles + fold of DSYMV / DSPMV (mode SY_MV_SYM) and of DTRMV / DTPMV
 // (SY_MV_N / SY_MV_T, the result written over x through the fold: every tile
 // has read x before the fold starts), full or packed storage
-int symv_run(hipStream_t s, int lower, bool packed, int mode, bool unit, int vec, int n,
+int symv_run(hipStream_t s, int lower, bool packed, int mode, bool unit, int n,
              double alpha, const double *A, int lda, const double *x, int incx, double beta,
              double *y, int incy, long y0)
 {
@@ -734,7 +737,7 @@ int symv_run(hipStream_t s, int lower, bool packed, int mode, bool unit, int vec
     static const char *const names[2][3] = {{"dsymv", "dtrmv", "dtrmv"}, {"dspmv", "dtpmv", "dtpmv"}};
     PROF_BEGIN(s, names[packed][mode]);
 #define GB_SYT(L, P, M, U)                                                                        \
-    hipLaunchKernelGGL((symv_tile<L, P, M, U>), dim3((unsigned)tiles), dim3(64), 0, s, n, nb, vec, \
+    hipLaunchKernelGGL((symv_tile<L, P, M, U>), dim3((unsigned)tiles), dim3(64), 0, s, n, nb, \
                        A, (long)lda, x, (long)incx, start_of(n, incx), rowP, colP)
 #define GB_SYT_M(L, P)                                                                            \
     {                                                                                             \
@@ -778,8 +781,7 @@ int gpublas_dev_dsymv(void *stream, char uplo, int n, double alpha, const double
         return (int)hipGetLastError();
     }
     const int lower = uplo == 'L' || uplo == 'l';
-    const int vec = (((uintptr_t)d_A & 15) == 0) && (lda % 2 == 0);
-    return symv_run(s, lower, false, SY_MV_SYM, false, vec, n, alpha, d_A, lda, d_x, incx, beta, d_y,
+    return symv_run(s, lower, false, SY_MV_SYM, false, n, alpha, d_A, lda, d_x, incx, beta, d_y,
                     incy, y0);
 }
 
@@ -792,7 +794,7 @@ int gpublas_dev_dspmv(void *stream, char uplo, int n, double alpha, const double
     if (n <= 0) return 0;
     if (alpha == 0.0) return gpublas_dev_dsymv(s, uplo, n, alpha, nullptr, n, d_x, incx, beta, d_y, incy);
     const int lower = uplo == 'L' || uplo == 'l';
-    return symv_run(s, lower, true, SY_MV_SYM, false, 1, n, alpha, d_AP, 0, d_x, incx, beta, d_y,
+    return symv_run(s, lower, true, SY_MV_SYM, false, n, alpha, d_AP, 0, d_x, incx, beta, d_y,
                     incy, start_of(n, incy));
 }
 
@@ -807,8 +809,7 @@ int gpublas_dev_dtrmv(void *stream, char uplo, char trans, char diag, int n, con
     const int lower = uplo == 'L' || uplo == 'l';
     const int mode = trans == 'N' || trans == 'n' ? SY_MV_N : SY_MV_T;
     const bool unit = diag == 'U' || diag == 'u';
-    const int vec = (((uintptr_t)d_A & 15) == 0) && (lda % 2 == 0);
-    return symv_run(s, lower, false, mode, unit, vec, n, 1.0, d_A, lda, d_x, incx, 0.0, d_x, incx,
+    return symv_run(s, lower, false, mode, unit, n, 1.0, d_A, lda, d_x, incx, 0.0, d_x, incx,
                     start_of(n, incx));
 }
 
@@ -820,7 +821,7 @@ int gpublas_dev_dtpmv(void *stream, char uplo, char trans, char diag, int n, con
     const int lower = uplo == 'L' || uplo == 'l';
     const int mode = trans == 'N' || trans == 'n' ? SY_MV_N : SY_MV_T;
     const bool unit = diag == 'U' || diag == 'u';
-    return symv_run(s, lower, true, mode, unit, 1, n, 1.0, d_AP, 0, d_x, incx, 0.0, d_x, incx,
+    return symv_run(s, lower, true, mode, unit, n, 1.0, d_AP, 0, d_x, incx, 0.0, d_x, incx,
                     start_of(n, incx));
 }
 
@@ -830,15 +831,14 @@ int gpublas_dev_dsyr(void *stream, char uplo, int n, double alpha, const double 
     hipStream_t s = pick_stream(stream);
     if (n <= 0 || alpha == 0.0) return 0;
     const bool lower = uplo == 'L' || uplo == 'l';
-    const int vec = (((uintptr_t)d_A & 15) == 0) && (lda % 2 == 0);
     dim3 grid((unsigned)ceil_div(n, SR_ROWS), (unsigned)ceil_div(n, SR_COLS));
     PROF_BEGIN(s, "dsyr");
     if (lower)
         hipLaunchKernelGGL((syr_kernel<true, false>), grid, dim3(256), 0, s, n, alpha, d_x,
-                           (long)incx, start_of(n, incx), d_x, 1L, 0L, d_A, (long)lda, vec);
+                           (long)incx, start_of(n, incx), d_x, 1L, 0L, d_A, (long)lda);
     else
         hipLaunchKernelGGL((syr_kernel<false, false>), grid, dim3(256), 0, s, n, alpha, d_x,
-                           (long)incx, start_of(n, incx), d_x, 1L, 0L, d_A, (long)lda, vec);
+                           (long)incx, start_of(n, incx), d_x, 1L, 0L, d_A, (long)lda);
     PROF_END(s);
     return (int)hipGetLastError();
 }
@@ -849,17 +849,16 @@ int gpublas_dev_dsyr2(void *stream, char uplo, int n, double alpha, const double
     hipStream_t s = pick_stream(stream);
     if (n <= 0 || alpha == 0.0) return 0;
     const bool lower = uplo == 'L' || uplo == 'l';
-    const int vec = (((uintptr_t)d_A & 15) == 0) && (lda % 2 == 0);
     dim3 grid((unsigned)ceil_div(n, SR_ROWS), (unsigned)ceil_div(n, SR_COLS));
     PROF_BEGIN(s, "dsyr2");
     if (lower)
         hipLaunchKernelGGL((syr_kernel<true, true>), grid, dim3(256), 0, s, n, alpha, d_x,
                            (long)incx, start_of(n, incx), d_y, (long)incy, start_of(n, incy), d_A,
-                           (long)lda, vec);
+                           (long)lda);
     else
         hipLaunchKernelGGL((syr_kernel<false, true>), grid, dim3(256), 0, s, n, alpha, d_x,
                            (long)incx, start_of(n, incx), d_y, (long)incy, start_of(n, incy), d_A,
-                           (long)lda, vec);
+                           (long)lda);
     PROF_END(s);
     return (int)hipGetLastError();
 }

@@ -74,8 +74,6 @@ struct GGemv {
     int m, n, trans;
     int split;   // N: column blocks; T: row chunks
     int span;    // N: columns per block; T: rows per chunk
-    int vec_ok;  // A 16-B aligned, lda even
-    int x_vec;   // x 16-B aligned, incx == 1
     int direct;  // split == 1: the partial kernel writes y itself
     long x0, y0; // offsets of logical element 0 (negative strides start at the far end)
     double alpha, beta;
@@ -242,6 +240,10 @@ constexpr int GV_ROWS = 512;    // N: rows per unit (2 per thread)
 constexpr int GV_TCOLS = 16;    // T: columns per unit (4 per wave)
 constexpr int GV_FOLD = 256;    // fold: outputs per unit
 
+// two neighbouring elements, in registers and at any element address
+typedef double d2 __attribute__((ext_vector_type(2)));
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
+
 __device__ __forceinline__ void gemv_out(const GGemv &d, long i, double acc)
 {
     double *y = d.y + d.y0 + i * d.incy;
@@ -253,24 +255,24 @@ __device__ __forceinline__ void gemv_out(const GGemv &d, long i, double acc)
 // columns [cb*span, +span), eight 16-B column loads in flight per lane
 __device__ void gemv_n_unit(const GGemv &d, int local)
 {
-    typedef double d2 __attribute__((ext_vector_type(2)));
     const int nrb = (d.m + GV_ROWS - 1) / GV_ROWS;
     const int rb = local % nrb, cb = local / nrb;
-    const long r0 = (long)rb * GV_ROWS + 2 * (int)threadIdx.x;
+    long r0 = (long)rb * GV_ROWS + 2 * (int)threadIdx.x;
     const int c0 = cb * d.span, c1 = min(d.n, c0 + d.span);
     const double *x = d.x + d.x0;
     const long incx = d.incx;
     double acc0 = 0.0, acc1 = 0.0;
     if (r0 >= d.m) return;
     const bool pair = r0 + 1 < d.m;
-    if (pair && d.vec_ok) {
+    if (d.m > 1) {
+        if (!pair) r0 = d.m - 2;  // the last row of an odd m: the second of a pair
         const double *a = d.A + r0;
         int j = c0;
         for (; j + 8 <= c1; j += 8) {
             d2 v[8];
 #pragma unroll
             for (int u = 0; u < 8; ++u)
-                v[u] = __builtin_nontemporal_load((const d2 *)(a + (long)(j + u) * d.lda));
+                v[u] = __builtin_nontemporal_load((const d2u *)(a + (long)(j + u) * d.lda));
 #pragma unroll
             for (int u = 0; u < 8; ++u) {
                 const double xv = x[(long)(j + u) * incx];
@@ -279,18 +281,14 @@ __device__ void gemv_n_unit(const GGemv &d, int local)
             }
         }
         for (; j < c1; ++j) {
-            const d2 v = *(const d2 *)(a + (long)j * d.lda);
+            const d2 v = *(const d2u *)(a + (long)j * d.lda);
             const double xv = x[(long)j * incx];
             acc0 = fma(v.x, xv, acc0);
             acc1 = fma(v.y, xv, acc1);
         }
+        if (!pair) ++r0, acc0 = acc1;
     } else {
-        for (int j = c0; j < c1; ++j) {
-            const double xv = x[(long)j * incx];
-            const double *a = d.A + r0 + (long)j * d.lda;
-            acc0 = fma(a[0], xv, acc0);
-            if (pair) acc1 = fma(a[1], xv, acc1);
-        }
+        for (int j = c0; j < c1; ++j) acc0 = fma(d.A[(long)j * d.lda], x[(long)j * incx], acc0);
     }
     if (d.direct) {
         gemv_out(d, r0, acc0);
@@ -307,7 +305,6 @@ __device__ void gemv_n_unit(const GGemv &d, int local)
 // row steps (16 loads) in flight
 __device__ void gemv_t_unit(const GGemv &d, int local)
 {
-    typedef double d2 __attribute__((ext_vector_type(2)));
     const int ncb = (d.n + GV_TCOLS - 1) / GV_TCOLS;
     const int cb = local % ncb, rc = local / ncb;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -321,16 +318,16 @@ __device__ void gemv_t_unit(const GGemv &d, int local)
     for (int c = 0; c < 4; ++c) a[c] = d.A + (long)min(j0 + c, d.n - 1) * d.lda;
     const bool cok[4] = {j0 < d.n, j0 + 1 < d.n, j0 + 2 < d.n, j0 + 3 < d.n};
     int i = r0 + 2 * lane;
-    if (d.vec_ok && d.x_vec) {
+    if (incx == 1) {
         // full steps: 4 x 128 rows, every row pair inside [r0, r1)
         for (; i + 3 * 128 + 1 < r1; i += 4 * 128) {
             d2 av[4][4], xv[4];
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                xv[q] = *(const d2 *)(x + i + 128 * q);
+                xv[q] = *(const d2u *)(x + i + 128 * q);
 #pragma unroll
                 for (int c = 0; c < 4; ++c)
-                    av[q][c] = cok[c] ? __builtin_nontemporal_load((const d2 *)(a[c] + i + 128 * q))
+                    av[q][c] = cok[c] ? __builtin_nontemporal_load((const d2u *)(a[c] + i + 128 * q))
                                       : d2{0.0, 0.0};
             }
 #pragma unroll
@@ -342,7 +339,7 @@ __device__ void gemv_t_unit(const GGemv &d, int local)
                 }
         }
     }
-    // remaining rows (and the general-stride / unaligned case)
+    // remaining rows (and the general-stride case)
     for (; i < r1; i += 128) {
         const bool pair = i + 1 < r1;
         const double x0 = x[(long)i * incx];
@@ -903,8 +900,6 @@ int gpublas_dev_batch_dgemv(gpublas_batch *b, char trans, int m, int n, double a
     d.trans = !is_n(trans);
     d.alpha = alpha;
     d.beta = beta;
-    d.vec_ok = (((uintptr_t)d_A & 15) == 0) && (lda % 2 == 0);
-    d.x_vec = (((uintptr_t)d_x & 15) == 0) && incx == 1;
     int units, len;
     if (!d.trans) {
         // N: 512-row blocks; column blocks (>= 64 columns) for about 512 units

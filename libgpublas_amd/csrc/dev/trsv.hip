@@ -40,6 +40,8 @@ constexpr int TTHREADS = 512;     // 8 waves per workgroup
 constexpr int LDD = TB + 1;       // LDS leading dimension of the diagonal block (doubles)
 
 typedef double d2 __attribute__((ext_vector_type(2)));
+// two neighbouring elements at any element address (16-byte accesses need no more)
+typedef double d2u __attribute__((ext_vector_type(2), aligned(8)));
 
 __device__ __forceinline__ double readlane_d(double v, int l)
 {
@@ -185,7 +187,6 @@ struct TrsvLb {
     u64 *xmail;        // nb * kMailWords words
     u64 *pmail;        // nb * nh * kMailWords words
     long long timeout; // steady-clock ticks a wait may last
-    int vec;           // A 16-B aligned with even lda
     int packed, plower;  // A is the packed triangle (DTPSV), lower or upper
 };
 
@@ -284,23 +285,14 @@ __device__ __forceinline__ void tile_load(const TrsvLb &g, int p0, int pn, int c
                                           Tile &tl)
 {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    // whole tiles load unguarded: 16-B loads when A allows them, else
-    // (packed columns at any 8-byte offset) two 8-B loads
-    const bool whole = pn == TB && cn == TB, full = g.vec && whole;
+    const bool full = pn == TB && cn == TB;  // whole tiles load unguarded
     if constexpr (!TRANS) {
         const long r = c0 + 2 * lane;
         const int k0 = 16 * wave;
         if (full) {
 #pragma unroll
             for (int u = 0; u < 16; ++u)
-                tl.v[u] = __builtin_nontemporal_load((const d2 *)(colp(g, p0 + k0 + u) + r));
-        } else if (whole) {
-#pragma unroll
-            for (int u = 0; u < 16; ++u) {
-                const double *a = colp(g, p0 + k0 + u) + r;
-                tl.v[u].x = __builtin_nontemporal_load(a);
-                tl.v[u].y = __builtin_nontemporal_load(a + 1);
-            }
+                tl.v[u] = __builtin_nontemporal_load((const d2u *)(colp(g, p0 + k0 + u) + r));
         } else {
 #pragma unroll
             for (int u = 0; u < 16; ++u) {
@@ -320,10 +312,7 @@ __device__ __forceinline__ void tile_load(const TrsvLb &g, int p0, int pn, int c
             for (int q = 0; q < TB / 16; ++q) {
                 const int e = 16 * q + 2 * j;
                 if (full) {
-                    tl.v[8 * half + q] = __builtin_nontemporal_load((const d2 *)(col + e));
-                } else if (whole) {
-                    tl.v[8 * half + q].x = __builtin_nontemporal_load(col + e);
-                    tl.v[8 * half + q].y = __builtin_nontemporal_load(col + e + 1);
+                    tl.v[8 * half + q] = __builtin_nontemporal_load((const d2u *)(col + e));
                 } else {
                     tl.v[8 * half + q].x = (ii < cn && e < pn) ? col[e] : 0.0;
                     tl.v[8 * half + q].y = (ii < cn && e + 1 < pn) ? col[e + 1] : 0.0;
@@ -447,7 +436,6 @@ __device__ void lb_solver(const TrsvLb &g, int t, double *D, double (*part)[TB],
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     int c0, cn;
     block_of<FWD>(g, t, c0, cn);
-    const bool vec = g.vec != 0;
     const int own = min(2, t), last = t - own;
 
     // the diagonal block, its diagonal, b and the own tiles (one round trip)
@@ -458,16 +446,13 @@ __device__ void lb_solver(const TrsvLb &g, int t, double *D, double (*part)[TB],
         const int idx = tid + u * TTHREADS;
         const int a = 2 * (idx % (TB / 2)), b = idx / (TB / 2);
         const double *src = colp(g, c0 + b) + (c0 + a);
-        if (vec && a + 1 < cn && b < cn) {
-            const d2 v = *(const d2 *)src;
-            va[u] = v.x;
-            vb[u] = v.y;
-        } else if (cn == TB) {
+        if (cn == TB) {
             // a whole block: every address is inside A (packed: the unstored
             // half's addresses are the neighbouring columns'), and no select
             // follows the loads (it would wait for each one in turn)
-            va[u] = src[0];
-            vb[u] = src[1];
+            const d2 v = *(const d2u *)src;
+            va[u] = v.x;
+            vb[u] = v.y;
         } else {
             va[u] = (a < cn && b < cn) ? src[0] : 0.0;
             vb[u] = (a + 1 < cn && b < cn) ? src[1] : 0.0;
@@ -587,7 +572,6 @@ int run(hipStream_t s, int n, const double *A, long lda, bool packed, double *x)
     g.lda = lda;
     g.x = x;
     // packed columns start at any 8-byte offset: element loads only
-    g.vec = !packed && (((uintptr_t)A & 15) == 0) && (lda % 2 == 0);
     g.packed = packed;
     g.plower = LOWER;
     const long words = g.nb > 1 ? (long)g.nb * (1 + g.nh) * kMailWords : 0;
