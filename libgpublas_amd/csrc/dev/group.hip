@@ -109,7 +109,7 @@ static_assert(sizeof(GemmGroup<double>) <= 4000 && sizeof(GemvGroup) <= 4000 &&
                   sizeof(TrsmGroup) <= 4000,
               "group structs must fit a kernel argument");
 
-struct BatchTable {
+struct alignas(16) BatchTable {
     GemmGroup<double> dg[kCfgs];
     GemmGroup<float> sg[kCfgs];
     GemvGroup gv;
@@ -195,33 +195,24 @@ __device__ __forceinline__ void gemm_group_body(const GemmGroup<T> &G)
 // C = alpha * sum_s part_s + beta * C for the split products, 256 elements
 // per unit, chunks summed in order.
 template <typename T>
-__device__ __forceinline__ void gemm_fold_body(const GemmGroup<T> &G)
+__device__ __forceinline__ void gemm_fold_unit(const GemmGroup<T> &G, int u)
 {
-    const int np = min(G.np, kCapGemm);
-    const int total = G.fold_units;
-    for (int u = blockIdx.x; u < total; u += gridDim.x) {
-        const int p = find_unit(&G.p[0].fold_begin, sizeof(GGemm<T>), np, u);
-        const GGemm<T> &e = G.p[p];
-        const long mn = (long)e.g.m * e.g.n;
-        const long idx = (long)(u - e.fold_begin) * 256 + threadIdx.x;
-        if (idx >= mn) continue;
-        T s = T(0);
-        for (int q = 0; q < e.ksplit; ++q) s += e.part[(long)q * mn + idx];
-        T *c = e.g.C + idx % e.g.m + (idx / e.g.m) * e.g.ldc;
-        const T v = e.g.alpha * s;
-        *c = e.g.beta == T(0) ? v : v + e.g.beta * *c;
-    }
+    const int p = find_unit(&G.p[0].fold_begin, sizeof(GGemm<T>), min(G.np, kCapGemm), u);
+    const GGemm<T> &e = G.p[p];
+    const long mn = (long)e.g.m * e.g.n;
+    const long idx = (long)(u - e.fold_begin) * 256 + threadIdx.x;
+    if (idx >= mn) return;
+    T s = T(0);
+    for (int q = 0; q < e.ksplit; ++q) s += e.part[(long)q * mn + idx];
+    T *c = e.g.C + idx % e.g.m + (idx / e.g.m) * e.g.ldc;
+    const T v = e.g.alpha * s;
+    *c = e.g.beta == T(0) ? v : v + e.g.beta * *c;
 }
 
 template <typename T>
 __global__ __launch_bounds__(256) void group_gemm_fold_arg(const GemmGroup<T> G)
 {
-    gemm_fold_body<T>(G);
-}
-template <typename T>
-__global__ __launch_bounds__(256) void group_gemm_fold_tab(const GemmGroup<T> *G)
-{
-    gemm_fold_body<T>(*G);
+    for (int u = blockIdx.x; u < G.fold_units; u += gridDim.x) gemm_fold_unit<T>(G, u);
 }
 
 template <typename T, int BM>
@@ -375,36 +366,63 @@ __device__ __forceinline__ void gemv_part_body(const GemvGroup &G)
     }
 }
 
-__device__ __forceinline__ void gemv_fold_body(const GemvGroup &G)
+__device__ __forceinline__ void gemv_fold_unit(const GemvGroup &G, int u)
 {
-    const int np = min(G.np, kCapGemv);
-    const int total = G.fold_units;
-    for (int u = blockIdx.x; u < total; u += gridDim.x) {
-        const int p = find_unit(&G.p[0].fold_begin, sizeof(GGemv), np, u);
-        const GGemv d = G.p[p];
-        const int len = d.trans ? d.n : d.m;
-        const int i = (u - d.fold_begin) * GV_FOLD + (int)threadIdx.x;
-        if (i >= len) continue;
-        const double *pp = d.part + i;
-        double s = 0.0;
-        int q = 0;
-        for (; q + 4 <= d.split; q += 4) {
-            const double p0 = pp[(long)q * len], p1 = pp[(long)(q + 1) * len];
-            const double p2 = pp[(long)(q + 2) * len], p3 = pp[(long)(q + 3) * len];
-            s += p0;
-            s += p1;
-            s += p2;
-            s += p3;
-        }
-        for (; q < d.split; ++q) s += pp[(long)q * len];
-        gemv_out(d, i, s);
+    const int p = find_unit(&G.p[0].fold_begin, sizeof(GGemv), min(G.np, kCapGemv), u);
+    const GGemv d = G.p[p];
+    const int len = d.trans ? d.n : d.m;
+    const int i = (u - d.fold_begin) * GV_FOLD + (int)threadIdx.x;
+    if (i >= len) return;
+    const double *pp = d.part + i;
+    double s = 0.0;
+    int q = 0;
+    for (; q + 4 <= d.split; q += 4) {
+        const double p0 = pp[(long)q * len], p1 = pp[(long)(q + 1) * len];
+        const double p2 = pp[(long)(q + 2) * len], p3 = pp[(long)(q + 3) * len];
+        s += p0;
+        s += p1;
+        s += p2;
+        s += p3;
     }
+    for (; q < d.split; ++q) s += pp[(long)q * len];
+    gemv_out(d, i, s);
 }
 
 __global__ __launch_bounds__(256) void group_gemv_part_arg(const GemvGroup G) { gemv_part_body(G); }
 __global__ __launch_bounds__(256) void group_gemv_part_tab(const GemvGroup *G) { gemv_part_body(*G); }
-__global__ __launch_bounds__(256) void group_gemv_fold_arg(const GemvGroup G) { gemv_fold_body(G); }
-__global__ __launch_bounds__(256) void group_gemv_fold_tab(const GemvGroup *G) { gemv_fold_body(*G); }
+__global__ __launch_bounds__(256) void group_gemv_fold_arg(const GemvGroup G)
+{
+    for (int u = blockIdx.x; u < G.fold_units; u += gridDim.x) gemv_fold_unit(G, u);
+}
+
+// Every fold of a captured batch in one kernel.
+__global__ __launch_bounds__(256) void group_fold_tab(const BatchTable *t)
+{
+    int total = t->gv.fold_units;
+    for (int c = 0; c < kCfgs; ++c) total += t->dg[c].fold_units + t->sg[c].fold_units;
+    for (int u = blockIdx.x; u < total; u += gridDim.x) {
+        int v = u;
+        if (v < t->gv.fold_units) {
+            gemv_fold_unit(t->gv, v);
+            continue;
+        }
+        v -= t->gv.fold_units;
+        for (int c = 0; c < kCfgs; ++c) {
+            if (v >= 0 && v < t->dg[c].fold_units) gemm_fold_unit<double>(t->dg[c], v);
+            v -= t->dg[c].fold_units;
+            if (v >= 0 && v < t->sg[c].fold_units) gemm_fold_unit<float>(t->sg[c], v);
+            v -= t->sg[c].fold_units;
+        }
+    }
+}
+
+// The batch table, pinned host memory to device memory, 16 bytes a thread: one
+// link round trip (3 us; a copy node took 6.5).
+__global__ __launch_bounds__(256) void table_copy(const uint4 *h, uint4 *d, int n)
+{
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) d[i] = h[i];
+}
 
 // ---- grouped TRSM (left side) ----------------------------------------------
 // One workgroup per 16-column panel of B (trsm_panel.hpp).  Orders past 512
@@ -673,7 +691,6 @@ void launch_gemm_group(gpublas_batch *b, hipStream_t s, int cfg, bool capture)
     if (capture) {
         const GemmGroup<T> *dG = &group_of<T>(b->d_tab, cfg);
         hipLaunchKernelGGL((group_gemm_tab<T, BM>), dim3(fix), dim3(256), 0, s, dG);
-        hipLaunchKernelGGL((group_gemm_fold_tab<T>), dim3(512), dim3(256), 0, s, dG);
         return;
     }
     const int tiles = G.fast_tiles + G.edge_tiles;
@@ -749,30 +766,36 @@ void enqueue(gpublas_batch *b, unsigned mask, bool capture)
         }
         return;
     }
-    (void)hipMemcpyAsync(b->d_tab, b->h_tab, sizeof(BatchTable), hipMemcpyHostToDevice, s0);
+    // Nodes are submitted in the order they are captured here, a few us apart, so
+    // the longest chains come first and the kinds overlap; with the shortest first
+    // they ran one after the other.  A batch of 32 calls, from the first add to the
+    // end of the wait: 123 -> 110 us, about 70 of them the caller's adds.
+    constexpr int words = (int)(sizeof(BatchTable) / 16);
+    hipLaunchKernelGGL(table_copy, dim3(ceil_div(words, 256)), dim3(256), 0, s0,
+                       (const uint4 *)b->h_tab, (uint4 *)b->d_tab, words);
     (void)hipEventRecord(b->ev_fork, s0);
-    sg = b->br[0];
+    for (int i = 0; i < 3; ++i) (void)hipStreamWaitEvent(b->br[i], b->ev_fork, 0);
+    st = b->br[0];
     sv = b->br[1];
-    st = b->br[2];
-    (void)hipStreamWaitEvent(sg, b->ev_fork, 0);
-    (void)hipStreamWaitEvent(sv, b->ev_fork, 0);
-    (void)hipStreamWaitEvent(st, b->ev_fork, 0);
-    if (mask & 1u) launch_gemm_group<double, 32>(b, sg, CFG_32, true);
-    if (mask & 2u) launch_gemm_group<double, 64>(b, sg, CFG_64, true);
-    if (mask & 4u) launch_gemm_group<double, 128>(b, sg, CFG_128, true);
-    if (mask & 8u) launch_gemm_group<float, 32>(b, sg, CFG_32, true);
-    if (mask & 16u) launch_gemm_group<float, 64>(b, sg, CFG_64, true);
-    if (mask & 32u) launch_gemm_group<float, 128>(b, sg, CFG_128, true);
-    if (mask & 64u) {
-        hipLaunchKernelGGL(group_gemv_part_tab, dim3(kGridGemv), dim3(256), 0, sv, &b->d_tab->gv);
-        hipLaunchKernelGGL(group_gemv_fold_tab, dim3(kGridFold), dim3(256), 0, sv, &b->d_tab->gv);
-    }
+    sg = b->br[2];
     if (mask & 128u)
         hipLaunchKernelGGL(group_trsm_tab, dim3(kGridTrsm), dim3(TP_THREADS), 0, st, &b->d_tab->tr);
-    (void)hipEventRecord(b->ev_join[0], sg);
+    if (mask & 64u)
+        hipLaunchKernelGGL(group_gemv_part_tab, dim3(kGridGemv), dim3(256), 0, sv, &b->d_tab->gv);
+    if (mask & 4u) launch_gemm_group<double, 128>(b, s0, CFG_128, true);
+    if (mask & 32u) launch_gemm_group<float, 128>(b, sg, CFG_128, true);
+    if (mask & 2u) launch_gemm_group<double, 64>(b, s0, CFG_64, true);
+    if (mask & 16u) launch_gemm_group<float, 64>(b, sg, CFG_64, true);
+    if (mask & 1u) launch_gemm_group<double, 32>(b, s0, CFG_32, true);
+    if (mask & 8u) launch_gemm_group<float, 32>(b, sg, CFG_32, true);
     (void)hipEventRecord(b->ev_join[1], sv);
-    (void)hipEventRecord(b->ev_join[2], st);
-    for (int i = 0; i < 3; ++i) (void)hipStreamWaitEvent(s0, b->ev_join[i], 0);
+    (void)hipEventRecord(b->ev_join[2], sg);
+    (void)hipStreamWaitEvent(s0, b->ev_join[1], 0);
+    (void)hipStreamWaitEvent(s0, b->ev_join[2], 0);
+    if (mask & 127u)
+        hipLaunchKernelGGL(group_fold_tab, dim3(kGridFold), dim3(256), 0, s0, b->d_tab);
+    (void)hipEventRecord(b->ev_join[0], st);
+    (void)hipStreamWaitEvent(s0, b->ev_join[0], 0);
 }
 
 // Branch streams exist only for capture: created on the first capture, so
