@@ -45,6 +45,7 @@ struct OzArgs {
     int M, N, Mp, Np, KT;   // Mp, Np: rows padded to 128; KT: 16-deep k slabs
     const bf16 *SA, *SB;    // [s][KT][Mp][16], [s][KT][Np][16]
     const int *ea, *eb;     // row exponents of op(A), column exponents of op(B)
+    const int *bad;         // set: an input holds an Inf or NaN
     double alpha, beta;
     double *C;
     long ldc;
@@ -63,6 +64,21 @@ __device__ __forceinline__ int exp_of(double mx)
     return e;
 }
 
+// Largest |v| so far, and whether any v was Inf or NaN.  Kept in registers over
+// a line: a store to `bad` inside the loop keeps the compiler from moving the next
+// loads ahead of it (4096^2: 46 us with one load in flight per lane, 28 to 36 with
+// eight).
+struct LineMax {
+    double mx = 0;
+    bool odd = false;
+    __device__ __forceinline__ void take(double x)
+    {
+        const double v = fabs(x);
+        odd |= !(v <= 1.7976931348623157e308);
+        mx = fmax(mx, v);
+    }
+};
+
 // line r of an operand stored so that consecutive r are contiguous
 // (element (r, k) at X[r + k*ld]): thread per line, coalesced over r, with K
 // cut into gridDim.y chunks so the pass fills the chip; chunk c writes the
@@ -73,22 +89,43 @@ __global__ void exp_rows_strided(int R, int K, const double *X, long ld, double 
     if (r >= R) return;
     const int chunk = (K + gridDim.y - 1) / gridDim.y;
     const int k0 = blockIdx.y * chunk, k1 = min(K, k0 + chunk);
-    double mx = 0;
-    for (int k = k0; k < k1; ++k) {
-        const double v = fabs(X[r + (long)k * ld]);
-        if (!(v <= 1.7976931348623157e308)) *bad = 1;
-        mx = fmax(mx, v);
+    LineMax m;
+    int k = k0;
+    for (; k + 8 <= k1; k += 8) {
+        double v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = X[r + (long)(k + u) * ld];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) m.take(v[u]);
     }
-    part[(long)blockIdx.y * R + r] = mx;
+    for (; k < k1; ++k) m.take(X[r + (long)k * ld]);
+    if (m.odd) *bad = 1;
+    part[(long)blockIdx.y * R + r] = m.mx;
 }
 
+// four threads per line, each over every fourth chunk
 __global__ void exp_rows_finish(int R, int chunks, const double *part, int *e)
 {
-    const long r = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (r >= R) return;
+    const long r = (long)blockIdx.x * (blockDim.x / 4) + threadIdx.x % (blockDim.x / 4);
+    const int q = threadIdx.x / (blockDim.x / 4);
+    __shared__ double t[256];
     double mx = 0;
-    for (int c = 0; c < chunks; ++c) mx = fmax(mx, part[(long)c * R + r]);
-    e[r] = exp_of(mx);
+    if (r < R) {
+        int c = q;
+        for (; c + 28 < chunks; c += 32) {
+            double v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = part[(long)(c + 4 * u) * R + r];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) mx = fmax(mx, v[u]);
+        }
+        for (; c < chunks; c += 4) mx = fmax(mx, part[(long)c * R + r]);
+    }
+    t[threadIdx.x] = mx;
+    __syncthreads();
+    if (q == 0 && r < R)
+        e[r] = exp_of(fmax(fmax(t[threadIdx.x], t[threadIdx.x + 64]),
+                           fmax(t[threadIdx.x + 128], t[threadIdx.x + 192])));
 }
 
 // line r stored contiguously (element (r, k) at X[k + r*ld]): one wave per line.
@@ -97,12 +134,19 @@ __global__ void exp_rows_contig(int R, int K, const double *X, long ld, int *e, 
     const int lane = threadIdx.x & 63;
     const long r = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
     if (r >= R) return;
-    double mx = 0;
-    for (int k = lane; k < K; k += 64) {
-        const double v = fabs(X[k + r * ld]);
-        if (!(v <= 1.7976931348623157e308)) *bad = 1;
-        mx = fmax(mx, v);
+    const double *x = X + r * ld;
+    LineMax m;
+    int k = lane;
+    for (; k + 64 * 7 < K; k += 64 * 8) {
+        double v[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v[u] = x[k + 64 * u];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) m.take(v[u]);
     }
+    for (; k < K; k += 64) m.take(x[k]);
+    if (m.odd) *bad = 1;
+    double mx = m.mx;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o, 64));
     if (lane == 0) e[r] = exp_of(mx);
@@ -309,6 +353,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void ozaki_gemm_kernel(OzArgs g)
         else return L3.r;
     };
 
+    if (*g.bad) return;  // an input is not finite: C is left to the FP64 kernel
     int tm, tn;
     tile_of(blockIdx.x, g.tiles_m, g.tiles_n, tm, tn);
     const int m0 = tm * TM, n0 = tn * TN;
@@ -508,6 +553,7 @@ struct OzI8Args {
     int kt0, nkt;           // slabs [kt0, kt0 + nkt) in this launch
     const int8_t *SA, *SB;  // [s][KT][Mp][32], [s][KT][Np][32]
     const int *ea, *eb;
+    const int *bad;  // set: an input holds an Inf or NaN
     double alpha, beta;
     double *C;
     long ldc;
@@ -549,6 +595,7 @@ __global__ __launch_bounds__(64 * NW, OCC) void ozaki_i8_kernel(OzI8Args g)
         else return L3.r;
     };
 
+    if (*g.bad) return;  // an input is not finite: C is left to the FP64 kernel
     int tm, tn;
     tile_of(blockIdx.x, g.tiles_m, g.tiles_n, tm, tn);
     const int m0 = tm * TM, n0 = tn * TN;
@@ -749,7 +796,7 @@ int make_split(hipStream_t st, int R, int K, int KT, int s, const double *X, lon
         const int chunks = exp_chunks(R, K);
         hipLaunchKernelGGL(exp_rows_strided, dim3((unsigned)ceil_div(R, 256), (unsigned)chunks),
                            dim3(256), 0, st, R, K, X, ld, part, bad);
-        hipLaunchKernelGGL(exp_rows_finish, dim3((unsigned)ceil_div(R, 256)), dim3(256), 0, st, R,
+        hipLaunchKernelGGL(exp_rows_finish, dim3((unsigned)ceil_div(R, 64)), dim3(256), 0, st, R,
                            chunks, part, out.e);
     } else
         hipLaunchKernelGGL(exp_rows_contig, dim3((unsigned)ceil_div(R, 4)), dim3(256), 0, st, R, K,
@@ -781,7 +828,7 @@ void launch_i8(hipStream_t st, unsigned blocks, const OzI8Args &g)
 // INT8 slice products over all KT slabs: one launch per i8_max_slabs(s)
 // slabs, the later ones accumulating into C (beta 1).
 int run_products_i8(hipStream_t st, int M, int N, int KT, int s, const Split &a, const Split &b,
-                    double alpha, double beta, double *C, int ldc, int tri)
+                    const int *bad, double alpha, double beta, double *C, int ldc, int tri)
 {
     OzI8Args g;
     g.M = M;
@@ -792,6 +839,7 @@ int run_products_i8(hipStream_t st, int M, int N, int KT, int s, const Split &a,
     g.SA = a.S8;
     g.SB = b.S8;
     g.ea = a.e;
+    g.bad = bad;
     g.eb = b.e;
     g.alpha = alpha;
     g.C = C;
@@ -830,7 +878,7 @@ void launch_products(hipStream_t st, unsigned blocks, const OzArgs &g)
 }
 
 int run_products(hipStream_t st, int M, int N, int KT, int s, int f16, const Split &a,
-                 const Split &b, double alpha, double beta, double *C, int ldc, int tri)
+                 const Split &b, const int *bad, double alpha, double beta, double *C, int ldc, int tri)
 {
     OzArgs g;
     g.M = M;
@@ -841,6 +889,7 @@ int run_products(hipStream_t st, int M, int N, int KT, int s, int f16, const Spl
     g.SA = a.S;
     g.SB = b.S;
     g.ea = a.e;
+    g.bad = bad;
     g.eb = b.e;
     g.alpha = alpha;
     g.beta = beta;
@@ -909,19 +958,19 @@ int gpublas_dev_dgemm_split_fmt(void *stream, int slices, int fmt, char transa, 
     int err = make_split(st, m, k, KT, slices, d_A, lda, isN(transa), fmt, a, bad, ws.part);
     // op(B) columns: B 'N' -> element (k, j) at B[k + j*ldb] (k contiguous); 'T' -> B[j + k*ldb]
     if (!err) err = make_split(st, n, k, KT, slices, d_B, ldb, !isN(transb), fmt, b, bad, ws.part);
+    // The products are queued behind the splitting and leave C alone where the
+    // flag is set (a host check between the two cost 20 to 30 us of an idle GPU).
+    if (!err && i8)
+        err = run_products_i8(st, m, n, KT, slices, a, b, bad, alpha, beta, d_C, ldc, 0);
+    else if (!err)
+        err = run_products(st, m, n, KT, slices, fmt == GPUBLAS_SLICE_FP16, a, b, bad, alpha, beta,
+                           d_C, ldc, 0);
     int hbad = 0;
     if (!err) err = (int)hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, st);
     if (!err) err = (int)hipStreamSynchronize(st);
-    if (!err) {
-        if (hbad)  // Inf / NaN input: the splitting is undefined, use the FP64 kernel
-            err = gpublas_gemm_d(st, transa, transb, m, n, k, alpha, d_A, lda, d_B, ldb, beta, d_C, ldc);
-        else if (i8)
-            err = run_products_i8(st, m, n, KT, slices, a, b, alpha, beta, d_C, ldc, 0);
-        else
-            err = run_products(st, m, n, KT, slices, fmt == GPUBLAS_SLICE_FP16, a, b, alpha, beta,
-                               d_C, ldc, 0);
-    }
-    (void)hipStreamSynchronize(st);
+    if (!err && hbad)  // Inf / NaN input: the splitting is undefined, use the FP64 kernel
+        err = gpublas_gemm_d(st, transa, transb, m, n, k, alpha, d_A, lda, d_B, ldb, beta, d_C, ldc);
+    if (err || hbad) (void)hipStreamSynchronize(st);
     free_split(a);
     free_split(b);
     return err;
@@ -956,17 +1005,17 @@ int gpublas_dev_dsyrk_split_fmt(void *stream, int slices, int fmt, char uplo, ch
     Split a{};
     // op(A) = A (trans N: rows contiguous) or A^T; op(B) = op(A)^T has the same lines
     int err = make_split(st, n, k, KT, slices, d_A, lda, isN(trans), fmt, a, bad, ws.part);
+    const int tri = (uplo == 'U' || uplo == 'u') ? 2 : 1;
+    if (!err && i8)
+        err = run_products_i8(st, n, n, KT, slices, a, a, bad, alpha, beta, d_C, ldc, tri);
+    else if (!err)
+        err = run_products(st, n, n, KT, slices, fmt == GPUBLAS_SLICE_FP16, a, a, bad, alpha, beta,
+                           d_C, ldc, tri);
     int hbad = 0;
     if (!err) err = (int)hipMemcpyAsync(&hbad, bad, sizeof(int), hipMemcpyDeviceToHost, st);
     if (!err) err = (int)hipStreamSynchronize(st);
-    if (!err) {
-        const int tri = (uplo == 'U' || uplo == 'u') ? 2 : 1;
-        if (hbad) err = gpublas_dev_dsyrk(st, uplo, trans, n, k, alpha, d_A, lda, beta, d_C, ldc);
-        else if (i8) err = run_products_i8(st, n, n, KT, slices, a, a, alpha, beta, d_C, ldc, tri);
-        else err = run_products(st, n, n, KT, slices, fmt == GPUBLAS_SLICE_FP16, a, a, alpha, beta,
-                                d_C, ldc, tri);
-    }
-    (void)hipStreamSynchronize(st);
+    if (!err && hbad) err = gpublas_dev_dsyrk(st, uplo, trans, n, k, alpha, d_A, lda, beta, d_C, ldc);
+    if (err || hbad) (void)hipStreamSynchronize(st);
     free_split(a);
     return err;
 }
