@@ -183,9 +183,8 @@ def gemm_figures():
         bufs = [lib.gpublas_dev_alloc(n * n * 8) for _ in range(3)]
         for i, b in enumerate(bufs):
             lib.gpublas_dev_fill_uniform(None, 101 + i, n * n, b)
-        # 1024^3 runs as split-K over 64 x 64 tiles (its 256 tiles fill half
-        # the workgroup slots); 8192^3 on 128 x 128 tiles
-        kerns = ["dgemm_fast_128x128"] if n >= 2048 else ["dgemm_splitk", "dgemm_fast_64x64"]
+        # 1024^3 runs on 64 x 64 tiles (one a CU), 8192^3 on 128 x 64 ones
+        kerns = ["dgemm_fast_128x64"] if n >= 2048 else ["dgemm_fast_64x64"]
         for _ in range(2):
             lib.gpublas_dev_dgemm(None, b"N", b"N", n, n, n, 1.0, bufs[0], n, bufs[1], n, 0.5, bufs[2], n)
         lib.gpublas_dev_sync(None)
@@ -342,7 +341,7 @@ def split_suite(n=8192, variants=SPLIT_VARIANTS):
                     lib.gpublas_dev_dgemm_split_fmt(None, s, SLICE_FMT[fmt], b"N", b"N", n, n, n,
                                                     1.0, dA, n, dB, n, 0.0, dC, n)
             lib.gpublas_dev_sync(None)
-            ms = ktime(["dgemm_fast_128x128"] if kind == "fp64" else
+            ms = ktime(["dgemm_fast_128x64"] if kind == "fp64" else
                        ["ozaki_split", "ozaki_i8" if fmt == "int8" else "ozaki_gemm"]) / 2
             lib.gpublas_dev_d2h(host.ctypes.data, dC, bytes_, None)
             lib.gpublas_dev_sync(None)

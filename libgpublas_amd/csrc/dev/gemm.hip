@@ -4,8 +4,9 @@
 // Replaces the vendor calls at blas_level3/gemm.cc:62-82 (cublasDgemm),
 // syrk.cc:57-75 (cublasDsyrk) and symm.cc:57-78 (cublasDsymm).
 //
-// One tile routine (gemm_tile.hpp) serves all three routines, plus a
-// specialised full-tile kernel for aligned rectangular operands:
+// Products at least 32 wide in both dimensions run on the fast tile (any
+// alignment, ragged edges by moved-back tiles, a tile shape by cost); the generic
+// tile (both in gemm_tile.hpp) serves the rest and symmetric operands:
 //  * SYRK is the same product with B = A (transposed), restricted to tiles
 //    on and below (above) the diagonal and masked to the triangle;
 //  * SYMM reads the symmetric operand from its stored triangle: per k-tile
@@ -190,7 +191,9 @@ long device_cus()
 // CUs idle: k is cut into as many chunks as fill them (at most 16, each at least
 // 256 deep, a multiple of 16; the fold costs about 5 us, 256 of k about 3).  More
 // than one workgroup a CU gains too little to pay the fold.  Returns -1 when the
-// shape does not qualify, so the caller takes the ordinary grid.
+// shape does not qualify, when no scratch is left, or while s records a graph (a
+// replay would find the partial sums' pool block in other hands), so the caller
+// takes the ordinary grid.
 template <typename T>
 int launch_splitk(hipStream_t s, const GemmArgs<T> &g, int m, int n, int k)
 {
@@ -199,6 +202,11 @@ int launch_splitk(hipStream_t s, const GemmArgs<T> &g, int m, int n, int k)
     if (want < 2) return -1;
     const int kchunk = ceil_div(ceil_div(k, want), 16) * 16, ks = ceil_div(k, kchunk);
     if (ks < 2) return -1;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return -1;
+    }
     T *P = (T *)gpublas_dev_alloc((size_t)ks * m * n * sizeof(T));
     if (!P) return -1;
     GemmArgs<T> f = g;

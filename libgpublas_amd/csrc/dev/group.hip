@@ -21,9 +21,8 @@
 //  * group_gemm_arg / _tab<T, S>: every tile of every GEMM problem that the
 //    tile-shape table assigns to shape S (FastShape), in one grid;
 //    tile t -> problem by binary search over the prefix sums; the tile
-//    itself is the per-call fast tile routine (gemm_tile.hpp; its guarded
-//    variant for ragged tiles), so a product's bits do not depend on the
-//    batch;
+//    itself is the per-call fast tile routine (gemm_tile.hpp), so a
+//    product's bits do not depend on the batch;
 //  * group_gemv_part_kernel / group_gemv_fold_kernel: y = alpha*op(A)*x +
 //    beta*y as column-block (N) or row-chunk (T) partial sums followed by a
 //    fixed-order fold; the split depends only on (m, n);
@@ -723,7 +722,7 @@ void kind_costs(const BatchTable *t, double (&cost)[4])
 }
 
 // Enqueue the batch's kernels.  Captured: fixed persistent grids reading
-// the device table (copied by the first node), the three kinds on parallel
+// the device table (copied by the first node), the kinds on parallel
 // branches.  Eager: grids capped by the work, groups passed by value, kinds
 // in increasing estimated cost, each followed by its completion event.
 void enqueue(gpublas_batch *b, unsigned mask, bool capture)

@@ -39,7 +39,7 @@ inline int gemm_t(hipStream_t s, char ta, char tb, int m, int n, int k, float al
 // sides (trsm_panel.hpp).  The smaller SB, the more workgroups share a CU (4, 2,
 // 1: LDS) and the shorter the prologue.  Measured with 4096 right-hand sides,
 // left, lower, FP64 (FP32): order 16 8.0 -> 4.4 us (7.6 -> 4.2), 128 16.4 -> 8.3
-// (30.7 -> 7.9), 256 23.6 -> 15.0 (50.0 -> 14.3), 512 67.4 -> 36.6 in one launch
+// (30.7 -> 7.9), 256 23.6 -> 15.0 (50.0 -> 14.3), 512 67.4 -> 35.4 in one launch
 // instead of two solves and a product (115 -> 35.8); order 64 with 100000 right-
 // hand sides 151 -> 56 us (103 -> 51).
 template <typename T, int SB, bool KC>

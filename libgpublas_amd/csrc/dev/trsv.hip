@@ -571,13 +571,13 @@ int run(hipStream_t s, int n, const double *A, long lda, bool packed, double *x)
     g.A = A;
     g.lda = lda;
     g.x = x;
-    // packed columns start at any 8-byte offset: element loads only
     g.packed = packed;
     g.plower = LOWER;
     const long words = g.nb > 1 ? (long)g.nb * (1 + g.nh) * kMailWords : 0;
     g.xmail = g.pmail = nullptr;
+    Scratch scr;  // lives until the launches that use it are enqueued
     if (words) {
-        Scratch scr = dev_scratch((size_t)words * sizeof(u64), s);
+        scr = dev_scratch((size_t)words * sizeof(u64), s);
         if (!scr.p) return (int)hipErrorOutOfMemory;
         g.xmail = (u64 *)scr.p;
         g.pmail = g.xmail + (long)g.nb * kMailWords;

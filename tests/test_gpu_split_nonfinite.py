@@ -7,18 +7,15 @@ import ctypes
 import numpy as np
 import pytest
 
+from _devmem import Matrix
+
 pytestmark = pytest.mark.gpu
 FORMATS = [(0, 6), (1, 5), (2, 7)]  # BF16, FP16, INT8 with their slices
 
 
-def _device(a):
-    import torch
-    return torch.tensor(np.ascontiguousarray(a.T), device="cuda")
-
-
 def _call(gpu, f, *args):
     conv = [ctypes.c_char(a.encode()) if isinstance(a, str) else ctypes.c_double(a)
-            if isinstance(a, float) else ctypes.c_void_p(a.data_ptr()) if hasattr(a, "data_ptr")
+            if isinstance(a, float) else ctypes.c_void_p(a.ptr) if isinstance(a, Matrix)
             else a for a in args]
     assert f(None, *conv) == 0
     gpu.sync()
@@ -29,7 +26,6 @@ def _call(gpu, f, *args):
 @pytest.mark.parametrize("m,n,k,at", [(70, 65, 33, (0, 0)), (130, 64, 71, (129, 70)),
                                       (64, 200, 600, (13, 517))])
 def test_gemm(gpu, fmt, slices, bad, m, n, k, at):
-    import torch
     lib = gpu.library()
     rng = np.random.default_rng(m)
     a, b, c = (rng.uniform(-1, 1, s) for s in ((m, k), (k, n), (m, n)))
@@ -37,21 +33,22 @@ def test_gemm(gpu, fmt, slices, bad, m, n, k, at):
         if inject:
             (a if inject == "a" else b.T)[at[0] % (m if inject == "a" else n), at[1]] = bad
         for ta, tb in (("N", "N"), ("T", "T")):
-            A = _device(a if ta == "N" else a.T)
-            B = _device(b if tb == "N" else b.T)
-            C, D = _device(c), _device(c)
-            torch.cuda.synchronize()
-            shape = (ta, tb, m, n, k, 1.5, A, A.shape[1], B, B.shape[1], -0.5)
+            A = Matrix(gpu, a if ta == "N" else a.T)
+            B = Matrix(gpu, b if tb == "N" else b.T)
+            C, D = Matrix(gpu, c), Matrix(gpu, c)
+            shape = (ta, tb, m, n, k, 1.5, A, A.like.shape[0], B, B.like.shape[0], -0.5)
             _call(gpu, lib.gpublas_dev_dgemm_split_fmt, slices, fmt, *shape, C, m)
             _call(gpu, lib.gpublas_dev_dgemm, *shape, D, m)
+            got, plain = C.get(), D.get()
+            for x in (A, B, C, D):
+                x.free()
             if inject:
-                assert torch.equal(C.view(torch.int64), D.view(torch.int64)) or \
-                    np.array_equal(C.cpu().numpy(), D.cpu().numpy(), equal_nan=True)
+                assert np.array_equal(got, plain, equal_nan=True)
             else:
                 # s slices of w bits leave k products of relative size 2^-(w s) each
                 w = 7 if fmt == 2 else 8
                 bound = 4 * k * 2.0 ** -(w * slices) + 64 * np.finfo(float).eps * np.sqrt(k)
-                assert float((C - D).abs().max()) <= bound * 1.5
+                assert np.abs(got - plain).max() <= bound * 1.5
         if inject == "a":
             a = rng.uniform(-1, 1, (m, k))
 
@@ -59,16 +56,16 @@ def test_gemm(gpu, fmt, slices, bad, m, n, k, at):
 @pytest.mark.parametrize("fmt,slices", FORMATS)
 @pytest.mark.parametrize("uplo,trans", [("L", "N"), ("U", "T")])
 def test_syrk(gpu, fmt, slices, uplo, trans):
-    import torch
     lib = gpu.library()
     n, k = 133, 75
     rng = np.random.default_rng(3)
     a, c = rng.uniform(-1, 1, (n, k)), rng.uniform(-1, 1, (n, n))
     a[100, 40] = np.nan
-    A = _device(a if trans == "N" else a.T)
-    C, D = _device(c), _device(c)
-    torch.cuda.synchronize()
-    shape = (uplo, trans, n, k, 1.0, A, A.shape[1], 0.25)
+    A = Matrix(gpu, a if trans == "N" else a.T)
+    C, D = Matrix(gpu, c), Matrix(gpu, c)
+    shape = (uplo, trans, n, k, 1.0, A, A.like.shape[0], 0.25)
     _call(gpu, lib.gpublas_dev_dsyrk_split_fmt, slices, fmt, *shape, C, n)
     _call(gpu, lib.gpublas_dev_dsyrk, *shape, D, n)
-    assert np.array_equal(C.cpu().numpy(), D.cpu().numpy(), equal_nan=True)
+    assert np.array_equal(C.get(), D.get(), equal_nan=True)
+    for x in (A, C, D):
+        x.free()

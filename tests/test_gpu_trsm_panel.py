@@ -13,6 +13,8 @@ import math
 import numpy as np
 import pytest
 
+from _devmem import Matrix
+
 pytestmark = pytest.mark.gpu
 EPS64, EPS32 = np.finfo(np.float64).eps, np.finfo(np.float32).eps
 FORMS = [(s, u, t, d) for s in "LR" for u in "LU" for t in "NT" for d in "NU"]
@@ -77,20 +79,20 @@ def test_panel_orders(gpu, single, side, uplo, trans, diag):
 @pytest.mark.parametrize("uplo,trans", [("L", "N"), ("L", "T"), ("U", "N"), ("U", "T")])
 @pytest.mark.parametrize("diag", ["N", "U"])
 def test_batch_panel_orders(gpu, uplo, trans, diag):
-    import torch
     for m, n in ((1, 16), (33, 5), (256, 17), (257, 16), (512, 20), (513, 16), (900, 3), (1024, 18)):
         rng = np.random.default_rng(m)
         a, b = _triangle(rng, m, diag, np.float64), rng.uniform(-1, 1, (m, n))
-        A, B = (torch.tensor(np.ascontiguousarray(x.T), device="cuda") for x in (a, b))
-        torch.cuda.synchronize()
+        A, B = Matrix(gpu, a), Matrix(gpu, b)
         slot = gpu.Batch(use_graph=False)
         try:
-            assert slot.dtrsm("L", uplo, trans, diag, m, n, 2.0, A.data_ptr(), m, B.data_ptr(), m) == 0
+            assert slot.dtrsm("L", uplo, trans, diag, m, n, 2.0, A.ptr, m, B.ptr, m) == 0
             slot.run()
         finally:
             slot.close()
-        got, want = B.cpu().numpy().T, _substitute(a, 2.0 * b, uplo, trans, diag)
+        got, want = B.get(), _substitute(a, 2.0 * b, uplo, trans, diag)
         err = np.linalg.norm((got - want).astype(np.float64)) / np.linalg.norm(want.astype(np.float64))
+        A.free()
+        B.free()
         assert err <= m * EPS64, (m, n, err)
 
 
