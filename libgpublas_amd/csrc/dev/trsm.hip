@@ -38,10 +38,11 @@ inline int gemm_t(hipStream_t s, char ta, char tb, int m, int n, int k, float al
 // Base solve of an order of at most 128 * SB, one workgroup per 16 right-hand
 // sides (trsm_panel.hpp).  The smaller SB, the more workgroups share a CU (4, 2,
 // 1: LDS) and the shorter the prologue.  Measured with 4096 right-hand sides,
-// left, lower, FP64 (FP32): order 16 8.0 -> 4.4 us (7.6 -> 4.2), 128 16.4 -> 8.3
-// (30.7 -> 7.9), 256 23.6 -> 15.0 (50.0 -> 14.3), 512 67.4 -> 35.4 in one launch
-// instead of two solves and a product (115 -> 35.8); order 64 with 100000 right-
-// hand sides 151 -> 56 us (103 -> 51).
+// left, lower, FP64 (FP32): order 16 8.0 -> 4.6 us (7.6 -> 4.5), 128 16.4 -> 8.3
+// (30.7 -> 8.0), 256 23.6 -> 14.5 (50.0 -> 14.0), 512 67.4 -> 35.8 in one launch
+// instead of two solves and a product (115 -> 34.7); order 64 with 100000 right-
+// hand sides 151 -> 53 us (103 -> 55).  With every diagonal block substituted, FP64:
+// order 16 6.2 us, 128 22.6, 256 43.8, 512 92.
 template <typename T, int SB, bool KC>
 __global__ __launch_bounds__(TP_THREADS) void trsm_base(int order, int n, double alpha, const T *A,
                                                         long lda, int transN, int lower, int unit,

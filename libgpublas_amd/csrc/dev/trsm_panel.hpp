@@ -10,12 +10,14 @@
 // rounded once.
 //
 //  * Prologue: the 16 x 16 diagonal blocks are inverted in LDS, four per wave,
-//    one lane per column, while the panel's loads are still in flight.
+//    one lane per column, while the panel's loads are still in flight.  A block
+//    whose inverse would cost accuracy (kInverseGrowth) stays as it is.
 //  * Wave w keeps the sums of T[J, I] X_I over the solved blocks I for its blocks
 //    J = w, w + 8, ... in MFMA accumulators.  When X of block st is published,
 //    every wave adds T[J, st] X_st for its later blocks, the owner of block st + 1
 //    that one first: it then forms X = inv(T_JJ) (B_J - sum) (the accumulator
-//    layout is the operand layout) and publishes it.
+//    layout is the operand layout), or substitutes where the block was left, and
+//    publishes it.
 //  * No barrier between steps: X_st is followed by a flag word in LDS, and a
 //    wave waits for that word alone, so the chain of solves never waits for
 //    the other blocks' updates.  The next owner reads word and X together (LDS
@@ -27,10 +29,11 @@
 // Bound: per step the chain of 4 + 4 dependent v_mfma_f64_16x16x4 (64 cycles
 // each) and two LDS trips: 0.7 us a block where barriers between the steps and
 // substitution or an LDS wait before each read took 1.0 to 1.4.  Order 256, 4096
-// right-hand sides: 15 us, 4 of them the loads and the inversion.
-// Error of FP64 solves against 80-bit arithmetic, orders 64..2000: 1.0 to 2.7e-16
-// (substitution and recursion with products: 1.9 to 4.8e-16); FP32: 2.5e-8 up to
-// order 512, 1.4e-7 at 2000 (1.4 to 3.2e-7).
+// right-hand sides: 14.5 us, 4 of them the loads and the inversion.
+// Error of FP64 solves against 80-bit arithmetic, orders 64..2000, triangles whose
+// diagonal outweighs their other entries: 1.0 to 2.7e-16 (substitution and
+// recursion with products: 1.9 to 4.8e-16); FP32: 2.5e-8 up to order 512, 1.4e-7 at
+// 2000 (1.4 to 3.2e-7).
 #pragma once
 #include "devcommon.hpp"
 #include <type_traits>
@@ -38,6 +41,17 @@
 namespace {
 
 constexpr int TP_WAVES = 8, TP_THREADS = 64 * TP_WAVES;
+
+// A product with the inverse Y of a block T can leave a residual far above that of
+// a substitution.  How far shows in the inverse of the block scaled to a unit
+// diagonal, Y_ij T_jj: a block with an entry beyond this limit is substituted.
+// Residuals over random blocks, in units of u |T| |X| (substitution: up to 3):
+// factors with a dominant diagonal, Cholesky factors and the L of a pivoted LU have
+// entries up to 3 and leave 2 to 5; blocks within the limit 25 at most but for a few
+// near bidiagonal ones (80); past it, off-diagonal entries to 2 beside a unit
+// diagonal 600, entries to 4 1e5, the R of a 16-term monomial fit 2300.  FP32
+// operands are solved in FP64: 2^20 times the limit is still far below their u.
+template <typename IO> constexpr double kInverseGrowth = sizeof(IO) == 8 ? 4.0 : 4194304.0;
 
 // LDS of one panel of order up to 128 * SB.
 template <int SB>
@@ -47,6 +61,7 @@ struct PanelLds {
     double X[128 * SB][20];
     double L[8 * SB][16][17];  // diagonal blocks, then their inverses
     double R[8 * SB][16];      // reciprocals of the diagonal
+    int kept[8 * SB];          // the block was not inverted: it is substituted
     int ready[8 * SB];         // X of the block is in place
     int odd;                   // a result that is not finite
 };
@@ -74,6 +89,12 @@ __device__ __forceinline__ double lds_value(const double *p)
 {
     return __builtin_bit_cast(double, __hip_atomic_load((const unsigned long long *)p, __ATOMIC_RELAXED,
                                                         __HIP_MEMORY_SCOPE_WORKGROUP));
+}
+
+// |v| as an integer to compare (20 bits of the mantissa; a NaN is above all).
+__device__ __forceinline__ unsigned magnitude(double v)
+{
+    return (unsigned)(__builtin_bit_cast(unsigned long long, v) >> 32) & 0x7fffffffu;
 }
 
 // The same panel by plain substitution, row by row, from the right-hand sides
@@ -146,7 +167,7 @@ __device__ __forceinline__ void trsm_panel(const PanelArgs &p, PanelLds<SB> &s)
     const int pr = runs ? tid & 31 : tid >> 4, pc = runs ? tid >> 5 : tid & 15;
     auto in_panel = [&](int e) { return pr + 32 * e < order && pc < p.cols; };
     const long pstep = 32 * p.ss;
-    IO *const bp = B + pr * p.ss + pc * p.rs;
+    const IO *const bp = B + pr * p.ss + pc * p.rs;
 #pragma unroll
     for (int e = 0; e < PER; ++e) v[e] = *(in_panel(e) ? bp + e * pstep : B);
 #pragma unroll
@@ -159,7 +180,9 @@ __device__ __forceinline__ void trsm_panel(const PanelArgs &p, PanelLds<SB> &s)
         const int bk = 4 * wave + q0;
         if (bk < nb && bk < NBMAX) {
             double y[16];
-            s.R[bk][cl] = 1.0 / s.L[bk][cl][cl];
+            const double own = 1.0 / s.L[bk][cl][cl];
+            s.R[bk][cl] = own;
+            const unsigned limit = magnitude(kInverseGrowth<IO> * own);
             lds_order();
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
@@ -170,8 +193,14 @@ __device__ __forceinline__ void trsm_panel(const PanelArgs &p, PanelLds<SB> &s)
                 y[i] = t * rc;
             }
             lds_order();  // every lane's reads of the block are done
+            unsigned top = 0;
 #pragma unroll
-            for (int i = 0; i < 16; ++i) s.L[bk][i][cl] = y[i];
+            for (int i = 0; i < 16; ++i) top = max(top, magnitude(y[i]));
+            const bool kept = (__ballot(top > limit) >> (16 * q0) & 0xffff) != 0;
+            if (cl == 0) s.kept[bk] = kept;
+            if (__builtin_expect(!kept, 1))
+#pragma unroll
+                for (int i = 0; i < 16; ++i) s.L[bk][i][cl] = y[i];
         }
     }
 #pragma unroll
@@ -226,14 +255,37 @@ __device__ __forceinline__ void trsm_panel(const PanelArgs &p, PanelLds<SB> &s)
         }
     };
     upcoming(0);
+    unsigned kept = 0;  // bit q: the wave's block q is substituted
+#pragma unroll
+    for (int q = 0; q < SB; ++q) {
+        const int J = wave + TP_WAVES * q;
+        if (J < nb) kept |= (unsigned)__builtin_amdgcn_readfirstlane(s.kept[J]) << q;
+    }
     bool finite = true;
     // X_J = inv(T_JJ) B_J, published
     auto solve = [&](int q) {
         const int J = wave + TP_WAVES * q;
         v4d x = {0.0, 0.0, 0.0, 0.0};
+        if (__builtin_expect(kept >> q & 1, 0)) {
+            // substitution, row r in element r / 4 of the lanes with q0 = r % 4 (T is
+            // zero above its diagonal)
 #pragma unroll
-        for (int u = 0; u < 4; ++u)
-            x = __builtin_amdgcn_mfma_f64_16x16x4f64(inv[u], rhs[u] - acc[q][u], x, 0, 0, 0);
+            for (int u = 0; u < 4; ++u) x[u] = rhs[u] - acc[q][u];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll 1
+                for (int h = 0; h < 4; ++h) {
+                    const int r = 4 * e + h;
+                    const double xr = __shfl(x[e], cl + 16 * h) * s.R[J][r];
+                    x[e] = q0 == h ? xr : fma(-s.L[J][4 * e + q0][r], xr, x[e]);
+#pragma unroll
+                    for (int u = e + 1; u < 4; ++u) x[u] = fma(-s.L[J][4 * u + q0][r], xr, x[u]);
+                }
+        } else {
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                x = __builtin_amdgcn_mfma_f64_16x16x4f64(inv[u], rhs[u] - acc[q][u], x, 0, 0, 0);
+        }
 #pragma unroll
         for (int u = 0; u < 4; ++u) s.X[16 * J + q0 + 4 * u][cl] = x[u];
         __atomic_signal_fence(__ATOMIC_SEQ_CST);
@@ -295,9 +347,15 @@ __device__ __forceinline__ void trsm_panel(const PanelArgs &p, PanelLds<SB> &s)
     if (__any(!finite) && lane == 0) s.odd = 1;
     __syncthreads();  // all of X, and whether it is finite
     if (s.odd) panel_by_rows<IO, SB>(p, s);
+    // (the thread's place in the panel once more: kept over the steps it would cost
+    // the registers of a third workgroup per CU where SB is 1)
+    int out = threadIdx.x;
+    asm volatile("" : "+v"(out));
+    const int orow = runs ? out & 31 : out >> 4, ocol = runs ? out >> 5 : out & 15;
+    IO *const op = B + orow * p.ss + ocol * p.rs;
 #pragma unroll
     for (int e = 0; e < PER; ++e)
-        if (in_panel(e)) bp[e * pstep] = (IO)s.X[pr + 32 * e][pc];
+        if (orow + 32 * e < order && ocol < p.cols) op[e * pstep] = (IO)s.X[orow + 32 * e][ocol];
 }
 
 // Panel arguments of op(T) X = alpha B: T lower (`lower`) in plain or transposed
