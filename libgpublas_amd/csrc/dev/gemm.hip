@@ -38,8 +38,8 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemmArgs<T> g)
 
 // Fast kernel: every tile of a product at least a tile wide in both dimensions,
 // access patterns compile-time constants (PA / PB), operands of any alignment
-// (gemm_fast_tile, tile shape S).
-template <typename T, int S, int PA, int PB, int TRI>
+// (gemm_fast_tile, tile shape S, lane offsets Off).
+template <typename T, int S, int PA, int PB, int TRI, typename Off>
 __global__ __launch_bounds__(256, 2) void gemm_fast_kernel(GemmArgs<T> g)
 {
     typedef FastShape<T, S> F;
@@ -55,7 +55,7 @@ __global__ __launch_bounds__(256, 2) void gemm_fast_kernel(GemmArgs<T> g)
         tri_decode(blockIdx.x, hi, lo);
         if (TRI == SYM_LOWER) { tm = hi; tn = lo; } else { tm = lo; tn = hi; }
     }
-    gemm_fast_tile<T, F::BM, F::BN, F::BK, F::NST, PA, PB, TRI>(g, tm, tn, As, Bs);
+    gemm_fast_tile<T, F::BM, F::BN, F::BK, F::NST, PA, PB, TRI, Off>(g, tm, tn, As, Bs);
 }
 
 // Split-K for problems with too few tiles to fill the chip and a long k:
@@ -64,7 +64,7 @@ __global__ __launch_bounds__(256, 2) void gemm_fast_kernel(GemmArgs<T> g)
 // n, leading dimension m); splitk_fold_kernel then forms alpha * (sum of chunks
 // in chunk order) + beta * C.  The decomposition depends only on the shape, so
 // the bits repeat from call to call.
-template <typename T, int PA, int PB>
+template <typename T, int PA, int PB, typename Off>
 __global__ __launch_bounds__(256, 2) void gemm_fast_splitk_kernel(GemmArgs<T> g, int kchunk, T *P)
 {
     typedef FastShape<T, 32> F;
@@ -82,8 +82,8 @@ __global__ __launch_bounds__(256, 2) void gemm_fast_splitk_kernel(GemmArgs<T> g,
     h.beta = T(0);
     h.C = P + (long)kc * g.m * g.n;
     h.ldc = g.m;
-    gemm_fast_tile<T, F::BM, F::BN, F::BK, F::NST, PA, PB, SYM_NONE>(h, t % g.tiles_m, t / g.tiles_m,
-                                                                     As, Bs);
+    gemm_fast_tile<T, F::BM, F::BN, F::BK, F::NST, PA, PB, SYM_NONE, Off>(h, t % g.tiles_m,
+                                                                          t / g.tiles_m, As, Bs);
 }
 
 template <typename T>
@@ -146,11 +146,11 @@ template <> const char *kname<float>(int shape)
                          : "sgemm_edge_64x64";
 }
 
-template <typename T, int S>
+template <typename T, int S, typename Off = unsigned>
 void launch_fast(hipStream_t s, const GemmArgs<T> &g, unsigned blocks)
 {
 #define GB_FAST(PA_, PB_, TRI_)                                                                  \
-    hipLaunchKernelGGL((gemm_fast_kernel<T, S, PA_, PB_, TRI_>), dim3(blocks), dim3(256), 0, s, g)
+    hipLaunchKernelGGL((gemm_fast_kernel<T, S, PA_, PB_, TRI_, Off>), dim3(blocks), dim3(256), 0, s, g)
     const int pa = g.a.form, pb = g.b.form;
     if (g.tri == SYM_NONE) {
         if (pa == PAT_OUTER && pb == PAT_KCONT) GB_FAST(PAT_OUTER, PAT_KCONT, SYM_NONE);      // NN
@@ -194,7 +194,7 @@ long device_cus()
 // shape does not qualify, when no scratch is left, or while s records a graph (a
 // replay would find the partial sums' pool block in other hands), so the caller
 // takes the ordinary grid.
-template <typename T>
+template <typename T, typename Off>
 int launch_splitk(hipStream_t s, const GemmArgs<T> &g, int m, int n, int k)
 {
     const long tiles = (long)ceil_div(m, 32) * ceil_div(n, 32);
@@ -214,7 +214,7 @@ int launch_splitk(hipStream_t s, const GemmArgs<T> &g, int m, int n, int k)
     f.tiles_n = ceil_div(n, 32);
     const unsigned blocks = (unsigned)(tiles * ks);
 #define GB_SK(PA_, PB_)                                                                          \
-    hipLaunchKernelGGL((gemm_fast_splitk_kernel<T, PA_, PB_>), dim3(blocks), dim3(256), 0, s, \
+    hipLaunchKernelGGL((gemm_fast_splitk_kernel<T, PA_, PB_, Off>), dim3(blocks), dim3(256), 0, s, \
                        f, kchunk, P)
     const int pa = g.a.form, pb = g.b.form;
     PROF_BEGIN(s, sizeof(T) == 8 ? "dgemm_splitk" : "sgemm_splitk");
@@ -281,7 +281,10 @@ template <typename T> bool skewed(const Operand<T> &o)
 // Core launcher: C = alpha*op(A)*op(B) + beta*C on an (optionally
 // triangular) tile grid.  k > 0, alpha != 0 assumed.  Products at least 32 wide
 // in both dimensions go to the fast kernel; the generic kernel takes the narrow
-// ones, symmetric operands and leading dimensions past FAST_LD_MAX.
+// ones and symmetric operands.  Leading dimensions past FAST_LD_MAX (`wide`) take its
+// 64 x 64 and split-K forms with 64-bit offsets (FP64, leading dimension 2 x 10^7: 64 x
+// 64 x 2048 TN 176 us on the generic kernel, 12 here; 2 x 10^7 rows of 64 columns times
+// 64 x 64 5.8 and 4.5 ms).
 template <typename T>
 int launch_gemm(hipStream_t s, int m, int n, int k, T alpha, const Operand<T> &a,
                 const Operand<T> &b, T beta, T *C, long ldc, int tri)
@@ -292,19 +295,22 @@ int launch_gemm(hipStream_t s, int m, int n, int k, T alpha, const Operand<T> &a
     g.a = a; g.b = b;
     g.C = C; g.ldc = ldc;
     g.tri = tri;
-    const bool plain = a.sym == SYM_NONE && b.sym == SYM_NONE && a.ld <= FAST_LD_MAX &&
-                       b.ld <= FAST_LD_MAX;
-    const int shape = plain ? fast_shape<T>(m, n, tri, skewed(a) || skewed(b)) : 0;
+    const bool wide = a.ld > FAST_LD_MAX || b.ld > FAST_LD_MAX;
+    int shape = a.sym == SYM_NONE && b.sym == SYM_NONE
+                    ? fast_shape<T>(m, n, tri, skewed(a) || skewed(b)) : 0;
     if (shape && tri == SYM_NONE) {
-        const int err = launch_splitk<T>(s, g, m, n, k);
+        const int err = wide ? launch_splitk<T, size_t>(s, g, m, n, k)
+                             : launch_splitk<T, unsigned>(s, g, m, n, k);
         if (err >= 0) return err;
     }
+    if (wide && shape) shape = m >= 64 && n >= 64 ? 64 : 0;
     const int bm = shape ? shape : 64, bn = shape == 128 && sizeof(T) == 8 ? 64 : bm;
     g.tiles_m = ceil_div(m, bm);
     g.tiles_n = ceil_div(n, bn);
     const long blocks = tri ? (long)g.tiles_m * (g.tiles_m + 1) / 2 : (long)g.tiles_m * g.tiles_n;
     PROF_BEGIN(s, kname<T>(shape));
-    if (shape == 128) launch_fast<T, 128>(s, g, (unsigned)blocks);
+    if (shape && wide) launch_fast<T, 64, size_t>(s, g, (unsigned)blocks);
+    else if (shape == 128) launch_fast<T, 128>(s, g, (unsigned)blocks);
     else if (shape == 64) launch_fast<T, 64>(s, g, (unsigned)blocks);
     else if (shape == 32) launch_fast<T, 32>(s, g, (unsigned)blocks);
     else

@@ -135,23 +135,24 @@ struct TileLoader {
     // time.  `base` is the tile's first element (uniform over the workgroup),
     // so a load is one 32-bit lane offset (voff) on a scalar address that the
     // scalar unit advances; per-lane 64-bit addresses for the 2 * NV loads of
-    // a k-tile cost the registers that the fragment double buffer needs.
+    // a k-tile cost the registers that the fragment double buffer needs.  (Off:
+    // unsigned up to FAST_LD_MAX, size_t past it.)
     // Operands may have any alignment: 16-byte loads that are only
     // element-aligned are legal in global memory.
     typedef T VecU __attribute__((ext_vector_type(VEC), aligned(sizeof(T))));
     static constexpr int OUTER_K = 256 * VEC / R;   // k rows one pass covers (PAT_OUTER)
     static constexpr int KCONT_O = 256 * VEC / BK;  // operand rows one pass covers (PAT_KCONT)
 
-    template <int PAT> __device__ __forceinline__ static unsigned voff(long ld)
+    template <int PAT, typename Off> __device__ __forceinline__ static Off voff(long ld)
     {
-        const unsigned t = threadIdx.x, l = (unsigned)ld;
+        const unsigned t = threadIdx.x;
+        const Off l = (Off)ld;
         return (PAT == PAT_OUTER ? (t % (R / VEC)) * VEC + (t / (R / VEC)) * l
                                  : (t % (BK / VEC)) * VEC + (t / (BK / VEC)) * l) *
-               (unsigned)sizeof(T);
+               (Off)sizeof(T);
     }
-    template <int PAT>
-    __device__ __forceinline__ static void load_pat(const T *base, long ld, unsigned vo,
-                                                    Vec (&st)[NV])
+    template <int PAT, typename Off>
+    __device__ __forceinline__ static void load_pat(const T *base, long ld, Off vo, Vec (&st)[NV])
     {
         const long step = (PAT == PAT_OUTER ? OUTER_K : KCONT_O) * ld;
 #pragma unroll
@@ -160,7 +161,7 @@ struct TileLoader {
     }
     // The last k-tile when only krem < BK of its k rows exist: rows past them
     // read as zero (their addresses stay on the last row that exists).
-    template <int PAT>
+    template <int PAT, typename Off>
     __device__ __forceinline__ static void load_ktail(const T *base, long ld, int krem,
                                                       Vec (&st)[NV])
     {
@@ -169,8 +170,8 @@ struct TileLoader {
         for (int r = 0; r < NV; ++r) {
             if (PAT == PAT_OUTER) {
                 const int o = (t % (R / VEC)) * VEC, kk = t / (R / VEC) + r * OUTER_K;
-                const unsigned off = (unsigned)min(kk, krem - 1) * (unsigned)ld + (unsigned)o;
-                const Vec x = *(const VecU *)((const char *)base + (size_t)(off * (unsigned)sizeof(T)));
+                const Off off = (Off)min(kk, krem - 1) * (Off)ld + (Off)o;
+                const Vec x = *(const VecU *)((const char *)base + (size_t)(off * (Off)sizeof(T)));
 #pragma unroll
                 for (int e = 0; e < VEC; ++e) st[r][e] = kk < krem ? x[e] : T(0);
             } else {
@@ -178,9 +179,8 @@ struct TileLoader {
                 const T *row = base + r * (KCONT_O * ld);
 #pragma unroll
                 for (int e = 0; e < VEC; ++e) {
-                    const unsigned off =
-                        (unsigned)o * (unsigned)ld + (unsigned)min(kk + e, krem - 1);
-                    const T x = *(const T *)((const char *)row + (size_t)(off * (unsigned)sizeof(T)));
+                    const Off off = (Off)o * (Off)ld + (Off)min(kk + e, krem - 1);
+                    const T x = *(const T *)((const char *)row + (size_t)(off * (Off)sizeof(T)));
                     st[r][e] = kk + e < krem ? x : T(0);
                 }
             }
@@ -475,9 +475,10 @@ struct TileMath {
     }
 };
 
-// Leading dimensions that the fast tile's 32-bit lane offsets reach (a pass
-// of one operand covers at most 64 rows of its leading dimension).
-constexpr long FAST_LD_MAX = 1l << 23;
+// Leading dimensions that the fast tile's 32-bit lane offsets reach: a lane is at
+// most 31 (FP32: 63) columns and 32 elements from its tile's scalar address, 63 * 4 *
+// 2^24 + 128 < 2^32.  Longer ones take 64-bit offsets.
+constexpr long FAST_LD_MAX = 1l << 24;
 
 // The fast tile's shapes.  NST: k-tiles of one operand on their way in registers.
 // A 32 x 32 FP32 tile takes 32 of k at a time, one 16-byte load per thread.
@@ -508,7 +509,7 @@ template <typename T, int S> struct FastShape {
 // (NST 3 was slower than 2).  128 x 128 FP64 tiles have no registers for a second
 // stage; more than 256 registers a lane make the compiler move the accumulators to
 // and from the accumulation registers in every k-tile (48 TFLOP/s).
-template <typename T, int BM, int BN, int BK, int NST, int PA, int PB, int TRI>
+template <typename T, int BM, int BN, int BK, int NST, int PA, int PB, int TRI, typename Off = unsigned>
 __device__ __forceinline__ void gemm_fast_tile(const GemmArgs<T> &g, int tm, int tn,
                                                T (*As)[BK][BM + 128 / sizeof(T)],
                                                T (*Bs)[BK][BN + 128 / sizeof(T)])
@@ -525,7 +526,7 @@ __device__ __forceinline__ void gemm_fast_tile(const GemmArgs<T> &g, int tm, int
     const T *pa = g.a.p + (PA == PAT_OUTER ? (long)m0 : (long)m0 * lda);
     const T *pb = g.b.p + (PB == PAT_OUTER ? (long)n0 : (long)n0 * ldb);
     const long stepa = PA == PAT_OUTER ? BK * lda : BK, stepb = PB == PAT_OUTER ? BK * ldb : BK;
-    const unsigned va = LA::template voff<PA>(lda), vb = LB::template voff<PB>(ldb);
+    const Off va = LA::template voff<PA, Off>(lda), vb = LB::template voff<PB, Off>(ldb);
 
     typename M::Acc acc[M::FM][M::FN];
 #pragma unroll
@@ -547,8 +548,8 @@ __device__ __forceinline__ void gemm_fast_tile(const GemmArgs<T> &g, int tm, int
         if (t < kfull) {
             load_full(r);
         } else if (t < ktiles) {
-            LA::template load_ktail<PA>(pa, lda, K - t * BK, sa[r]);
-            LB::template load_ktail<PB>(pb, ldb, K - t * BK, sb[r]);
+            LA::template load_ktail<PA, Off>(pa, lda, K - t * BK, sa[r]);
+            LB::template load_ktail<PB, Off>(pb, ldb, K - t * BK, sb[r]);
         }
     };
     auto store = [&](int buf, int r) {
