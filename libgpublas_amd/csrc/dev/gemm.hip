@@ -405,7 +405,7 @@ __global__ __launch_bounds__(256) void symmetrize_kernel(int n, const T *__restr
 // (tm, tn) runs only over the k range where that factor is nonzero (the
 // other products are exact zeros), so a triangular multiply costs half a
 // GEMM.  KR: 1 k < (tm+1)*BM, 2 k >= tm*BM (left factor lower / upper),
-// 3 k >= tn*BM, 4 k < (tn+1)*BM (right factor lower / upper).  Operand
+// 3 k >= tn*BN, 4 k < (tn+1)*BN (right factor lower / upper).  Operand
 // pointers are shifted to the range start as in the split-K kernel; tiles
 // are dispatched longest range first.  (A ragged last tile is moved back, but
 // stores only its own rows and columns, for which the range is right.)
@@ -413,8 +413,7 @@ template <typename T, int S, int PA, int PB, int KR>
 __global__ __launch_bounds__(256, 2) void gemm_fast_krange_kernel(GemmArgs<T> g)
 {
     typedef FastShape<T, S> F;
-    constexpr int BM = F::BM;
-    static_assert(BM == F::BN, "square tiles");
+    constexpr int BM = F::BM, BN = F::BN;
     __shared__ __attribute__((aligned(16))) T As[2][F::BK][F::LDA];
     __shared__ __attribute__((aligned(16))) T Bs[2][F::BK][F::LDB];
     // longest ranges first, so the last round holds the shortest tiles
@@ -432,13 +431,13 @@ __global__ __launch_bounds__(256, 2) void gemm_fast_krange_kernel(GemmArgs<T> g)
     int kb = 0, ke = g.k;
     if (KR == 1) ke = min(g.k, (tm + 1) * BM);
     if (KR == 2) kb = tm * BM;
-    if (KR == 3) kb = tn * BM;
-    if (KR == 4) ke = min(g.k, (tn + 1) * BM);
+    if (KR == 3) kb = tn * BN;
+    if (KR == 4) ke = min(g.k, (tn + 1) * BN);
     GemmArgs<T> h = g;
     h.a.p += PA == PAT_OUTER ? (long)kb * g.a.ld : kb;
     h.b.p += PB == PAT_OUTER ? (long)kb * g.b.ld : kb;
     h.k = ke - kb;
-    gemm_fast_tile<T, BM, BM, F::BK, F::NST, PA, PB, SYM_NONE>(h, tm, tn, As, Bs);
+    gemm_fast_tile<T, BM, BN, F::BK, F::NST, PA, PB, SYM_NONE>(h, tm, tn, As, Bs);
 }
 
 // Full n x n matrix of a triangle of A: the stored triangle copied, zeros
@@ -520,11 +519,12 @@ int symm_entry(void *stream, char side, char uplo, int m, int n, T alpha, const 
 // Triangular-k product (see gemm_fast_krange_kernel); -1 when the shape or
 // the operands do not allow the fast tiles (the caller then runs the
 // ordinary full-k GEMM).  beta = 0.
-template <typename T, int BM>
+template <typename T, int S>
 int launch_krange(hipStream_t s, int m, int n, int k, T alpha, const Operand<T> &a,
                   const Operand<T> &b, T *C, long ldc, int kr)
 {
-    if (m < BM || n < BM || a.ld > FAST_LD_MAX || b.ld > FAST_LD_MAX) return -1;
+    constexpr int BM = FastShape<T, S>::BM, BN = FastShape<T, S>::BN;
+    if (m < BM || n < BN || a.ld > FAST_LD_MAX || b.ld > FAST_LD_MAX) return -1;
     GemmArgs<T> g;
     g.m = m; g.n = n; g.k = k;
     g.alpha = alpha; g.beta = T(0);
@@ -532,14 +532,14 @@ int launch_krange(hipStream_t s, int m, int n, int k, T alpha, const Operand<T> 
     g.C = C; g.ldc = ldc;
     g.tri = SYM_NONE;
     g.tiles_m = ceil_div(m, BM);
-    g.tiles_n = ceil_div(n, BM);
+    g.tiles_n = ceil_div(n, BN);
     const unsigned blocks = (unsigned)(g.tiles_m * g.tiles_n);
 #define GB_KR(PA_, PB_)                                                                          \
     do {                                                                                         \
-        if (kr == 1) hipLaunchKernelGGL((gemm_fast_krange_kernel<T, BM, PA_, PB_, 1>), dim3(blocks), dim3(256), 0, s, g); \
-        else if (kr == 2) hipLaunchKernelGGL((gemm_fast_krange_kernel<T, BM, PA_, PB_, 2>), dim3(blocks), dim3(256), 0, s, g); \
-        else if (kr == 3) hipLaunchKernelGGL((gemm_fast_krange_kernel<T, BM, PA_, PB_, 3>), dim3(blocks), dim3(256), 0, s, g); \
-        else hipLaunchKernelGGL((gemm_fast_krange_kernel<T, BM, PA_, PB_, 4>), dim3(blocks), dim3(256), 0, s, g); \
+        if (kr == 1) hipLaunchKernelGGL((gemm_fast_krange_kernel<T, S, PA_, PB_, 1>), dim3(blocks), dim3(256), 0, s, g); \
+        else if (kr == 2) hipLaunchKernelGGL((gemm_fast_krange_kernel<T, S, PA_, PB_, 2>), dim3(blocks), dim3(256), 0, s, g); \
+        else if (kr == 3) hipLaunchKernelGGL((gemm_fast_krange_kernel<T, S, PA_, PB_, 3>), dim3(blocks), dim3(256), 0, s, g); \
+        else hipLaunchKernelGGL((gemm_fast_krange_kernel<T, S, PA_, PB_, 4>), dim3(blocks), dim3(256), 0, s, g); \
     } while (0)
     const int pa = a.form, pb = b.form;
     PROF_BEGIN(s, sizeof(T) == 8 ? "dgemm_krange" : "sgemm_krange");
@@ -612,12 +612,14 @@ int trmm_entry(void *stream, char side, char uplo, char transa, char diag, int m
                                   : make_op<T>(Tm, ldt, n, tn ? PAT_KCONT : PAT_OUTER, SYM_NONE);
         const int k = left ? m : n;
         const int kr = left ? (oplower ? 1 : 2) : (oplower ? 3 : 4);
-        if constexpr (sizeof(T) == 8)
-            err = launch_krange<T, 64>(s, m, n, k, alpha, a, b, W, ldw, kr);
-        else
-            err = fast_shape<T>(m, n, SYM_NONE, false) == 128
-                      ? launch_krange<T, 128>(s, m, n, k, alpha, a, b, W, ldw, kr)
-                      : launch_krange<T, 64>(s, m, n, k, alpha, a, b, W, ldw, kr);
+        // the full product's shape; FP64 from 24 large tiles a CU on, as their ranges
+        // even out late (8192^2 9.27 ms on 64 x 64 tiles, 8.42 on 128 x 64; 6144^2 3.44
+        // and 3.56, 4096^2 1.07 and 1.11)
+        const bool many = sizeof(T) == 4 ||
+                          (long)ceil_div(m, 128) * ceil_div(n, 64) >= 24 * device_cus();
+        err = many && fast_shape<T>(m, n, SYM_NONE, false) == 128
+                  ? launch_krange<T, 128>(s, m, n, k, alpha, a, b, W, ldw, kr)
+                  : launch_krange<T, 64>(s, m, n, k, alpha, a, b, W, ldw, kr);
         if (err < 0) err = launch_gemm<T>(s, m, n, k, alpha, a, b, T(0), W, ldw, SYM_NONE);
     }
     if (!err)
