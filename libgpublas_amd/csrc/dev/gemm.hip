@@ -36,6 +36,28 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemmArgs<T> g)
     gemm_tile<T, BM, BN, BK>(g, tm, tn, As, Bs);
 }
 
+// Tile of block b of a rectangular grid: down the rows, column by column.  Blocks
+// go round the eight XCDs, each with an L2 of its own, one by one, so with fewer
+// than eight row tiles beside more column tiles every XCD would read most of B.
+// Then the tiles of a column stay on one XCD: block 8 i + x takes XCD x's i-th tile
+// of columns x, x + 8, ...; what is left of the columns runs in the plain order
+// (FP64 NN 128 x 4096 x 4096 106 -> 78 us, 64 x 4096 x 4096 61 -> 43, NT 100 x 10000 x
+// 256 23.2 -> 16.6; FP32 NT 128 x 4096 x 4096 75 -> 49).
+template <typename T>
+__device__ __forceinline__ void tile_at(const GemmArgs<T> &g, int b, int &tm, int &tn)
+{
+    const int whole = g.tiles_m < 8 && g.tiles_n > g.tiles_m ? g.tiles_n / 8 * 8 : 0;
+    if (b < whole * g.tiles_m) {
+        const int i = b / 8;
+        tm = i % g.tiles_m;
+        tn = i / g.tiles_m * 8 + b % 8;
+    } else {
+        b -= whole * g.tiles_m;
+        tm = b % g.tiles_m;
+        tn = whole + b / g.tiles_m;
+    }
+}
+
 // Fast kernel: every tile of a product at least a tile wide in both dimensions,
 // access patterns compile-time constants (PA / PB), operands of any alignment
 // (gemm_fast_tile, tile shape S, lane offsets Off).
@@ -48,8 +70,7 @@ __global__ __launch_bounds__(256, 2) void gemm_fast_kernel(GemmArgs<T> g)
 
     int tm, tn;
     if (TRI == SYM_NONE) {
-        tm = blockIdx.x % g.tiles_m;
-        tn = blockIdx.x / g.tiles_m;
+        tile_at(g, (int)blockIdx.x, tm, tn);
     } else {
         int hi, lo;
         tri_decode(blockIdx.x, hi, lo);
@@ -82,8 +103,9 @@ __global__ __launch_bounds__(256, 2) void gemm_fast_splitk_kernel(GemmArgs<T> g,
     h.beta = T(0);
     h.C = P + (long)kc * g.m * g.n;
     h.ldc = g.m;
-    gemm_fast_tile<T, F::BM, F::BN, F::BK, F::NST, PA, PB, SYM_NONE, Off>(h, t % g.tiles_m,
-                                                                          t / g.tiles_m, As, Bs);
+    int tm, tn;
+    tile_at(g, t, tm, tn);
+    gemm_fast_tile<T, F::BM, F::BN, F::BK, F::NST, PA, PB, SYM_NONE, Off>(h, tm, tn, As, Bs);
 }
 
 template <typename T>
