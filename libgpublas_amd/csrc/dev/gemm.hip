@@ -44,18 +44,19 @@ __global__ __launch_bounds__(256) void gemm_mfma_kernel(GemmArgs<T> g)
 // (FP64 NN 128 x 4096 x 4096 106 -> 78 us, 64 x 4096 x 4096 61 -> 43, NT 100 x 10000 x
 // 256 23.2 -> 16.6; FP32 NT 128 x 4096 x 4096 75 -> 49).
 template <typename T>
-__device__ __forceinline__ void tile_at(const GemmArgs<T> &g, int b, int &tm, int &tn)
+__device__ __forceinline__ void tile_at(const GemmArgs<T> &g, unsigned b, int &tm, int &tn)
 {
-    const int whole = g.tiles_m < 8 && g.tiles_n > g.tiles_m ? g.tiles_n / 8 * 8 : 0;
-    if (b < whole * g.tiles_m) {
-        const int i = b / 8;
-        tm = i % g.tiles_m;
-        tn = i / g.tiles_m * 8 + b % 8;
-    } else {
-        b -= whole * g.tiles_m;
-        tm = b % g.tiles_m;
-        tn = whole + b / g.tiles_m;
-    }
+    const unsigned rows = g.tiles_m, dealt = g.dealt * rows;
+    const bool in = b < dealt;
+    const unsigned i = in ? b >> 3 : b - dealt, q = i / rows;
+    tm = i - q * rows;
+    tn = in ? 8 * q + (b & 7) : g.dealt + q;
+}
+template <typename T> void set_tiles(GemmArgs<T> &g, int tiles_m, int tiles_n)
+{
+    g.tiles_m = tiles_m;
+    g.tiles_n = tiles_n;
+    g.dealt = tiles_m < 8 && tiles_n > tiles_m ? tiles_n / 8 * 8 : 0;
 }
 
 // Fast kernel: every tile of a product at least a tile wide in both dimensions,
@@ -70,7 +71,7 @@ __global__ __launch_bounds__(256, 2) void gemm_fast_kernel(GemmArgs<T> g)
 
     int tm, tn;
     if (TRI == SYM_NONE) {
-        tile_at(g, (int)blockIdx.x, tm, tn);
+        tile_at(g, blockIdx.x, tm, tn);
     } else {
         int hi, lo;
         tri_decode(blockIdx.x, hi, lo);
@@ -232,8 +233,7 @@ int launch_splitk(hipStream_t s, const GemmArgs<T> &g, int m, int n, int k)
     T *P = (T *)gpublas_dev_alloc((size_t)ks * m * n * sizeof(T));
     if (!P) return -1;
     GemmArgs<T> f = g;
-    f.tiles_m = ceil_div(m, 32);
-    f.tiles_n = ceil_div(n, 32);
+    set_tiles(f, ceil_div(m, 32), ceil_div(n, 32));
     const unsigned blocks = (unsigned)(tiles * ks);
 #define GB_SK(PA_, PB_)                                                                          \
     hipLaunchKernelGGL((gemm_fast_splitk_kernel<T, PA_, PB_, Off>), dim3(blocks), dim3(256), 0, s, \
@@ -327,8 +327,7 @@ int launch_gemm(hipStream_t s, int m, int n, int k, T alpha, const Operand<T> &a
     }
     if (wide && shape) shape = m >= 64 && n >= 64 ? 64 : 0;
     const int bm = shape ? shape : 64, bn = shape == 128 && sizeof(T) == 8 ? 64 : bm;
-    g.tiles_m = ceil_div(m, bm);
-    g.tiles_n = ceil_div(n, bn);
+    set_tiles(g, ceil_div(m, bm), ceil_div(n, bn));
     const long blocks = tri ? (long)g.tiles_m * (g.tiles_m + 1) / 2 : (long)g.tiles_m * g.tiles_n;
     PROF_BEGIN(s, kname<T>(shape));
     if (shape && wide) launch_fast<T, 64, size_t>(s, g, (unsigned)blocks);
@@ -553,8 +552,7 @@ int launch_krange(hipStream_t s, int m, int n, int k, T alpha, const Operand<T> 
     g.a = a; g.b = b;
     g.C = C; g.ldc = ldc;
     g.tri = SYM_NONE;
-    g.tiles_m = ceil_div(m, BM);
-    g.tiles_n = ceil_div(n, BN);
+    set_tiles(g, ceil_div(m, BM), ceil_div(n, BN));
     const unsigned blocks = (unsigned)(g.tiles_m * g.tiles_n);
 #define GB_KR(PA_, PB_)                                                                          \
     do {                                                                                         \

@@ -50,6 +50,7 @@ struct GemmArgs {
     T *C;
     long ldc;
     int tiles_m, tiles_n;
+    int dealt;  // columns of tiles dealt to the XCDs one by one (tile_at)
     int tri;  // 0 rectangular grid, SYM_LOWER / SYM_UPPER: triangular tile grid + mask
 };
 
