@@ -81,15 +81,16 @@ __global__ __launch_bounds__(256, 2) void gemm_fast_kernel(GemmArgs<T> g)
 }
 
 // Split-K for problems with too few tiles to fill the chip and a long k:
-// block b is 32 x 32 tile b % tiles over k chunk b / tiles (kchunk deep, a
+// block b is tile b % tiles (shape S) over k chunk b / tiles (kchunk deep, a
 // multiple of 16; the last one what is left), written unscaled to P[chunk] (m x
 // n, leading dimension m); splitk_fold_kernel then forms alpha * (sum of chunks
-// in chunk order) + beta * C.  The decomposition depends only on the shape, so
-// the bits repeat from call to call.
-template <typename T, int PA, int PB, typename Off>
+// in chunk order) + beta * C.  The decomposition depends on the shape and the
+// card alone, so the bits repeat from call to call; a call that is recorded into a
+// graph, or finds no scratch, is not split and sums k in one run.
+template <typename T, int S, int PA, int PB, typename Off>
 __global__ __launch_bounds__(256, 2) void gemm_fast_splitk_kernel(GemmArgs<T> g, int kchunk, T *P)
 {
-    typedef FastShape<T, 32> F;
+    typedef FastShape<T, S> F;
     __shared__ __attribute__((aligned(16))) T As[2][F::BK][F::LDA];
     __shared__ __attribute__((aligned(16))) T Bs[2][F::BK][F::LDB];
     const int tiles = g.tiles_m * g.tiles_n;
@@ -210,21 +211,66 @@ long device_cus()
     return n;
 }
 
-// Split-K launch of a rectangular product whose 32 x 32 tiles leave half of the
-// CUs idle: k is cut into as many chunks as fill them (at most 16, each at least
-// 256 deep, a multiple of 16; the fold costs about 5 us, 256 of k about 3).  More
-// than one workgroup a CU gains too little to pay the fold.  Returns -1 when the
-// shape does not qualify, when no scratch is left, or while s records a graph (a
-// replay would find the partial sums' pool block in other hands), so the caller
-// takes the ordinary grid.
-template <typename T, typename Off>
-int launch_splitk(hipStream_t s, const GemmArgs<T> &g, int m, int n, int k)
+// Tile shape of a product on the fast kernel, by the time the busiest CU takes:
+// its number of tiles times a tile's area over the rate that the shape reaches
+// with the chip full (TFLOP/s at 4096^3: FP64 57 / 68 / 69.5 for 32 x 32, 64 x 64
+// and 128 x 64; FP32 88 / 130 / 138 for 32 x 32, 64 x 64 and 128 x 128).  A 32 x 32
+// tile is bound by L2: where a column's 32 rows (`skewed`: an operand read along
+// its columns whose leading dimension is no multiple of 128 bytes) lie across one
+// more cache line, it reaches three quarters of that (3001 x 768 x 768 NN FP64: 95
+// us against 77 with 64 x 64, but 73 where the leading dimensions are even).  The
+// large shape also needs several tiles a CU (FP64 eight, FP32 two), below which
+// the 64 x 64 one measured the same.  Both sides, 32 against 64: FP64 512^3 8.2 and
+// 20.8 us, 768^3 24.5 and 30.3, 1024^3 41.2 and 39.2, 1536^2 x 1024 84 and 98, 2047 x
+// 1531 x 1789 209 and 173; FP32 512^3 6.0 and 11.9, 768^3 16.9 and 16.7, 1024^3 28.9
+// and 21.9.  64 against 128: FP64 8192^2 x 2048 4.08 and 3.97 ms, FP32 2900^2 x 1500
+// 229 and 287 us, 4096^3 1007 and 996.  0: narrower than every tile.
+template <typename T>
+double shape_cost(long m, long n, int tri, int shape, bool skewed)
 {
-    const long tiles = (long)ceil_div(m, 32) * ceil_div(n, 32);
-    const int want = (int)std::min<long>(std::min<long>(device_cus() / tiles, 16), k / 256);
-    if (want < 2) return -1;
-    const int kchunk = ceil_div(ceil_div(k, want), 16) * 16, ks = ceil_div(k, kchunk);
-    if (ks < 2) return -1;
+    const bool dp = sizeof(T) == 8;
+    const long bm = shape, bn = shape == 128 && dp ? 64 : shape, cus = device_cus();
+    const long tm = (m + bm - 1) / bm, tn = (n + bn - 1) / bn;
+    const long tiles = tri ? tm * (tm + 1) / 2 : tm * tn;
+    const double rate = shape == 32   ? (dp ? 57 : 88) * (skewed ? 0.75 : 1)
+                        : shape == 64 ? (dp ? 68 : 130)
+                                      : (dp ? 69.5 : 138);
+    return (double)((tiles + cus - 1) / cus * bm * bn) / rate;
+}
+
+template <typename T>
+int fast_shape(long m, long n, int tri, bool skewed)
+{
+    const bool dp = sizeof(T) == 8;
+    const long bn = dp ? 64 : 128;
+    if (m < 32 || n < 32) return 0;
+    int best = 32;
+    double least = shape_cost<T>(m, n, tri, 32, skewed);
+    if (m >= 64 && n >= 64) {
+        const double c = shape_cost<T>(m, n, tri, 64, skewed);
+        if (c <= least) best = 64, least = c;
+    }
+    if (m >= 128 && n >= bn && !(dp && tri) &&
+        ((m + 127) / 128) * ((n + bn - 1) / bn) >= (dp ? 8 : 2) * device_cus() &&
+        shape_cost<T>(m, n, tri, 128, skewed) <= least)
+        best = 128;
+    return best;
+}
+
+// An operand read along its columns whose columns start at any byte of a cache line.
+template <typename T> bool skewed(const Operand<T> &o)
+{
+    return o.form == PAT_OUTER && (o.ld * sizeof(T)) % 128 != 0;
+}
+
+// Split-K launch of a rectangular product on S x S tiles, k cut into chunks of
+// kchunk (a multiple of 16).  Returns -1 when no scratch is left, or while s records
+// a graph (a replay would find the partial sums' pool block in other hands), so the
+// caller takes the ordinary grid.
+template <typename T, int S, typename Off>
+int launch_splitk(hipStream_t s, const GemmArgs<T> &g, int m, int n, int k, int kchunk)
+{
+    const int ks = ceil_div(k, kchunk);
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
         (void)hipGetLastError();
@@ -233,10 +279,10 @@ int launch_splitk(hipStream_t s, const GemmArgs<T> &g, int m, int n, int k)
     T *P = (T *)gpublas_dev_alloc((size_t)ks * m * n * sizeof(T));
     if (!P) return -1;
     GemmArgs<T> f = g;
-    set_tiles(f, ceil_div(m, 32), ceil_div(n, 32));
-    const unsigned blocks = (unsigned)(tiles * ks);
+    set_tiles(f, ceil_div(m, S), ceil_div(n, S));
+    const unsigned blocks = (unsigned)((long)f.tiles_m * f.tiles_n * ks);
 #define GB_SK(PA_, PB_)                                                                          \
-    hipLaunchKernelGGL((gemm_fast_splitk_kernel<T, PA_, PB_, Off>), dim3(blocks), dim3(256), 0, s, \
+    hipLaunchKernelGGL((gemm_fast_splitk_kernel<T, S, PA_, PB_, Off>), dim3(blocks), dim3(256), 0, s, \
                        f, kchunk, P)
     const int pa = g.a.form, pb = g.b.form;
     PROF_BEGIN(s, sizeof(T) == 8 ? "dgemm_splitk" : "sgemm_splitk");
@@ -254,50 +300,42 @@ int launch_splitk(hipStream_t s, const GemmArgs<T> &g, int m, int n, int k)
     return (int)hipGetLastError();
 }
 
-// Tile shape of a product on the fast kernel, by the time the busiest CU takes:
-// its number of tiles times a tile's area over the rate that the shape reaches
-// with the chip full (TFLOP/s at 4096^3: FP64 57 / 68 / 69.5 for 32 x 32, 64 x 64
-// and 128 x 64; FP32 88 / 130 / 138 for 32 x 32, 64 x 64 and 128 x 128).  A 32 x 32
-// tile is bound by L2: where a column's 32 rows (`skewed`: an operand read along
-// its columns whose leading dimension is no multiple of 128 bytes) lie across one
-// more cache line, it reaches three quarters of that (3001 x 768 x 768 NN FP64: 95
-// us against 77 with 64 x 64, but 73 where the leading dimensions are even).  The
-// large shape also needs several tiles a CU (FP64 eight, FP32 two), below which
-// the 64 x 64 one measured the same.  Both sides, 32 against 64: FP64 512^3 8.2 and
-// 20.8 us, 768^3 24.5 and 30.3, 1024^3 41.2 and 39.2, 1536^2 x 1024 84 and 98, 2047 x
-// 1531 x 1789 209 and 173; FP32 512^3 6.0 and 11.9, 768^3 16.9 and 16.7, 1024^3 28.9
-// and 21.9.  64 against 128: FP64 8192^2 x 2048 4.08 and 3.97 ms, FP32 2900^2 x 1500
-// 229 and 287 us, 4096^3 1007 and 996.  0: narrower than every tile.
+// How a rectangular product of at least 32 x 32 is split along k, if it is: shape 32
+// where 32 x 32 tiles leave half of the CUs idle, as many chunks as fill them (at most
+// 16, each at least 256 deep; the fold costs about 5 us, 256 of k about 3).  Else
+// shape 64, two workgroups a CU, where that beats the unsplit `shape` by the cost rule
+// above, the fold counted as 5 us and the partial sums' traffic at 3 TB/s: only a long
+// k pays it.  (A skewed operand costs little where the chip is not full; FP32 tiles of
+// 32 x 32 reach 100, 87 and 74 TFLOP/s with none, one and both operands contiguous
+// along k.)  Unsplit and split: FP32 TN 512 x 512 x 16384 129 and 77 us, x 8192 66 and
+// 45, 640 x 640 x 16384 232 and 117; FP64 NN 512 x 512 x 16384 159 and 142, 640 x 640 x
+// 16384 275 and 220.
+struct SplitPlan {
+    int shape, kchunk;
+};
 template <typename T>
-int fast_shape(long m, long n, int tri, bool skewed)
+SplitPlan split_plan(long m, long n, long k, int shape, int along_k)
 {
-    const bool dp = sizeof(T) == 8;
+    if (k < 512) return {0, 0};
     const long cus = device_cus();
-    auto count = [&](long bm, long bn) {
-        const long tm = (m + bm - 1) / bm, tn = (n + bn - 1) / bn;
-        return tri ? tm * (tm + 1) / 2 : tm * tn;
+    auto chunk = [&](long tiles, long slots) {
+        const long want = std::min(std::min(slots / tiles, 16l), k / 256);
+        return want < 2 ? (int)k : ceil_div(ceil_div(k, want), 16) * 16;
     };
-    auto cost = [&](long bm, long bn, double rate) {
-        return (double)((count(bm, bn) + cus - 1) / cus * bm * bn) / rate;
-    };
-    const long bn = dp ? 64 : 128;
-    if (m < 32 || n < 32) return 0;
-    int best = 32;
-    double least = cost(32, 32, (dp ? 57 : 88) * (skewed ? 0.75 : 1));
-    if (m >= 64 && n >= 64) {
-        const double c = cost(64, 64, dp ? 68 : 130);
-        if (c <= least) best = 64, least = c;
-    }
-    if (m >= 128 && n >= bn && !(dp && tri) && count(128, bn) >= (dp ? 8 : 2) * cus &&
-        cost(128, bn, dp ? 69.5 : 138) <= least)
-        best = 128;
-    return best;
-}
-
-// An operand read along its columns whose columns start at any byte of a cache line.
-template <typename T> bool skewed(const Operand<T> &o)
-{
-    return o.form == PAT_OUTER && (o.ld * sizeof(T)) % 128 != 0;
+    const int c32 = chunk((long)ceil_div(m, 32) * ceil_div(n, 32), cus);
+    if (c32 < k) return {32, c32};
+    if (m < 64 || n < 64) return {0, 0};
+    const long tiles = (long)ceil_div(m, 64) * ceil_div(n, 64);
+    const int c64 = chunk(tiles, 2 * cus);
+    if (c64 >= k) return {0, 0};
+    const long ks = ceil_div(k, c64);
+    const double us = 2e-6 * cus;  // of a unit of cost, per k
+    const double one = shape_cost<T>(64, 64 * tiles * ks, SYM_NONE, 64, false) * c64 * us;
+    const double fold = 5 + 2.0 * ks * m * n * sizeof(T) / 3e6;
+    double whole = shape_cost<T>(m, n, SYM_NONE, shape, false) * k * us;
+    if (sizeof(T) == 4 && shape == 32) whole *= 88.0 / (along_k == 0 ? 100 : along_k == 1 ? 87 : 74);
+    if (one + fold >= whole) return {0, 0};
+    return {64, c64};
 }
 
 // Core launcher: C = alpha*op(A)*op(B) + beta*C on an (optionally
@@ -321,8 +359,11 @@ int launch_gemm(hipStream_t s, int m, int n, int k, T alpha, const Operand<T> &a
     int shape = a.sym == SYM_NONE && b.sym == SYM_NONE
                     ? fast_shape<T>(m, n, tri, skewed(a) || skewed(b)) : 0;
     if (shape && tri == SYM_NONE) {
-        const int err = wide ? launch_splitk<T, size_t>(s, g, m, n, k)
-                             : launch_splitk<T, unsigned>(s, g, m, n, k);
+        const SplitPlan p = split_plan<T>(m, n, k, shape, (a.form == PAT_KCONT) + (b.form == PAT_KCONT));
+        const int err = p.shape == 32 ? wide ? launch_splitk<T, 32, size_t>(s, g, m, n, k, p.kchunk)
+                                             : launch_splitk<T, 32, unsigned>(s, g, m, n, k, p.kchunk)
+                        : p.shape == 64 && !wide ? launch_splitk<T, 64, unsigned>(s, g, m, n, k, p.kchunk)
+                                                 : -1;
         if (err >= 0) return err;
     }
     if (wide && shape) shape = m >= 64 && n >= 64 ? 64 : 0;

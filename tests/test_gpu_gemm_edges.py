@@ -104,3 +104,17 @@ def test_trmm_ragged_range(gpu, single, side, uplo, trans, m, n):
     want = hb.astype(np.float64)
     want[:m] = 2.0 * (t @ want[:m] if side == "L" else want[:m] @ t)
     assert np.array_equal(np.array(B), want)
+
+
+@pytest.mark.parametrize("ta,tb", [("N", "N"), ("N", "T"), ("T", "N"), ("T", "T")])
+@pytest.mark.parametrize("m,n,k", [(500, 449, 16411), (129, 2000, 10007)])
+def test_long_k_split_on_64(gpu, ta, tb, m, n, k):
+    """FP32 products past 128 tiles of 32 x 32 whose k is long enough to split on 64 x 64 ones,
+    the last tiles and the last chunk ragged.  Sums stay below 2^24, so they are exact."""
+    rng = np.random.default_rng(k)
+    a, b = (rng.integers(-3, 4, s).astype(np.float32) for s in ((m, k), (k, n)))
+    want = a.astype(np.float64) @ b.astype(np.float64)
+    A, B = (np.asfortranarray(x if t == "N" else x.T) for x, t in ((a, ta), (b, tb)))
+    C = np.full((m, n), 3.0, np.float32, order="F")
+    gpu.sgemm(ta, tb, m, n, k, 1.0, A, A.shape[0], B, B.shape[0], -1.0, C, m)
+    assert np.array_equal(C, want - 3.0)
