@@ -10,7 +10,9 @@
  * (case-insensitive).  `stream` is a hipStream_t or NULL for the calling
  * thread's own stream.  Arguments are assumed legal (the host layer checks
  * them netlib-style first).  Every function returns 0 on success or a
- * hipError_t code; launches are asynchronous on the stream.
+ * hipError_t code; launches are asynchronous on the stream.  A call on a stream
+ * that records a HIP graph leaves its scratch memory to that graph: destroy an
+ * executable graph only once its launches have ended.
  */
 #ifndef GPUBLAS_DEV_H
 #define GPUBLAS_DEV_H

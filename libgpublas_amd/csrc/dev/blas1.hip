@@ -38,8 +38,8 @@ __global__ void zero_ticket(unsigned *t)
 
 // Partials and ticket of one reduction on stream st.  On the calling thread's
 // own stream: one of its kSlots rotating slots (tickets kept zero between
-// launches, calls ordered by the stream).  On another stream: a pool block of
-// its own, whose ticket a one-thread kernel clears first (a fill kernel rather
+// launches, calls ordered by the stream).  On another stream, or into a graph: a
+// pool block of its own, whose ticket a one-thread kernel clears first (a fill kernel rather
 // than a memset, so the call can be captured into a graph).
 struct RedSlot {
     Scratch scr;
@@ -51,16 +51,15 @@ RedSlot next_slot(hipStream_t st)
 {
     DevCtx *c = dev_ctx();
     RedSlot r;
-    if (st == c->stream) {
-        r.scr = dev_scratch(kSlots * kSlotBytes, st);
-        if (!r.scr.p) return r;
+    static_assert(kSlots * kSlotBytes >= kSlotBytes + 256, "a block of its own fits too");
+    r.scr = dev_scratch(st == c->stream ? kSlots * kSlotBytes : kSlotBytes + 256, st);
+    if (!r.scr.p) return r;
+    if (!r.scr.pooled) {
         unsigned s = t_slot++ % kSlots;
         r.partials = (char *)r.scr.p + s * kSlotBytes;
         r.ticket = c->tickets + s;
         return r;
     }
-    r.scr = dev_scratch(kSlotBytes + 256, st);
-    if (!r.scr.p) return r;
     r.partials = r.scr.p;
     r.ticket = (unsigned *)((char *)r.scr.p + kSlotBytes);
     hipLaunchKernelGGL(zero_ticket, dim3(1), dim3(64), 0, st, r.ticket);

@@ -43,10 +43,12 @@ void dev_release_after(void *d_ptr, hipStream_t s);  // pool release ordered beh
 // Scratch memory (partial sums, tickets) of one call whose kernels run on
 // stream s.  On the calling thread's own stream it is the thread's workspace:
 // only that stream ever uses it, so growing it after a sync of that stream is
-// safe.  On any other stream it is a pool block, released behind s (once the
-// work queued on s so far completes) when the Scratch goes out of scope --
-// after the call has enqueued its launches.  Two calls on two streams thus
-// never share partials, and no queued kernel loses its workspace.
+// safe.  On any other stream, and on a stream that records a graph (a replay may
+// run anywhere, after the workspace has grown), it is a pool block, released
+// behind s (once the work queued on s so far completes; with the graph where s
+// records one) when the Scratch goes out of scope -- after the call has enqueued
+// its launches.  Two calls on two streams thus never share partials, and no
+// queued or recorded kernel loses its workspace.
 struct Scratch {
     void *p = nullptr;
     hipStream_t s = nullptr;
@@ -90,7 +92,10 @@ extern int g_prof_on;
 #define PROF_BEGIN(s, name) do { if (g_prof_on) prof_begin((s), (name)); } while (0)
 #define PROF_END(s) do { if (g_prof_on) prof_end((s)); } while (0)
 
-static inline hipStream_t pick_stream(void *s) { return s ? (hipStream_t)s : dev_ctx()->stream; }
+// The stream of a call (NULL: the calling thread's own); notes for the rest of the
+// call whether that stream records a graph.
+hipStream_t pick_stream(void *s);
+bool call_is_recorded();
 
 static inline int ceil_div(long a, long b) { return (int)((a + b - 1) / b); }
 

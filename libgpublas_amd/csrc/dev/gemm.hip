@@ -265,17 +265,13 @@ template <typename T> bool skewed(const Operand<T> &o)
 
 // Split-K launch of a rectangular product on S x S tiles, k cut into chunks of
 // kchunk (a multiple of 16).  Returns -1 when no scratch is left, or while s records
-// a graph (a replay would find the partial sums' pool block in other hands), so the
-// caller takes the ordinary grid.
+// a graph (whose scratch would be held as long as the graph is), so the caller takes
+// the ordinary grid.
 template <typename T, int S, typename Off>
 int launch_splitk(hipStream_t s, const GemmArgs<T> &g, int m, int n, int k, int kchunk)
 {
     const int ks = ceil_div(k, kchunk);
-    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
-        (void)hipGetLastError();
-        return -1;
-    }
+    if (call_is_recorded()) return -1;
     T *P = (T *)gpublas_dev_alloc((size_t)ks * m * n * sizeof(T));
     if (!P) return -1;
     GemmArgs<T> f = g;

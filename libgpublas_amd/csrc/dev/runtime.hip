@@ -8,6 +8,7 @@
 #include "devcommon.hpp"
 #include "gpublas_dev.h"
 
+#include <atomic>
 #include <mutex>
 #include <unordered_map>
 #include <vector>
@@ -50,6 +51,47 @@ size_t size_class(size_t b)
     return (b + two_mib - 1) / two_mib * two_mib;
 }
 
+// Blocks whose graph is gone.  The runtime calls block_of_graph_done() from inside
+// its own destroy functions, so it takes no lock under which the pool calls the
+// runtime; the next allocation or trim moves them to the free lists.
+std::mutex g_returned_mu;
+std::vector<void *> *g_returned;
+std::atomic<bool> g_any_returned{false};
+
+void block_of_graph_done(void *p)
+{
+    std::lock_guard<std::mutex> g(g_returned_mu);
+    g_returned->push_back(p);
+    g_any_returned.store(true, std::memory_order_release);
+}
+
+void take_returned_locked()  // the pool's lock is held
+{
+    if (!g_any_returned.load(std::memory_order_acquire)) return;
+    std::vector<void *> v;
+    {
+        std::lock_guard<std::mutex> g(g_returned_mu);
+        v.swap(*g_returned);
+        g_any_returned.store(false, std::memory_order_relaxed);
+    }
+    for (void *p : v) {
+        auto it = g_live->find(p);
+        if (it == g_live->end()) continue;
+        (*g_free)[it->second].push_back(p);
+        g_live->erase(it);
+    }
+}
+
+// The calling thread's stream capture mode set to relaxed while in scope: an
+// allocation belongs to no stream and must not end a capture that is under way.
+struct RelaxedCapture {
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+    ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
+thread_local bool t_recorded = false;  // the thread's last call went to a recording stream
+
 // Move deferred blocks whose event has completed to the free lists
 // (all of them when `wait`).
 void pool_reap_locked(bool wait)
@@ -72,6 +114,7 @@ void pool_reap_locked(bool wait)
 void pool_trim_locked()
 {
     pool_reap_locked(true);
+    take_returned_locked();
     for (auto &kv : *g_free) {
         for (void *p : kv.second) {
             (void)hipFree(p);
@@ -176,6 +219,7 @@ void do_init()
     g_free = new std::unordered_map<size_t, std::vector<void *>>();
     g_live = new std::unordered_map<void *, size_t>();
     g_deferred = new std::vector<Deferred>();
+    g_returned = new std::vector<void *>();
     g_pending = new std::vector<Pending>();
     g_event_cache = new std::vector<hipEvent_t>();
     int n = 0;
@@ -268,12 +312,24 @@ DevCtx *ctx_of(hipStream_t stream)
     return nullptr;
 }
 
+static hipStream_t stream_of(void *s) { return s ? (hipStream_t)s : dev_ctx()->stream; }
+
+hipStream_t pick_stream(void *stream)
+{
+    hipStream_t s = stream_of(stream);
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (dev_ready() && hipStreamIsCapturing(s, &st) != hipSuccess) (void)hipGetLastError();
+    t_recorded = st == hipStreamCaptureStatusActive;
+    return s;
+}
+bool call_is_recorded() { return t_recorded; }
+
 Scratch dev_scratch(size_t bytes, hipStream_t s)
 {
     Scratch r;
     DevCtx *c = dev_ctx();
     r.s = s ? s : c->stream;
-    if (r.s != c->stream) {
+    if (r.s != c->stream || t_recorded) {
         r.p = gpublas_dev_alloc(bytes);
         r.pooled = r.p != nullptr;
         return r;
@@ -344,7 +400,7 @@ void *gpublas_dev_stream(void) { return (void *)dev_ctx()->stream; }
 
 int gpublas_dev_sync(void *stream)
 {
-    hipStream_t s = pick_stream(stream);
+    hipStream_t s = stream_of(stream);
     DevCtx *c = ctx_of(s);
     const uint64_t sub = c ? __atomic_load_n(&c->submitted, __ATOMIC_ACQUIRE) : 0;
     int err = (int)hipStreamSynchronize(s);
@@ -359,13 +415,13 @@ int gpublas_dev_sync(void *stream)
 
 uint64_t gpublas_dev_stream_mark(void *stream)
 {
-    DevCtx *c = ctx_of(pick_stream(stream));
+    DevCtx *c = ctx_of(stream_of(stream));
     return c ? __atomic_add_fetch(&c->submitted, 1, __ATOMIC_ACQ_REL) : 0;
 }
 
 int gpublas_dev_stream_done(void *stream, uint64_t seq)
 {
-    hipStream_t s = pick_stream(stream);
+    hipStream_t s = stream_of(stream);
     DevCtx *c = ctx_of(s);
     if (c && __atomic_load_n(&c->completed, __ATOMIC_ACQUIRE) >= seq) return 1;
     if (hipStreamQuery(s) != hipSuccess) return 0;
@@ -387,13 +443,13 @@ void gpublas_dev_forked_child(void)
 
 int gpublas_dev_stream_known_done(void *stream, uint64_t seq)
 {
-    DevCtx *c = ctx_of(pick_stream(stream));
+    DevCtx *c = ctx_of(stream_of(stream));
     return c && __atomic_load_n(&c->completed, __ATOMIC_ACQUIRE) >= seq;
 }
 
 void gpublas_dev_stream_observed(void *stream, uint64_t seq)
 {
-    DevCtx *c = ctx_of(pick_stream(stream));
+    DevCtx *c = ctx_of(stream_of(stream));
     if (!c) return;
     uint64_t cur = __atomic_load_n(&c->completed, __ATOMIC_RELAXED);
     while (cur < seq && !__atomic_compare_exchange_n(&c->completed, &cur, seq, false,
@@ -403,8 +459,8 @@ void gpublas_dev_stream_observed(void *stream, uint64_t seq)
 
 int gpublas_dev_stream_wait(void *stream, uint64_t seq)
 {
-    DevCtx *c = ctx_of(pick_stream(stream));
-    if (!c) return (int)hipStreamSynchronize(pick_stream(stream));
+    DevCtx *c = ctx_of(stream_of(stream));
+    if (!c) return (int)hipStreamSynchronize(stream_of(stream));
     if (__atomic_load_n(&c->completed, __ATOMIC_ACQUIRE) >= seq) return 0;
     return gpublas_dev_sync(c->stream);
 }
@@ -426,7 +482,7 @@ int gpublas_dev_scalar_wait(void *stream, uint64_t seq)
     for (unsigned spin = 1;; ++spin) {
         if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) == seq) return 0;
         if ((spin & 4095) == 0) {
-            hipError_t q = hipStreamQuery(pick_stream(stream));
+            hipError_t q = hipStreamQuery(stream_of(stream));
             if (q == hipSuccess) {
                 // stream drained: the flag must be there now
                 if (__atomic_load_n(flag, __ATOMIC_ACQUIRE) == seq) return 0;
@@ -442,13 +498,16 @@ void *gpublas_dev_alloc(size_t bytes)
     if (gpublas_dev_init() != 0) return nullptr;
     size_t c = size_class(bytes ? bytes : 1);
     std::lock_guard<std::mutex> g(g_pool_mu);
-    if (!g_deferred->empty()) pool_reap_locked(false);
+    // (querying an event of a stream that records would end its capture)
+    if (!g_deferred->empty() && !t_recorded) pool_reap_locked(false);
+    take_returned_locked();
     auto it = g_free->find(c);
     void *p = nullptr;
     if (it != g_free->end() && !it->second.empty()) {
         p = it->second.back();
         it->second.pop_back();
     } else {
+        RelaxedCapture relaxed;
         if (hipMalloc(&p, c) != hipSuccess) {
             (void)hipGetLastError();
             (void)hipDeviceSynchronize();
@@ -476,10 +535,23 @@ void gpublas_dev_release(void *d_ptr)
 
 // Release a block whose last users are queued on stream s: it returns to
 // the free lists once the work queued so far on s has completed, so the
-// caller need not wait for it.
+// caller need not wait for it.  While s records a graph the users run at every
+// replay: the block then belongs to the graph and the executables made of it (a
+// user object), and returns when the last of them is destroyed.
 extern "C++" void dev_release_after(void *d_ptr, hipStream_t s)
 {
     if (!d_ptr) return;
+    if (t_recorded) {
+        hipStreamCaptureStatus st;
+        hipGraph_t graph = nullptr;
+        hipUserObject_t obj = nullptr;
+        if (hipStreamGetCaptureInfo_v2(s, &st, nullptr, &graph, nullptr, nullptr) != hipSuccess ||
+            !graph || hipUserObjectCreate(&obj, d_ptr, block_of_graph_done, 1,
+                                          hipUserObjectNoDestructorSync) != hipSuccess ||
+            hipGraphRetainUserObject(graph, obj, 1, hipGraphUserObjectMove) != hipSuccess)
+            (void)hipGetLastError();  // not tied to the graph: kept until the process ends
+        return;
+    }
     std::lock_guard<std::mutex> g(g_pool_mu);
     auto it = g_live->find(d_ptr);
     if (it == g_live->end()) return;
@@ -515,19 +587,19 @@ size_t gpublas_dev_pool_bytes(void)
 int gpublas_dev_h2d(void *d_dst, const void *h_src, size_t bytes, void *stream)
 {
     if (!bytes) return 0;
-    return (int)hipMemcpyAsync(d_dst, h_src, bytes, hipMemcpyHostToDevice, pick_stream(stream));
+    return (int)hipMemcpyAsync(d_dst, h_src, bytes, hipMemcpyHostToDevice, stream_of(stream));
 }
 
 int gpublas_dev_d2h(void *h_dst, const void *d_src, size_t bytes, void *stream)
 {
     if (!bytes) return 0;
-    return (int)hipMemcpyAsync(h_dst, d_src, bytes, hipMemcpyDeviceToHost, pick_stream(stream));
+    return (int)hipMemcpyAsync(h_dst, d_src, bytes, hipMemcpyDeviceToHost, stream_of(stream));
 }
 
 int gpublas_dev_d2d(void *d_dst, const void *d_src, size_t bytes, void *stream)
 {
     if (!bytes) return 0;
-    return (int)hipMemcpyAsync(d_dst, d_src, bytes, hipMemcpyDeviceToDevice, pick_stream(stream));
+    return (int)hipMemcpyAsync(d_dst, d_src, bytes, hipMemcpyDeviceToDevice, stream_of(stream));
 }
 
 int gpublas_dev_h2d_2d(void *d_dst, size_t ldd, const void *h_src, size_t lds, size_t m, size_t n,
@@ -535,7 +607,7 @@ int gpublas_dev_h2d_2d(void *d_dst, size_t ldd, const void *h_src, size_t lds, s
 {
     if (!m || !n) return 0;
     return (int)hipMemcpy2DAsync(d_dst, ldd * es, h_src, lds * es, m * es, n,
-                                 hipMemcpyHostToDevice, pick_stream(stream));
+                                 hipMemcpyHostToDevice, stream_of(stream));
 }
 
 int gpublas_dev_d2h_2d(void *h_dst, size_t ldd, const void *d_src, size_t lds, size_t m, size_t n,
@@ -543,7 +615,7 @@ int gpublas_dev_d2h_2d(void *h_dst, size_t ldd, const void *d_src, size_t lds, s
 {
     if (!m || !n) return 0;
     return (int)hipMemcpy2DAsync(h_dst, ldd * es, d_src, lds * es, m * es, n,
-                                 hipMemcpyDeviceToHost, pick_stream(stream));
+                                 hipMemcpyDeviceToHost, stream_of(stream));
 }
 
 void *gpublas_dev_host_alloc(size_t bytes)
