@@ -534,7 +534,8 @@ int symm_entry(void *stream, char side, char uplo, int m, int n, T alpha, const 
     const int sym = is_u(uplo) ? SYM_UPPER : SYM_LOWER;
     // From order 256 up, the stored triangle is first expanded into a full
     // symmetric matrix (one pass over na^2 elements) so the product runs on
-    // the fast GEMM kernels; same products in the same k order, same bits.
+    // the fast GEMM kernels; the same products in the same k order (but where k
+    // is split).
     const int na = is_l(side) ? m : n;
     if (na >= 256) {
         const long lds = (na + 7) / 8 * 8;

@@ -1,7 +1,8 @@
 // gemm_tile.hpp -- the generic LDS-tiled MFMA GEMM tile shared by the
 // per-call kernels (gemm.hip) and the grouped persistent kernels of the
-// serving loop (group.hip).  Both paths compute a tile of C with the same
-// code, so a product's bits do not depend on how it was launched.
+// serving loop (group.hip).  Every form of the tile (generic, fast, guarded)
+// sums k in the same order, so neither the shape of a tile nor the path changes a
+// product's bits; a split of k does, and the two paths have a rule each for it.
 //
 // Tile scheme:
 //  * a 256-thread workgroup owns a BM x BN tile of C; its 4 waves split the
