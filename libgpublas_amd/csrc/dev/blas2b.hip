@@ -306,7 +306,7 @@ int band_sym_apply(hipStream_t s, int n, int kl, int ku, const double *A, long l
     if (w > BC_MAXW) return -1;
     if (n <= 0) return 0;
     const int BC = band_cols_bc(w), nb = ceil_div(n, BC), nt = BC + w - 1;
-    double *P = (double *)gpublas_dev_alloc((size_t)nb * nt * sizeof(double));
+    double *P = (double *)dev_block((size_t)nb * nt * sizeof(double));
     if (!P) return (int)hipErrorOutOfMemory;
     BandArgs a{n, n, kl, ku, A, lda, v, incv, v0, 0, 0, n, y, incy, y0, alpha, beta, P};
     PROF_BEGIN(s, "band_mv");
@@ -337,7 +337,7 @@ int band_apply(hipStream_t s, int m, int n, int kl, int ku, const double *A, lon
     const bool direct = npass == 1 && nsplit == 1;
     double *P = nullptr;
     if (!direct) {
-        P = (double *)gpublas_dev_alloc((size_t)npass * nsplit * lenout * sizeof(double));
+        P = (double *)dev_block((size_t)npass * nsplit * lenout * sizeof(double));
         if (!P) return (int)hipErrorOutOfMemory;
     }
     PROF_BEGIN(s, "band_mv");
@@ -1212,7 +1212,7 @@ int gpublas_dev_dtbmv(void *stream, char uplo, char trans, char diag, int n, int
 {
     hipStream_t s = pick_stream(stream);
     if (n <= 0) return 0;
-    double *t = (double *)gpublas_dev_alloc((size_t)n * sizeof(double));
+    double *t = (double *)dev_block((size_t)n * sizeof(double));
     if (!t) return (int)hipErrorOutOfMemory;
     const long x0 = start_of(n, incx);
     hipLaunchKernelGGL(copy_vec, dim3((unsigned)std::min(ceil_div(n, 256), 4096)), dim3(256), 0, s, n,

@@ -158,7 +158,7 @@ int cgemm_entry(void *stream, char transa, char transb, int m, int n, int k, T a
     const int Ra = ntA ? m : k, Ca = ntA ? k : m;  // A's stored shape
     const int Rb = ntB ? k : n, Cb = ntB ? n : k;  // B's stored shape
     const size_t na = 2 * (size_t)m * k, nb = 4 * (size_t)k * n, np = 2 * (size_t)m * n;
-    T *W = (T *)gpublas_dev_alloc((na + nb + np) * sizeof(T));
+    T *W = (T *)dev_block((na + nb + np) * sizeof(T));
     if (!W) return (int)hipErrorOutOfMemory;
     T *At = W, *Bt = W + na, *P = W + na + nb;
     PROF_BEGIN(s, sizeof(T) == 8 ? "zgemm_pack" : "cgemm_pack");
@@ -323,7 +323,7 @@ int crk_entry(void *stream, int kind, char uplo, char trans, int n, int k, T ar,
     const int kk = (two ? 4 : 2) * k;  // depth of the stacked real products
     const long ld = ((long)n + 7) / 8 * 8;
     const size_t opnd = (size_t)ld * kk, prod = (size_t)ld * n;
-    T *Wk = (T *)gpublas_dev_alloc((3 * opnd + 2 * prod) * sizeof(T));
+    T *Wk = (T *)dev_block((3 * opnd + 2 * prod) * sizeof(T));
     if (!Wk) return (int)hipErrorOutOfMemory;
     T *U = Wk, *V = U + opnd, *W = V + opnd, *Pr = W + opnd, *Pi = Pr + prod;
     // {src, part, sign} per column block (x = op(A) or alpha op(A), y = op(B))
@@ -395,7 +395,7 @@ int csymm_entry(void *stream, int herm, char side, char uplo, int m, int n, T ar
     const int na = left ? m : n;
     if ((ar == T(0) && ai == T(0)))
         return cgemm_entry<T>(s, 'N', 'N', m, n, 0, ar, ai, A, lda, B, ldb, br, bi, C, ldc);
-    T *F = (T *)gpublas_dev_alloc(2 * (size_t)na * na * sizeof(T));
+    T *F = (T *)dev_block(2 * (size_t)na * na * sizeof(T));
     if (!F) return (int)hipErrorOutOfMemory;
     hipLaunchKernelGGL(expand_sym<T>, dim3(grid_for((long)na * na)), dim3(256), 0, s, na, A,
                        (long)lda, (uplo == 'U' || uplo == 'u') ? 1 : 0, herm, F);
@@ -447,7 +447,7 @@ int ctrmm_entry(void *stream, char side, char uplo, char transa, char diag, int 
         return cgemm_entry<T>(s, 'N', 'N', m, n, 0, T(0), T(0), B, ldb, B, ldb, T(0), T(0), B, ldb);
     const bool left = side == 'L' || side == 'l';
     const int na = left ? m : n;
-    T *F = (T *)gpublas_dev_alloc(2 * ((size_t)na * na + (size_t)m * n) * sizeof(T));
+    T *F = (T *)dev_block(2 * ((size_t)na * na + (size_t)m * n) * sizeof(T));
     if (!F) return (int)hipErrorOutOfMemory;
     T *Wm = F + 2 * (size_t)na * na;
     hipLaunchKernelGGL(expand_tri<T>, dim3(grid_for((long)na * na)), dim3(256), 0, s, na, A,

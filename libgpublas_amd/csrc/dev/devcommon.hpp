@@ -92,10 +92,11 @@ extern int g_prof_on;
 #define PROF_BEGIN(s, name) do { if (g_prof_on) prof_begin((s), (name)); } while (0)
 #define PROF_END(s) do { if (g_prof_on) prof_end((s)); } while (0)
 
-// The stream of a call (NULL: the calling thread's own); notes for the rest of the
-// call whether that stream records a graph.
+// The stream of a call (NULL: the calling thread's own), whether it records a graph
+// (asked once a call, by those that take scratch), and a pool block for that call.
 hipStream_t pick_stream(void *s);
 bool call_is_recorded();
+void *dev_block(size_t bytes);
 
 static inline int ceil_div(long a, long b) { return (int)((a + b - 1) / b); }
 

@@ -278,7 +278,7 @@ int launch_splitk(hipStream_t s, const GemmArgs<T> &g, int m, int n, int k, int 
 {
     const int ks = ceil_div(k, kchunk);
     if (call_is_recorded()) return -1;
-    T *P = (T *)gpublas_dev_alloc((size_t)ks * m * n * sizeof(T));
+    T *P = (T *)dev_block((size_t)ks * m * n * sizeof(T));
     if (!P) return -1;
     GemmArgs<T> f = g;
     set_tiles(f, ceil_div(m, S), ceil_div(n, S));
@@ -545,7 +545,7 @@ int symm_entry(void *stream, char side, char uplo, int m, int n, T alpha, const 
     const int na = is_l(side) ? m : n;
     if (na >= 256) {
         const long lds = (na + 7) / 8 * 8;
-        T *S = (T *)gpublas_dev_alloc((size_t)lds * na * sizeof(T));
+        T *S = (T *)dev_block((size_t)lds * na * sizeof(T));
         if (S) {
             const unsigned tiles = (unsigned)ceil_div(na, 64);
             PROF_BEGIN(s, "symmetrize");
@@ -653,8 +653,8 @@ int trmm_entry(void *stream, char side, char uplo, char transa, char diag, int m
     const bool left = is_l(side);
     const int na = left ? m : n;
     const long ldt = (na + 7) / 8 * 8, ldw = (m + 7) / 8 * 8;
-    T *Tm = (T *)gpublas_dev_alloc((size_t)ldt * na * sizeof(T));
-    T *W = (T *)gpublas_dev_alloc((size_t)ldw * n * sizeof(T));
+    T *Tm = (T *)dev_block((size_t)ldt * na * sizeof(T));
+    T *W = (T *)dev_block((size_t)ldw * n * sizeof(T));
     if (!Tm || !W) {
         gpublas_dev_release(Tm);
         gpublas_dev_release(W);

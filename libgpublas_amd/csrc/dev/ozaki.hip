@@ -785,9 +785,9 @@ int make_split(hipStream_t st, int R, int K, int KT, int s, const double *X, lon
 {
     const int f16 = fmt == GPUBLAS_SLICE_FP16, i8 = fmt == GPUBLAS_SLICE_INT8;
     out.Rp = ceil_div(R, 128) * 128;
-    out.e = (int *)gpublas_dev_alloc((size_t)R * sizeof(int));
+    out.e = (int *)dev_block((size_t)R * sizeof(int));
     // both formats: 32 bytes per row of a slab
-    void *sl = gpublas_dev_alloc((size_t)s * KT * out.Rp * 32);
+    void *sl = dev_block((size_t)s * KT * out.Rp * 32);
     out.S = i8 ? nullptr : (bf16 *)sl;
     out.S8 = i8 ? (int8_t *)sl : nullptr;
     if (!out.e || !sl) return (int)hipErrorOutOfMemory;

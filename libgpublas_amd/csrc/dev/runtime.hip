@@ -90,7 +90,10 @@ struct RelaxedCapture {
     ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
 };
 
-thread_local bool t_recorded = false;  // the thread's last call went to a recording stream
+// The stream of the calling thread's current (or last) call, and whether it records a
+// graph: 1, 0, or -1 while no part of the call has asked (52 ns).
+thread_local hipStream_t t_call_stream = nullptr;
+thread_local signed char t_call_recorded = 0;
 
 // Move deferred blocks whose event has completed to the free lists
 // (all of them when `wait`).
@@ -316,21 +319,32 @@ static hipStream_t stream_of(void *s) { return s ? (hipStream_t)s : dev_ctx()->s
 
 hipStream_t pick_stream(void *stream)
 {
-    hipStream_t s = stream_of(stream);
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (dev_ready() && hipStreamIsCapturing(s, &st) != hipSuccess) (void)hipGetLastError();
-    t_recorded = st == hipStreamCaptureStatusActive;
-    return s;
+    t_call_recorded = -1;
+    return t_call_stream = stream_of(stream);
 }
-bool call_is_recorded() { return t_recorded; }
+bool call_is_recorded()
+{
+    if (t_call_recorded < 0) {
+        hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+        if (dev_ready() && hipStreamIsCapturing(t_call_stream, &st) != hipSuccess)
+            (void)hipGetLastError();
+        t_call_recorded = st == hipStreamCaptureStatusActive;
+    }
+    return t_call_recorded != 0;
+}
+void *dev_block(size_t bytes)
+{
+    (void)call_is_recorded();
+    return gpublas_dev_alloc(bytes);
+}
 
 Scratch dev_scratch(size_t bytes, hipStream_t s)
 {
     Scratch r;
     DevCtx *c = dev_ctx();
     r.s = s ? s : c->stream;
-    if (r.s != c->stream || t_recorded) {
-        r.p = gpublas_dev_alloc(bytes);
+    if (r.s != c->stream || call_is_recorded()) {
+        r.p = dev_block(bytes);
         r.pooled = r.p != nullptr;
         return r;
     }
@@ -499,7 +513,7 @@ void *gpublas_dev_alloc(size_t bytes)
     size_t c = size_class(bytes ? bytes : 1);
     std::lock_guard<std::mutex> g(g_pool_mu);
     // (querying an event of a stream that records would end its capture)
-    if (!g_deferred->empty() && !t_recorded) pool_reap_locked(false);
+    if (!g_deferred->empty() && t_call_recorded <= 0) pool_reap_locked(false);
     take_returned_locked();
     auto it = g_free->find(c);
     void *p = nullptr;
@@ -541,7 +555,7 @@ void gpublas_dev_release(void *d_ptr)
 extern "C++" void dev_release_after(void *d_ptr, hipStream_t s)
 {
     if (!d_ptr) return;
-    if (t_recorded) {
+    if (call_is_recorded()) {
         hipStreamCaptureStatus st;
         hipGraph_t graph = nullptr;
         hipUserObject_t obj = nullptr;

@@ -633,7 +633,7 @@ int solve_strided(hipStream_t s, char uplo, char trans, char diag, int n, const 
                   long lda, bool packed, double *x, int incx)
 {
     if (incx == 1) return solve(s, uplo, trans, diag, n, A, lda, packed, x);
-    double *t = (double *)gpublas_dev_alloc((size_t)n * sizeof(double));
+    double *t = (double *)dev_block((size_t)n * sizeof(double));
     if (!t) return (int)hipErrorOutOfMemory;
     const long x0 = incx < 0 ? -(long)(n - 1) * incx : 0;
     const int blocks = std::min(ceil_div(n, 256), 4096);
