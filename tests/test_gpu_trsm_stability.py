@@ -144,3 +144,41 @@ def test_single(gpu, uplo, trans):
         x = np.array(b, order="F")
         gpu.strsm("L", uplo, trans, "N", n, 18, 1.0, np.asfortranarray(a), n, x, n)
         assert _error(a, uplo, trans, False, x, b) <= np.finfo(np.float32).eps, n
+
+
+@pytest.mark.parametrize("batch", [False, True])
+@pytest.mark.parametrize("uplo,trans", FORMS)
+def test_limits_of_the_type(gpu, uplo, trans, batch):
+    """A NaN in one right-hand side, in the next a diagonal entry whose reciprocal is infinite
+    (and not the quotient), in the others a sum of products that is infinite (and not what remains
+    of B when they are subtracted one by one: two roundings, u * 1.8e308 at most)."""
+    for n in (7, 17, 40, 128, 200, 256, 300, 512):
+        mid = n // 2 | 1
+        t, b = np.eye(n), np.zeros((n, 18))
+        t[n - 1, [0, mid]] = 0.9
+        t[n - 2, n - 2] = 1e-310
+        b[0, 0] = np.nan
+        b[n - 2, 1] = 1e-310
+        b[[0, mid, n - 1], 2:] = 1e308
+        want = b.copy()
+        want[n - 2, 1] = 1
+        want[n - 1, 2:] = -0.8e308
+        a = _stored(t, uplo, trans)
+        step = 1 if (uplo == "L") == (trans == "N") else -1
+        x = np.array(b[::step], order="F")
+        if batch:
+            A, X, slot = Matrix(gpu, a), Matrix(gpu, x), gpu.Batch(use_graph=False)
+            try:
+                assert slot.dtrsm("L", uplo, trans, "N", n, 18, 1.0, A.ptr, n, X.ptr, n) == 0
+                slot.run()
+                x = X.get()
+            finally:
+                slot.close()
+                A.free()
+                X.free()
+        else:
+            gpu.dtrsm("L", uplo, trans, "N", n, 18, 1.0, a, n, x, n)
+        x = x[::step]
+        assert np.isnan(x[0, 0]), n
+        assert np.array_equal(x[: n - 1, 1:], want[: n - 1, 1:]) and x[n - 1, 1] == 0, n
+        assert np.abs(x[n - 1, 2:] + 0.8e308).max() <= U * 1.8e308, n
